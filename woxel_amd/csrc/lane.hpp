@@ -39,12 +39,12 @@ static_assert(sizeof(GridDev) == 64, "GridDev layout");
 // table at all (GridDev::root0), a larger table is scanned through the L1 cache.
 constexpr uint32_t kRootLds = 16u;
 // Stages the root table of g in s_root when it has 2..kRootLds entries; returns
-// whether it did (the lookups then scan s_root, else root0 or g.root). Call
-// before the workgroup's first barrier (init_tab / init_rcp), which publishes the
-// copy. n5count is uniform.
+// whether it did (the lookups then scan s_root, else root0 or g.root). Every lane of the
+// workgroup calls it; n5count is uniform, and so is the barrier that publishes the copy.
 __device__ __forceinline__ bool stage_root(const GridDev &g, int4 *s_root) {
     if (g.n5count <= 1u || g.n5count > kRootLds) return false;
     for (uint32_t i = threadIdx.x; i < g.n5count; i += blockDim.x) s_root[i] = g.root[i];
+    __syncthreads();
     return true;
 }
 
@@ -408,51 +408,221 @@ __device__ __forceinline__ void lane_step(const GridDev &g, RayLane &r, const Ta
     if (!kScalarIt && r.it >= kMaxSteps) r.state = WX_MAXSTEPS;
 }
 
-// The loop of lane_run for one grid-uniform choice of step variant, root lookup
-// and leaf addressing: at most kMaxSteps iterations, the trip count a scalar.
-template <bool kN5Lds, bool kClean, int kRoot, int kWide>
-__device__ __forceinline__ void lane_loop(const GridDev &g, RayLane &r, const float2 *s_tab, const uint4 *s_n5,
-                                          const int4 *s_root, bool root_lds) {
-    // a wave-uniform loop (the trip count stays scalar) whose body runs on the lanes
-    // still stepping; it ends when no lane of the wave steps or after kMaxSteps trips
-    uint32_t it = 0;
-    do {
-        if (lane_state(r) == kRun)
-            lane_step<kN5Lds, kClean, true, float2, kRoot, kWide>(g, r, s_tab, s_n5, s_root, root_lds);
+// The fast step of lane_loop is taken by waves whose running rays all satisfy, per axis:
+//  * the direction is finite and its reciprocal too, or the direction is +0 and the
+//    start p is >= 0 or <= -2^-9;
+//  * the start is finite and not -0;
+// and whose largest direction component is at least 2^-60, on a grid with bound <=
+// kFastBound. Then nothing in the step is a NaN and the shortcuts below give the
+// reference's values:
+//  * t = (1/d) * (size * max(0, s) - m) is finite on the largest axis, so the least t is
+//    finite and the advance t * d too. On an axis with d = +0 it is inf * c with c > 0:
+//    c = size - m, and m reaches size only by rounding, for p in [-2^-10, 0) (size <
+//    2^15); p never changes on that axis, as its t is never the least.
+//  * t <= both others exactly when t equals their minimum; a minimum of zeros of either
+//    sign may pick another zero than the reference's comparisons, which only the sign of a
+//    zero p can show -- and p is never -0, since a sum is -0 only if both terms are.
+//  * with p never -0, adding 0 instead of -0 on the axes not stepped changes nothing.
+//  * floor(p / size) of the rounded IEEE quotient equals the floor of the true one unless
+//    the quotient underflows: size is an integer, so p differs from a multiple k size by at
+//    least one ulp of p, more than half an ulp of k carries. And the true one is
+//    floor((floor(p) + 1/2) / size): that argument lies at least 1/(2 size) from every
+//    integer, so a reciprocal good to one ulp decides it for |p| <= 2^20 (error below
+//    0.2 / size). k size is an exact float, so p - k size in one fma rounds as the
+//    reference's product and difference do.
+// An underflowing quotient (p in (-2^-64, 0)) is looked at separately.
+constexpr float kFastBound = 0x1p20f;
+
+__device__ __forceinline__ bool axis_fast(float d, float inv, float p) {
+    constexpr float kInf = __builtin_inff();
+    const bool dir = (fabsf(d) < kInf && fabsf(inv) < kInf) ||
+                     (__float_as_uint(d) == 0u && (p >= 0.0f || p <= -0x1p-9f));
+    return dir && fabsf(p) < kInf && __float_as_uint(p) != 0x80000000u;
+}
+
+__device__ __forceinline__ bool lane_fast(const RayLane &r) {
+    return axis_fast(r.dx, r.ix, r.px) && axis_fast(r.dy, r.iy, r.py) && axis_fast(r.dz, r.iz, r.pz) &&
+           fmaxf(fmaxf(fabsf(r.dx), fabsf(r.dy)), fabsf(r.dz)) >= 0x1p-60f;
+}
+
+// The root lookup (get_vdb_leaf_from_nothing, :398-413): index of the first root entry
+// with the key of voxel (x, y, z), or -1.
+template <int kRoot>
+__device__ __forceinline__ int32_t root_find(const GridDev &g, int32_t x, int32_t y, int32_t z, const int4 *s_root,
+                                             bool root_lds) {
+    const int32_t kx = x >> 12, ky = y >> 12, kz = z >> 12;
+    if (kRoot == 0) return (kx == g.root0.x && ky == g.root0.y && kz == g.root0.z) ? g.root0.w : -1;
+    if (root_lds) {
+        for (uint32_t k = 0; k < g.n5count; ++k) {
+            const int4 e = s_root[k];
+            if (e.x == kx && e.y == ky && e.z == kz) return e.w;
+        }
+    } else {
+        for (uint32_t k = 0; k < g.n5count; ++k) {
+            const int4 e = g.root[k];
+            if (e.x == kx && e.y == ky && e.z == kz) return e.w;
+        }
+    }
+    return -1;
+}
+
+// The hdda_ray loop (raycast.comp.wgsl:92-123) of lanes that start together, to their end
+// (WX_HIT, WX_OOB, or WX_MAXSTEPS after kMaxSteps iterations): the trip count is a scalar,
+// and a lane's leaf lookups are its trips that ended at no other level.
+//  kFast  every running ray of the wave is fast (lane_fast) and the bound allows it
+//  kRoot  0: the grid has one node-5, its key in scalar registers; 1: a root table
+//  kWide  the leaf pool takes 64-bit addresses
+template <bool kFast, int kRoot, int kWide>
+__device__ __forceinline__ void lane_loop(const GridDev &g, RayLane &r, const int4 *s_root, bool root_lds) {
+    if (lane_state(r) != kRun) return;
+    float px = r.px, py = r.py, pz = r.pz, ax = 0.0f, ay = 0.0f, az = 0.0f;
+    const float gx = r.dx < 0.0f ? 0.0f : 1.0f, gy = r.dy < 0.0f ? 0.0f : 1.0f, gz = r.dz < 0.0f ? 0.0f : 1.0f;
+    const float nx = r.dx < 0.0f ? -4e-4f : 4e-4f, ny = r.dy < 0.0f ? -4e-4f : 4e-4f,
+                nz = r.dz < 0.0f ? -4e-4f : 4e-4f;
+    int32_t qx = 0, qy = 0, qz = 0;
+    // the least voxel difference the last lookup's cached nodes leave open: 4096 / 128 / 8
+    // after a lookup that ended at depth 0 / 1 / 2, 0 after a leaf lookup
+    uint32_t open = 4096u;
+    uint32_t i5 = 0, i4 = 0, i3 = 0, s01 = 0, s2 = 0, lk = 0, it = 0;
+    float size;
+    for (;;) {
+        float fx, fy, fz;
+        int32_t x, y, z;
+        fx = floorf(px), fy = floorf(py), fz = floorf(pz);
+        if (kFast) {
+            x = f2i_floor(px), y = f2i_floor(py), z = f2i_floor(pz);
+        } else {
+            x = f2i(fx), y = f2i(fy), z = f2i(fz);
+        }
+        // get_vdb_leaf_from_leaf (:360-396): the lookup starts at the deepest cached node
+        // that still contains the voxel
+        const uint32_t diff = (uint32_t)(x ^ qx) | (uint32_t)(y ^ qy) | (uint32_t)(z ^ qz) | open;
+        qx = x, qy = y, qz = z;
+        bool need5 = diff >= 128u, need4 = diff >= 8u, need3 = true;
+        if (diff >= 4096u) {
+            const int32_t found = root_find<kRoot>(g, x, y, z, s_root, root_lds);
+            i5 = (uint32_t)found;
+            if (found < 0) {  // dist 1 at depth 0 (:412)
+                size = 4096.0f;
+                open = 4096u;
+                s01 += 1u;
+                need5 = need4 = need3 = false;
+            }
+        }
+        if (need5) {  // get_vdb_leaf_from_node5 (:415-444)
+            lk += 1u;
+            // record (off >> 3) of 4096 16-byte records per node, off = x<<10 | y<<5 | z
+            const uint32_t rec = (((uint32_t)x >> 7) & 31u) << 7 | (((uint32_t)y >> 7) & 31u) << 2 |
+                                 (((uint32_t)z >> 7) & 31u) >> 3;
+            const uint4 q = load_rec(g.n5, (i5 << 16) | (rec << 4));
+            const uint32_t b = ((uint32_t)z >> 7) & 7u;
+            if ((q.x >> (8u + b)) & 1u) {
+                i4 = q.y + (uint32_t)__builtin_popcount(q.x & ((1u << b) - 1u));
+            } else {
+                const uint32_t dist = (uint32_t)((((uint64_t)q.w << 32) | q.z) >> (b * 8u)) & 0xFFu;
+                size = (float)dist * 128.0f;
+                open = 128u;
+                s01 += 1u << 16;
+                need4 = need3 = false;
+            }
+        }
+        if (need4) {  // get_vdb_leaf_from_node4 (:446-475)
+            lk += 1u << 10;
+            // record (off >> 4) of 256 per node, off = x<<8 | y<<4 | z
+            const uint32_t rec = (((uint32_t)x >> 3) & 15u) << 4 | (((uint32_t)y >> 3) & 15u);
+            const uint4 q = load_rec(g.n4, (i4 << 12) | (rec << 4));
+            const uint32_t b = ((uint32_t)z >> 3) & 15u;
+            if ((q.x >> (16u + b)) & 1u) {
+                i3 = q.y + (uint32_t)__builtin_popcount(q.x & ((1u << b) - 1u));
+            } else {
+                const uint32_t dist = (uint32_t)((((uint64_t)q.w << 32) | q.z) >> (b * 4u)) & 15u;
+                size = (float)dist * 8.0f;
+                open = 8u;
+                s2 += 1u;
+                need3 = false;
+            }
+        }
+        if (need3) {  // get_vdb_leaf_from_node3 (:477-494)
+            // word (off >> 3) of 64 per leaf holds 8 4-bit slots, off = x<<6 | y<<3 | z
+            const uint32_t w = load_leaf_word<kWide>(g, i3, ((uint32_t)x & 7u) << 5 | ((uint32_t)y & 7u) << 2);
+            size = (float)((w >> (((uint32_t)z & 7u) * 4u)) & 15u);
+            open = 0u;
+        }
         ++it;
-    } while (it < kMaxSteps && __builtin_amdgcn_ballot_w64(lane_state(r) == kRun) != 0ull);
-    if (lane_state(r) == kRun) set_state(r, WX_MAXSTEPS);
+        // :96-98 hit (distance 0), then :101-103 any(bound < |p|) (NaN components compare
+        // false either way)
+        const float hi = fmaxf(fmaxf(fabsf(px), fabsf(py)), fabsf(pz));
+        if (size == 0.0f || g.bound < hi) break;
+        // modulo_vec3f (:78-80): m = p - size * floor(p / size)
+        float mx, my, mz, tm;
+        bool bx, by, bz;
+        if (kFast) {
+            const float lo = fminf(fminf(fabsf(px), fabsf(py)), fabsf(pz));
+            if (lo < 0x1p-64f) {  // rare: a negative quotient that underflows has floor -0, not -1
+                if (fabsf(px) < 0x1p-64f && px / size == 0.0f) fx = 0.0f;
+                if (fabsf(py) < 0x1p-64f && py / size == 0.0f) fy = 0.0f;
+                if (fabsf(pz) < 0x1p-64f && pz / size == 0.0f) fz = 0.0f;
+            }
+            const float y1 = __builtin_amdgcn_rcpf(size), yh = 0.5f * y1;
+            mx = __builtin_fmaf(-size, floorf(__builtin_fmaf(fx, y1, yh)), px);
+            my = __builtin_fmaf(-size, floorf(__builtin_fmaf(fy, y1, yh)), py);
+            mz = __builtin_fmaf(-size, floorf(__builtin_fmaf(fz, y1, yh)), pz);
+        } else {
+            mx = px - size * floorf(px / size);
+            my = py - size * floorf(py / size);
+            mz = pz - size * floorf(pz / size);
+        }
+        // :114; size * max(0, sign) is size or 0, exact in the fma
+        const float tx = r.ix * __builtin_fmaf(size, gx, -mx);
+        const float ty = r.iy * __builtin_fmaf(size, gy, -my);
+        const float tz = r.iz * __builtin_fmaf(size, gz, -mz);
+        if (kFast) {  // :116, :118-120
+            tm = fminf(fminf(tx, ty), tz);
+            bx = tx == tm, by = ty == tm, bz = tz == tm;
+        } else {
+            tm = smin(smin(tx, ty), tz);
+            bx = (tx <= ty) & (tx <= tz);
+            by = (ty <= tz) & (ty <= tx);
+            bz = (tz <= tx) & (tz <= ty);
+        }
+        px = px + tm * r.dx;
+        py = py + tm * r.dy;
+        pz = pz + tm * r.dz;
+        // :122, p + (4e-4 * step) * f32(mask): the product is 4e-4 * step or a zero with
+        // the sign of step
+        ax = bx ? nx : (kFast ? 0.0f : 0.0f * nx);
+        ay = by ? ny : (kFast ? 0.0f : 0.0f * ny);
+        az = bz ? nz : (kFast ? 0.0f : 0.0f * nz);
+        px = px + ax;
+        py = py + ay;
+        pz = pz + az;
+        if (it == kMaxSteps) {
+            size = -1.0f;
+            break;
+        }
+    }
+    r.px = px, r.py = py, r.pz = pz;
+    r.ax = ax, r.ay = ay, r.az = az;
+    r.s01 = s01;
+    r.s23 = s2 | (it - (s01 & 0xFFFFu) - (s01 >> 16) - s2) << 16;
+    r.lk = lk;
+    r.state = size == 0.0f ? WX_HIT : (size < 0.0f ? WX_MAXSTEPS : WX_OOB);
 }
 
 // Runs the rays of a wave whose lanes all started together (the one-lane-per-ray
-// shapes) to their end (WX_HIT, WX_OOB, or WX_MAXSTEPS after kMaxSteps
-// iterations). The iteration count is the loop's trip count, a scalar; a wave
-// whose running rays are all clean takes the NaN-free step, any other wave the
-// general one. The grid-uniform choices (one node-5 or a root table, 32- or 64-bit
-// leaf addresses) are made once here, so the loop carries no branch on them.
-template <bool kN5Lds = false>
-__device__ __forceinline__ void lane_run(const GridDev &g, RayLane &r, const float2 *s_tab,
-                                         const uint4 *s_n5 = nullptr, const int4 *s_root = nullptr,
+// shapes) to their end. The choices that hold for the whole wave (fast rays, one node-5
+// or a root table, 32- or 64-bit leaf addresses) are made once here, so the loop carries
+// no branch on them. lane_start left the counters at zero.
+__device__ __forceinline__ void lane_run(const GridDev &g, RayLane &r, const int4 *s_root = nullptr,
                                          bool root_lds = false) {
-    const bool clean = __ballot(lane_state(r) == kRun && !lane_clean(r)) == 0ull;
+    const bool fast = g.bound <= kFastBound && __ballot(lane_state(r) == kRun && !lane_fast(r)) == 0ull;
     const bool one = g.n5count == 1u, wide = g.wide != 0u;
-    if (clean) {
-        if (one) {
-            if (wide) lane_loop<kN5Lds, true, 0, 1>(g, r, s_tab, s_n5, s_root, root_lds);
-            else lane_loop<kN5Lds, true, 0, 0>(g, r, s_tab, s_n5, s_root, root_lds);
-        } else {
-            if (wide) lane_loop<kN5Lds, true, 1, 1>(g, r, s_tab, s_n5, s_root, root_lds);
-            else lane_loop<kN5Lds, true, 1, 0>(g, r, s_tab, s_n5, s_root, root_lds);
-        }
-    } else {
-        if (one) {
-            if (wide) lane_loop<kN5Lds, false, 0, 1>(g, r, s_tab, s_n5, s_root, root_lds);
-            else lane_loop<kN5Lds, false, 0, 0>(g, r, s_tab, s_n5, s_root, root_lds);
-        } else {
-            if (wide) lane_loop<kN5Lds, false, 1, 1>(g, r, s_tab, s_n5, s_root, root_lds);
-            else lane_loop<kN5Lds, false, 1, 0>(g, r, s_tab, s_n5, s_root, root_lds);
-        }
-    }
+    if (fast && one && !wide) lane_loop<true, 0, 0>(g, r, s_root, root_lds);
+    else if (fast && one) lane_loop<true, 0, 1>(g, r, s_root, root_lds);
+    else if (fast && !wide) lane_loop<true, 1, 0>(g, r, s_root, root_lds);
+    else if (fast) lane_loop<true, 1, 1>(g, r, s_root, root_lds);
+    else if (!wide) lane_loop<false, 1, 0>(g, r, s_root, root_lds);
+    else lane_loop<false, 1, 1>(g, r, s_root, root_lds);
 }
 
 // cp_main (raycast.comp.wgsl:62-63): dir = normalize(p.x*u + p.y*mv + wp), p = pixel + offset,

@@ -212,8 +212,6 @@ __device__ void serve_poll(const ServeArgs &a) {
 // would otherwise hold it to 5 (measured 16 % slower on a burst of 256 requests);
 // the few spills it costs sit outside the traversal loops.
 __global__ __launch_bounds__(256, 8) void k_serve(ServeArgs a) {
-    __shared__ float2 s_tab[kTab];
-    init_tab(s_tab);
     if (blockIdx.x == 0 && threadIdx.x < 64u) {
         serve_poll(a);
         return;
@@ -322,14 +320,14 @@ __global__ __launch_bounds__(256, 8) void k_serve(ServeArgs a) {
                 camera_dir(q, px, py, dx, dy, dz);
                 RayLane r;
                 lane_start(r, q.ex, q.ey, q.ez, dx, dy, dz, g.bound, (q.flags & WX_TRACE_CLIP) != 0u);
-                lane_run(g, r, s_tab);
+                lane_run(g, r);
                 write_through(r, q.ex, q.ey, q.ez, q.out + pix);
                 if (q.flags & WX_TRACE_SHADOW) {
                     if (lane_state(r) == WX_HIT) {
                         float ox, oy, oz;
                         shadow_origin(r, ox, oy, oz);
                         start_shadow(r, q, g.bound, ox, oy, oz);
-                        lane_run(g, r, s_tab);
+                        lane_run(g, r);
                         write_through(r, ox, oy, oz, q.shadow + pix);
                     } else {
                         write_through_no_ray(q.shadow + pix);

@@ -12,8 +12,7 @@
 //    the queue is drained and its lanes are idle; every ray ends within 1000
 //    steps, so the grid always drains;
 //  * k_compact_camera: 16x16-pixel workgroups that move the rays of their emptiest
-//    wave into idle lanes of the others every `refill` iterations;
-//  * k_lds_camera: one lane per ray with the grid's node-5 records staged in LDS.
+//    wave into idle lanes of the others every `refill` iterations.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -44,9 +43,7 @@ constexpr uint32_t kMaxReqsLds = 1024u;
 // ---------------------------------------------------------------- simple shape
 
 // Shadow continuation of a finished primary in the same lane (WX_TRACE_SHADOW).
-template <bool kN5Lds = false>
 __device__ __forceinline__ void finish_with_shadow(const GridDev &g, const ReqDev &q, RayLane &r, uint32_t pix,
-                                                   const float2 *s_tab, const uint4 *s_n5 = nullptr,
                                                    const int4 *s_root = nullptr, bool root_lds = false) {
     if (lane_state(r) != WX_HIT) {
         write_no_ray(q.shadow + pix);
@@ -55,7 +52,7 @@ __device__ __forceinline__ void finish_with_shadow(const GridDev &g, const ReqDe
     float ox, oy, oz;
     shadow_origin(r, ox, oy, oz);
     start_shadow(r, q, g.bound, ox, oy, oz);
-    lane_run<kN5Lds>(g, r, s_tab, s_n5, s_root, root_lds);
+    lane_run(g, r, s_root, root_lds);
     lane_write(r, ox, oy, oz, q.shadow + pix);
 }
 
@@ -63,10 +60,8 @@ __device__ __forceinline__ void finish_with_shadow(const GridDev &g, const ReqDe
 // its slots for the next one sooner than a 16x16 one (measured faster).
 template <bool kShadow>
 __global__ __launch_bounds__(128) void k_simple_camera(GridDev g, ReqDev q, uint32_t band) {
-    __shared__ float2 s_tab[kTab];
     __shared__ int4 s_root_buf[kRootLds];
     const bool root_lds = stage_root(g, s_root_buf);
-    init_tab(s_tab);
     uint32_t bx, by;
     tile_of_block(band != 0u, bx, by);
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
@@ -77,50 +72,24 @@ __global__ __launch_bounds__(128) void k_simple_camera(GridDev g, ReqDev q, uint
     camera_dir(q, px, py, dx, dy, dz);
     RayLane r;
     lane_start(r, q.ex, q.ey, q.ez, dx, dy, dz, g.bound, (q.flags & WX_TRACE_CLIP) != 0u);
-    lane_run(g, r, s_tab, nullptr, s_root_buf, root_lds);
+    lane_run(g, r, s_root_buf, root_lds);
     const uint32_t pix = py * q.w + px;
     lane_write(r, q.ex, q.ey, q.ez, q.out + pix);
-    if (kShadow) finish_with_shadow(g, q, r, pix, s_tab, nullptr, s_root_buf, root_lds);
-}
-
-// The one-lane shape with the grid's single node-5 (4096 records, 64 KiB) staged in
-// LDS: a 1024-lane workgroup covers 32x32 pixels (sixteen 8x8 wave tiles), so two
-// workgroups (32 waves) share a CU's LDS. Node-5 lookups read LDS instead of the
-// cache hierarchy; everything else is k_simple_camera.
-template <bool kShadow>
-__global__ __launch_bounds__(1024) void k_lds_camera(GridDev g, ReqDev q) {
-    __shared__ float2 s_tab[kTab];
-    __shared__ uint4 s_n5[4096];
-    for (uint32_t i = threadIdx.x; i < 4096u; i += 1024u) s_n5[i] = g.n5[i];
-    init_tab(s_tab);  // its barrier also publishes s_n5
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t px = blockIdx.x * 32u + (wave & 3u) * 8u + (lane & 7u);
-    const uint32_t py = blockIdx.y * 32u + (wave >> 2) * 8u + (lane >> 3);
-    if (px >= q.w || py >= q.h) return;
-    float dx, dy, dz;
-    camera_dir(q, px, py, dx, dy, dz);
-    RayLane r;
-    lane_start(r, q.ex, q.ey, q.ez, dx, dy, dz, g.bound, (q.flags & WX_TRACE_CLIP) != 0u);
-    lane_run<true>(g, r, s_tab, s_n5);
-    const uint32_t pix = py * q.w + px;
-    lane_write(r, q.ex, q.ey, q.ez, q.out + pix);
-    if (kShadow) finish_with_shadow<true>(g, q, r, pix, s_tab, s_n5);
+    if (kShadow) finish_with_shadow(g, q, r, pix, s_root_buf, root_lds);
 }
 
 template <bool kShadow>
 __global__ __launch_bounds__(128) void k_simple_rays(GridDev g, ReqDev q) {
-    __shared__ float2 s_tab[kTab];
     __shared__ int4 s_root_buf[kRootLds];
     const bool root_lds = stage_root(g, s_root_buf);
-    init_tab(s_tab);
     const uint32_t i = blockIdx.x * 128u + threadIdx.x;
     if (i >= q.w) return;
     const float *p = reinterpret_cast<const float *>(q.rays + i);
     RayLane r;
     lane_start(r, p[0], p[1], p[2], p[3], p[4], p[5], g.bound, (q.flags & WX_TRACE_CLIP) != 0u);
-    lane_run(g, r, s_tab, nullptr, s_root_buf, root_lds);
+    lane_run(g, r, s_root_buf, root_lds);
     lane_write(r, p[0], p[1], p[2], q.out + i);
-    if (kShadow) finish_with_shadow(g, q, r, i, s_tab, nullptr, s_root_buf, root_lds);
+    if (kShadow) finish_with_shadow(g, q, r, i, s_root_buf, root_lds);
 }
 
 // ---------------------------------------------------------------- compact shape
@@ -238,8 +207,6 @@ struct BatchArgs {
 };
 
 __global__ __launch_bounds__(128) void k_simple_batch(BatchArgs a) {
-    __shared__ float2 s_tab[kTab];
-    init_tab(s_tab);
     const uint32_t slot = blockIdx.x * 128u + threadIdx.x;
     if (slot >= a.total) return;  // whole waves: every request has a multiple of 64 slots
     // so the 64 slots of a wave belong to one request: find it once per wave
@@ -270,9 +237,9 @@ __global__ __launch_bounds__(128) void k_simple_batch(BatchArgs a) {
     }
     RayLane r;
     lane_start(r, ox, oy, oz, dx, dy, dz, g.bound, (q.flags & WX_TRACE_CLIP) != 0u);
-    lane_run(g, r, s_tab);
+    lane_run(g, r);
     lane_write(r, ox, oy, oz, q.out + pix);
-    if (q.flags & WX_TRACE_SHADOW) finish_with_shadow(g, q, r, pix, s_tab);
+    if (q.flags & WX_TRACE_SHADOW) finish_with_shadow(g, q, r, pix);
 }
 
 // ---------------------------------------------------------------- persistent shape
@@ -804,17 +771,6 @@ int launch_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs
         return WX_OK;
     };
     hipError_t e;
-    if (t.persistent == 3u && one && q[0].kind == WX_REQ_CAMERA && grids[0]->dev.n5count == 1u) {
-        // LDS shape: the node-5 records in LDS
-        dim3 grid((q[0].w + 31u) / 32u, (q[0].h + 31u) / 32u, 1);
-        if (q[0].flags & WX_TRACE_SHADOW)
-            hipLaunchKernelGGL(k_lds_camera<true>, grid, dim3(1024), 0, stream, grids[0]->dev, q[0]);
-        else
-            hipLaunchKernelGGL(k_lds_camera<false>, grid, dim3(1024), 0, stream, grids[0]->dev, q[0]);
-        e = hipGetLastError();
-        if (e != hipSuccess) return hip_fail(e, "batch: launch");
-        return WX_OK;
-    }
     if (t.persistent == 2u && single && q[0].kind == WX_REQ_CAMERA) {
         // compact shape: primary camera rays, `refill` iterations between censuses
         dim3 grid((q[0].w + 15u) / 16u, (q[0].h + 15u) / 16u, 1);
@@ -823,7 +779,7 @@ int launch_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs
         if (e != hipSuccess) return hip_fail(e, "batch: launch");
         return WX_OK;
     }
-    if (t.persistent != 1u) {  // the one-lane shape (also for what the compact / LDS shapes do not cover)
+    if (t.persistent != 1u) {  // the one-lane shape (also for what the compact shape does not cover)
         if (one) {
             const bool sh = (q[0].flags & WX_TRACE_SHADOW) != 0u;
             if (q[0].kind == WX_REQ_CAMERA) {
@@ -1189,21 +1145,12 @@ int wx_autotune(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs,
         ms = acc / 3.f;
         return WX_OK;
     };
-    // the one-lane-per-ray shape, the LDS shape for a lone camera request on a grid
-    // with one node-5, the compact shape for a lone primary camera request (census
-    // intervals), then a coordinate search over the persistent shape: waves, refill,
+    // the one-lane-per-ray shape, the compact shape for a lone primary camera request
+    // (census intervals), then a coordinate search over the persistent shape: waves, refill,
     // chunk, XCD split
     {
         wx_tune c = default_tune();
         c.persistent = 0;
-        float ms;
-        rc = time_it(c, ms);
-        if (rc == WX_OK && ms < bms) bms = ms, bt = c;
-    }
-    if (rc == WX_OK && n_reqs == 1u && n_grids == 1u && reqs[0].kind == WX_REQ_CAMERA &&
-        grids[0]->dev.n5count == 1u) {
-        wx_tune c = default_tune();
-        c.persistent = 3;
         float ms;
         rc = time_it(c, ms);
         if (rc == WX_OK && ms < bms) bms = ms, bt = c;
