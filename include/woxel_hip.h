@@ -100,14 +100,9 @@ typedef struct wx_request {
 typedef struct wx_tune {
     uint32_t persistent;   /* 0: one lane per ray, one workgroup per 256 ray slots;
                               1: persistent waves refilled from a work queue (fields below);
-                              2: compact -- a lone primary camera request in 16x16 workgroups that
-                                 move the rays of their emptiest wave into idle lanes of the others
-                                 every `refill` iterations (other batches use shape 0);
-                              3: LDS -- a lone camera request (shadow rays too) on a grid with one
-                                 node-5: 32x32-pixel workgroups with the node-5 records staged in
-                                 LDS (other batches use shape 0) */
-    uint32_t refill;       /* 1: refill a wave's idle lanes once at least this many are idle (1..64);
-                              2: iterations between workgroup censuses */
+                              2, 3: as 0 (two shapes that measured slower than it: compacting
+                                 workgroups, node-5 records in LDS) */
+    uint32_t refill;       /* 1: refill a wave's idle lanes once at least this many are idle (1..64) */
     uint32_t chunk;        /* work slots a wave takes from the queue at once (multiple of 64) */
     uint32_t waves_per_cu; /* resident waves per CU launched (1..32) */
     uint32_t xcd_split;    /* shape 1: nonzero = one queue region per XCD, stealing when drained;
@@ -342,7 +337,7 @@ int wx_tune_set(const wx_tune *t);
  * requests and grids, and a shadow ray continues on-device in the lane of its
  * primary. The request table is copied to the device asynchronously on
  * `stream`; grids must stay alive until the work completes.
- * HIP graph capture: a call with one request on one grid in shape 0, 2 or 3
+ * HIP graph capture: a call with one request on one grid in any shape but 1
  * launches one kernel whose arguments are all passed by value, and may be captured
  * and replayed. Other calls (several requests or grids, shape 1) stage tables and
  * queue counters in per-stream scratch memory that later calls reuse or grow, and

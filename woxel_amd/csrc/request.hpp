@@ -21,12 +21,20 @@ struct ReqDev {
 };
 static_assert(sizeof(ReqDev) == 128, "ReqDev layout");
 
+// a + b with a as the first source: of two NaNs (a degenerate ray's) the sum is a in every
+// kernel, where the compiler may swap the operands of a plain sum.
+__device__ __forceinline__ float add_in_order(float a, float b) {
+    float r;
+    asm("v_add_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
 // The 32-byte hit record (wx_hit) of a finished lane as two 16-byte words; (ox, oy,
 // oz) is the ray origin before any clip.
 __device__ __forceinline__ void hit_words(const RayLane &r, float ox, float oy, float oz, uint4 &w0, uint4 &w1) {
     float t = (r.px - ox) * r.dx;
-    t = t + (r.py - oy) * r.dy;
-    t = t + (r.pz - oz) * r.dz;
+    t = add_in_order(t, (r.py - oy) * r.dy);
+    t = add_in_order(t, (r.pz - oz) * r.dz);
     const int32_t nx = r.ax != 0.0f ? (r.dx < 0.0f ? 1 : -1) : 0;
     const int32_t ny = r.ay != 0.0f ? (r.dy < 0.0f ? 1 : -1) : 0;
     const int32_t nz = r.az != 0.0f ? (r.dz < 0.0f ? 1 : -1) : 0;

@@ -10,9 +10,7 @@
 //    of the work queue (chunks come from per-XCD queue regions, with stealing).
 //    Shadow rays continue in the lane of their primary. Every wave exits once
 //    the queue is drained and its lanes are idle; every ray ends within 1000
-//    steps, so the grid always drains;
-//  * k_compact_camera: 16x16-pixel workgroups that move the rays of their emptiest
-//    wave into idle lanes of the others every `refill` iterations.
+//    steps, so the grid always drains.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -90,111 +88,6 @@ __global__ __launch_bounds__(128) void k_simple_rays(GridDev g, ReqDev q) {
     lane_run(g, r, s_root_buf, root_lds);
     lane_write(r, p[0], p[1], p[2], q.out + i);
     if (kShadow) finish_with_shadow(g, q, r, i, s_root_buf, root_lds);
-}
-
-// ---------------------------------------------------------------- compact shape
-
-// A camera request (primary rays only) traced by 256-lane workgroups of 16x16
-// pixels that keep their lanes busy: every `K` iterations the workgroup counts
-// the rays still running in each of its four waves; when the emptiest wave's
-// rays fit into the idle lanes of the other waves that still run, they move
-// there through LDS (the whole lane state, so results do not change) and that
-// wave idles. Every lane stays in the loop until the workgroup has no ray left
-// (the barriers need all 256), and every round advances each running ray by at
-// least one iteration, so the loop ends.
-constexpr int kLaneWords = 25;
-
-__device__ __forceinline__ void put_lane(uint32_t *buf, uint32_t slot, const RayLane &r, uint32_t pix) {
-    const uint32_t w[kLaneWords] = {
-        __float_as_uint(r.dx), __float_as_uint(r.dy), __float_as_uint(r.dz), __float_as_uint(r.ix),
-        __float_as_uint(r.iy), __float_as_uint(r.iz), __float_as_uint(r.px), __float_as_uint(r.py),
-        __float_as_uint(r.pz), __float_as_uint(r.ax), __float_as_uint(r.ay), __float_as_uint(r.az),
-        r.s01, r.s23, r.it, r.lk, r.np, r.state, (uint32_t)r.qx, (uint32_t)r.qy,
-        (uint32_t)r.qz, r.i5, r.i4, r.i3, pix};
-#pragma unroll
-    for (int k = 0; k < kLaneWords; ++k) buf[k * 64 + slot] = w[k];
-}
-
-__device__ __forceinline__ void get_lane(const uint32_t *buf, uint32_t slot, RayLane &r, uint32_t &pix) {
-    uint32_t w[kLaneWords];
-#pragma unroll
-    for (int k = 0; k < kLaneWords; ++k) w[k] = buf[k * 64 + slot];
-    r.dx = __uint_as_float(w[0]), r.dy = __uint_as_float(w[1]), r.dz = __uint_as_float(w[2]);
-    r.ix = __uint_as_float(w[3]), r.iy = __uint_as_float(w[4]), r.iz = __uint_as_float(w[5]);
-    r.px = __uint_as_float(w[6]), r.py = __uint_as_float(w[7]), r.pz = __uint_as_float(w[8]);
-    r.ax = __uint_as_float(w[9]), r.ay = __uint_as_float(w[10]), r.az = __uint_as_float(w[11]);
-    r.s01 = w[12], r.s23 = w[13];
-    r.it = w[14], r.lk = w[15], r.np = w[16], r.state = w[17];
-    r.qx = (int32_t)w[18], r.qy = (int32_t)w[19], r.qz = (int32_t)w[20];
-    r.i5 = w[21], r.i4 = w[22], r.i3 = w[23];
-    pix = w[24];
-}
-
-__global__ __launch_bounds__(256) void k_compact_camera(GridDev g, ReqDev q, uint32_t K) {
-    __shared__ float s_rcp[256];
-    __shared__ uint32_t s_buf[kLaneWords * 64];
-    __shared__ uint32_t s_cnt[4];
-    __shared__ int4 s_root_buf[kRootLds];
-    const bool root_lds = stage_root(g, s_root_buf);
-    init_rcp(s_rcp);
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t px = blockIdx.x * 16u + (wave & 1u) * 8u + (lane & 7u);
-    const uint32_t py = blockIdx.y * 16u + (wave >> 1) * 8u + (lane >> 3);
-    const uint64_t below = (1ull << lane) - 1ull;
-    RayLane r;
-    r.state = 0;
-    uint32_t pix = 0;
-    bool alive = false;
-    if (px < q.w && py < q.h) {
-        float dx, dy, dz;
-        camera_dir(q, px, py, dx, dy, dz);
-        lane_start(r, q.ex, q.ey, q.ez, dx, dy, dz, g.bound, (q.flags & WX_TRACE_CLIP) != 0u);
-        pix = py * q.w + px;
-        alive = true;
-    }
-    for (;;) {
-        if (alive) {
-            for (uint32_t k = 0; k < K && lane_state(r) == kRun; ++k)
-                lane_step(g, r, s_rcp, nullptr, s_root_buf, root_lds);
-            if (lane_state(r) != kRun) {
-                lane_write(r, q.ex, q.ey, q.ez, q.out + pix);
-                alive = false;
-            }
-        }
-        const uint64_t am = __ballot(alive);
-        if (lane == 0) s_cnt[wave] = (uint32_t)__popcll(am);
-        __syncthreads();
-        const uint32_t c0 = s_cnt[0], c1 = s_cnt[1], c2 = s_cnt[2], c3 = s_cnt[3];
-        const uint32_t c[4] = {c0, c1, c2, c3};
-        if (c0 + c1 + c2 + c3 == 0u) break;
-        // the emptiest wave that still runs, if the other running waves can take its rays
-        uint32_t src = 4u, running = 0u, room = 0u;
-        for (uint32_t w = 0; w < 4u; ++w)
-            if (c[w]) {
-                ++running;
-                if (src == 4u || c[w] < c[src]) src = w;
-            }
-        for (uint32_t w = 0; w < 4u; ++w)
-            if (c[w] && w != src) room += 64u - c[w];
-        if (running >= 2u && c[src] <= room) {
-            if (wave == src && alive) {
-                put_lane(s_buf, (uint32_t)__popcll(am & below), r, pix);
-                alive = false;
-            }
-            __syncthreads();
-            if (wave != src && c[wave] && !alive) {
-                uint32_t rank = 0;  // this idle lane's place among the idle lanes of the receiving waves
-                for (uint32_t w = 0; w < wave; ++w)
-                    if (c[w] && w != src) rank += 64u - c[w];
-                rank += (uint32_t)__popcll(~am & below);
-                if (rank < c[src]) {
-                    get_lane(s_buf, rank, r, pix);
-                    alive = true;
-                }
-            }
-        }
-        __syncthreads();
-    }
 }
 
 // Any batch, one lane per slot: slot s of the launch is request r's slot
@@ -291,68 +184,123 @@ struct WaveQueue {
     }
 };
 
-// One request (camera or ray list), no shadow rays: the single-request path.
-// Outer loop: refill idle lanes from the wave's chunk. Inner loop: step the
-// live lanes (the same body as the one-ray-per-lane kernel) until `refill`
-// lanes have finished or none is left.
+// Rays of one wave that are started and wait for a lane, in LDS: the wave starts 64 at a
+// time on full lanes (direction, reciprocals, entry clip: as many instructions as two
+// steps), and idle lanes take from here.
+struct ReadyRays {
+    float w[9][64];  // position, direction, reciprocal direction
+    uint32_t pix[64];
+};
+
+// The lanes of a wave within a persistent kernel: steps them until at most `keep` run.
+// trip counts the wave's iterations, start is the trip before a lane's first.
+template <bool kFast, uint32_t kForm>
+__device__ __forceinline__ void persist_run(const GridDev &g, RayLane &r, bool &running, bool &capped, uint32_t &trip,
+                                            uint32_t start, uint32_t keep, const int4 *s_root, bool root_lds) {
+    do {
+        ++trip;
+        if (running) {
+            running = lane_look<kFast, kForm>(g, r, s_root, root_lds);
+            if (running) {
+                lane_advance<kFast>(r);
+                if (trip - start == kMaxSteps) capped = true, running = false;
+            }
+        }
+    } while ((uint32_t)__popcll(__ballot(running)) > keep);
+}
+
+// One request (camera or ray list), no shadow rays: the single-request path. Once at
+// least `refill` lanes of a wave are idle, their records are written together and they
+// take new rays.
 template <uint32_t KIND>
 __global__ __launch_bounds__(256) void k_persist1(PersistArgs a, GridDev g, ReqDev q) {
-    __shared__ float2 s_tab[kTab];
     __shared__ int4 s_root_buf[kRootLds];
+    __shared__ ReadyRays s_ready[4];
     const bool root_lds = stage_root(g, s_root_buf);
-    init_tab(s_tab);
     const uint32_t lane = threadIdx.x & 63u;
+    ReadyRays &ready = s_ready[threadIdx.x >> 6];
     const uint64_t lt = (1ull << lane) - 1ull;
     const bool clip = (q.flags & WX_TRACE_CLIP) != 0u;
     WaveQueue wq;
     wq.init(a);
-    bool alive = false;
-    uint32_t pix = 0;
+    bool running = false, pending = false, capped = false;
+    uint32_t pix = 0, n_ready = 0, trip = 0, start = 0;
     RayLane r;
-    r.state = 0;
     for (;;) {
-        const uint64_t idle = __ballot(!alive);
-        const uint32_t nidle = (uint32_t)__popcll(idle);
-        wq.fetch(a, lane);
-        const uint32_t avail = wq.end - wq.cur;
-        const uint32_t rank = (uint32_t)__popcll(idle & lt);
-        if (!alive && rank < avail) {
-            const uint32_t s = wq.cur + rank;
+        if (pending && !running) {  // records of the rays that ended since the last refill
+            lane_finish(r, capped);
             if (KIND == WX_REQ_CAMERA) {
-                uint32_t px, py;
-                if (camera_pixel(q, s, px, py)) {
-                    float dx, dy, dz;
-                    camera_dir(q, px, py, dx, dy, dz);
-                    lane_start(r, q.ex, q.ey, q.ez, dx, dy, dz, g.bound, clip);
-                    pix = py * q.w + px;
-                    alive = true;
-                }
-            } else if (s < q.w) {
-                const float *p = reinterpret_cast<const float *>(q.rays + s);
-                lane_start(r, p[0], p[1], p[2], p[3], p[4], p[5], g.bound, clip);
-                pix = s;
-                alive = true;
+                lane_write(r, q.ex, q.ey, q.ez, q.out + pix);
+            } else {
+                const float *p = reinterpret_cast<const float *>(q.rays + pix);
+                lane_write(r, p[0], p[1], p[2], q.out + pix);
             }
+            pending = false;
         }
-        wq.cur += std::min(avail, nidle);
-        if (!__any(alive)) {
-            if (wq.drained(a)) break;
-            continue;
-        }
-        do {
-            if (alive) {
-                if (lane_state(r) == kRun) lane_step(g, r, s_tab, nullptr, s_root_buf, root_lds);
-                if (lane_state(r) != kRun) {
+        uint32_t n_idle = (uint32_t)__popcll(__ballot(!running));
+        while (n_idle) {
+            while (!n_ready) {  // start the next 64 slots; rays that miss the box end here
+                wq.fetch(a, lane);
+                const uint32_t n = std::min(wq.end - wq.cur, 64u);
+                if (!n) break;
+                const uint32_t s = wq.cur + lane;
+                wq.cur += n;
+                RayLane f;
+                f.state = WX_OOB;
+                uint32_t fp = s;
+                if (lane < n) {
                     if (KIND == WX_REQ_CAMERA) {
-                        lane_write(r, q.ex, q.ey, q.ez, q.out + pix);
-                    } else {
-                        const float *p = reinterpret_cast<const float *>(q.rays + pix);
-                        lane_write(r, p[0], p[1], p[2], q.out + pix);
+                        uint32_t px, py;
+                        if (camera_pixel(q, s, px, py)) {
+                            float dx, dy, dz;
+                            camera_dir(q, px, py, dx, dy, dz);
+                            fp = py * q.w + px;
+                            lane_start(f, q.ex, q.ey, q.ez, dx, dy, dz, g.bound, clip);
+                            if (lane_state(f) != kRun) lane_write(f, q.ex, q.ey, q.ez, q.out + fp);
+                        }
+                    } else if (s < q.w) {
+                        const float *p = reinterpret_cast<const float *>(q.rays + s);
+                        lane_start(f, p[0], p[1], p[2], p[3], p[4], p[5], g.bound, clip);
+                        if (lane_state(f) != kRun) lane_write(f, p[0], p[1], p[2], q.out + fp);
                     }
-                    alive = false;
                 }
+                const uint64_t m = __ballot(lane_state(f) == kRun);
+                if (lane_state(f) == kRun) {
+                    const uint32_t k = (uint32_t)__popcll(m & lt);
+                    ready.w[0][k] = f.px, ready.w[1][k] = f.py, ready.w[2][k] = f.pz;
+                    ready.w[3][k] = f.dx, ready.w[4][k] = f.dy, ready.w[5][k] = f.dz;
+                    ready.w[6][k] = f.ix, ready.w[7][k] = f.iy, ready.w[8][k] = f.iz;
+                    ready.pix[k] = fp;
+                }
+                n_ready = (uint32_t)__popcll(m);
+                // the wave's own LDS accesses stay in order; this keeps the compiler to it
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             }
-        } while ((uint32_t)__popcll(__ballot(!alive)) < a.refill);
+            if (!n_ready) break;
+            const uint32_t take = std::min(n_idle, n_ready);
+            const uint32_t rank = (uint32_t)__popcll(__ballot(!running) & lt);
+            if (!running && rank < take) {
+                const uint32_t k = n_ready - 1u - rank;
+                lane_resume(r, ready.w[0][k], ready.w[1][k], ready.w[2][k], ready.w[3][k], ready.w[4][k],
+                            ready.w[5][k], ready.w[6][k], ready.w[7][k], ready.w[8][k]);
+                pix = ready.pix[k];
+                start = trip;
+                capped = false;
+                running = pending = true;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            n_ready -= take;
+            n_idle -= take;
+        }
+        if (!__any(running)) break;  // every slot is started and no ray is left
+        const uint32_t keep = n_idle ? 0u : 64u - a.refill;  // idle lanes: the queue is drained
+        const bool fast = g.bound <= kFastBound && __ballot(running && !lane_fast(r)) == 0ull;
+        auto go = [&](auto step) { step(g, r, running, capped, trip, start, keep, s_root_buf, root_lds); };
+        if (fast && g.form == kOneRoot) go(persist_run<true, kOneRoot>);
+        else if (fast && g.form == kTable) go(persist_run<true, kTable>);
+        else if (fast) go(persist_run<true, kIndexed>);
+        else if (g.form != kIndexed) go(persist_run<false, kTable>);
+        else go(persist_run<false, kIndexed>);
     }
 }
 
@@ -361,19 +309,18 @@ __global__ __launch_bounds__(256) void k_persist1(PersistArgs a, GridDev g, ReqD
 // request's grid index in a register and reads that grid's descriptor from LDS
 // on each step; the 128-byte request record is read when a ray starts or ends.
 __global__ __launch_bounds__(256) void k_persist_batch(PersistArgs a) {
-    __shared__ float2 s_tab[kTab];
     __shared__ GridDev s_grid[kMaxGridsLds];
     __shared__ uint32_t s_begin[kMaxReqsLds + 1];
     __shared__ float s_org[3][256];
     for (uint32_t i = threadIdx.x; i < a.n_grids; i += 256u) s_grid[i] = a.grids[i];
     for (uint32_t i = threadIdx.x; i <= a.n_reqs; i += 256u) s_begin[i] = a.begin[i];
-    init_tab(s_tab);
+    __syncthreads();
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t lt = (1ull << lane) - 1ull;
     WaveQueue wq;
     wq.init(a);
-    bool alive = false, shadow = false;
-    uint32_t req = 0, gi = 0, pix = 0;
+    bool alive = false, shadow = false, slow = false;
+    uint32_t req = 0, gi = 0, pix = 0, it = 0;
     RayLane r;
     r.state = 0;
     for (;;) {
@@ -414,6 +361,8 @@ __global__ __launch_bounds__(256) void k_persist_batch(PersistArgs a) {
                     lane_start(r, ox, oy, oz, dx, dy, dz, s_grid[gi].bound, (q.flags & WX_TRACE_CLIP) != 0u);
                     s_org[0][threadIdx.x] = ox, s_org[1][threadIdx.x] = oy, s_org[2][threadIdx.x] = oz;
                     req = lo;
+                    it = 0;
+                    slow = s_grid[gi].bound > kFastBound || !lane_fast(r);
                     shadow = false;
                     alive = true;
                 }
@@ -426,31 +375,38 @@ __global__ __launch_bounds__(256) void k_persist_batch(PersistArgs a) {
         }
         if (alive) {
             const GridDev &g = s_grid[gi];
-            if (lane_state(r) == kRun) lane_step(g, r, s_tab);
+            if (lane_state(r) == kRun) {
+                ++it;
+                auto step = [&](auto look, auto advance) {
+                    const bool on = look(g, r, nullptr, false);
+                    if (on) advance(r);
+                    if (!on || it == kMaxSteps) lane_finish(r, on);
+                };
+                if (g.form == kIndexed) step(lane_look<false, kIndexed>, lane_advance<false>);
+                else if (__ballot(slow) == 0ull) step(lane_look<true, kTable>, lane_advance<true>);
+                else step(lane_look<false, kTable>, lane_advance<false>);
+            }
             if (lane_state(r) != kRun) {
                 const ReqDev &q = a.reqs[req];
                 const float ox = s_org[0][threadIdx.x], oy = s_org[1][threadIdx.x], oz = s_org[2][threadIdx.x];
-                if (shadow) {
-                    lane_write(r, ox, oy, oz, q.shadow + pix);
-                    alive = false;
-                } else {
-                    lane_write(r, ox, oy, oz, q.out + pix);
-                    alive = false;
-                    if (q.flags & WX_TRACE_SHADOW) {
-                        if (lane_state(r) == WX_HIT) {
-                            float sx, sy, sz;
-                            shadow_origin(r, sx, sy, sz);
-                            start_shadow(r, q, g.bound, sx, sy, sz);
-                            s_org[0][threadIdx.x] = sx, s_org[1][threadIdx.x] = sy, s_org[2][threadIdx.x] = sz;
-                            shadow = true;
-                            alive = true;
-                            if (lane_state(r) != kRun) {  // the shadow ray missed the bound box
-                                lane_write(r, sx, sy, sz, q.shadow + pix);
-                                alive = false;
-                            }
-                        } else {
-                            write_no_ray(q.shadow + pix);
+                lane_write(r, ox, oy, oz, (shadow ? q.shadow : q.out) + pix);
+                alive = false;
+                if (!shadow && (q.flags & WX_TRACE_SHADOW)) {
+                    if (lane_state(r) == WX_HIT) {
+                        float sx, sy, sz;
+                        shadow_origin(r, sx, sy, sz);
+                        start_shadow(r, q, g.bound, sx, sy, sz);
+                        s_org[0][threadIdx.x] = sx, s_org[1][threadIdx.x] = sy, s_org[2][threadIdx.x] = sz;
+                        it = 0;
+                        slow = g.bound > kFastBound || !lane_fast(r);
+                        shadow = true;
+                        alive = true;
+                        if (lane_state(r) != kRun) {  // the shadow ray missed the bound box
+                            lane_write(r, sx, sy, sz, q.shadow + pix);
+                            alive = false;
                         }
+                    } else {
+                        write_no_ray(q.shadow + pix);
                     }
                 }
             }
@@ -771,15 +727,7 @@ int launch_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs
         return WX_OK;
     };
     hipError_t e;
-    if (t.persistent == 2u && single && q[0].kind == WX_REQ_CAMERA) {
-        // compact shape: primary camera rays, `refill` iterations between censuses
-        dim3 grid((q[0].w + 15u) / 16u, (q[0].h + 15u) / 16u, 1);
-        hipLaunchKernelGGL(k_compact_camera, grid, dim3(256), 0, stream, grids[0]->dev, q[0], t.refill);
-        e = hipGetLastError();
-        if (e != hipSuccess) return hip_fail(e, "batch: launch");
-        return WX_OK;
-    }
-    if (t.persistent != 1u) {  // the one-lane shape (also for what the compact shape does not cover)
+    if (t.persistent != 1u) {  // the one-lane shape
         if (one) {
             const bool sh = (q[0].flags & WX_TRACE_SHADOW) != 0u;
             if (q[0].kind == WX_REQ_CAMERA) {
@@ -846,12 +794,51 @@ int launch_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs
     return WX_OK;
 }
 
+// Slot entries of the node pools (lane.hpp) from the layout's records: one record per
+// lane, its 8 (node-5) or 16 (node-4) slots written as 16-byte words. base[node] is taken
+// off the child indices of compact (2-byte) entries; base NULL makes 4-byte entries. Bound
+// by the entries written.
+template <int kSlots>
+__global__ __launch_bounds__(256) void k_expand(const uint4 *rec, uint64_t n, const uint32_t *base, int base_step,
+                                                uint4 *out) {
+    constexpr uint32_t kBits = 64u / kSlots, kMask = (1u << kBits) - 1u, kNodeRecs = kSlots == 8 ? 4096u : 256u;
+    constexpr float kVoxels = kSlots == 8 ? 128.0f : 8.0f;
+    for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256u) {
+        const uint4 q = rec[i];
+        const uint64_t dist = (uint64_t)q.w << 32 | q.z;
+        const uint32_t off = base ? base[(int64_t)(i / kNodeRecs) * base_step] : 0u;
+        uint32_t e[kSlots];
+#pragma unroll
+        for (uint32_t b = 0; b < (uint32_t)kSlots; ++b) {
+            const uint32_t size = __float_as_uint((float)(uint32_t)((dist >> (b * kBits)) & kMask) * kVoxels);
+            const uint32_t child = q.y - off + (uint32_t)__builtin_popcount(q.x & ((1u << b) - 1u));
+            const bool walk = (q.x >> (kSlots + b)) & 1u;
+            e[b] = base ? (walk ? kWalk | child : size >> 16) : (walk ? kWalk32 | child : size);
+        }
+        if (base) {
+#pragma unroll
+            for (uint32_t b = 0; b < (uint32_t)kSlots / 8u; ++b)
+                out[i * (kSlots / 8u) + b] =
+                    make_uint4(e[8u * b] | e[8u * b + 1u] << 16, e[8u * b + 2u] | e[8u * b + 3u] << 16,
+                               e[8u * b + 4u] | e[8u * b + 5u] << 16, e[8u * b + 6u] | e[8u * b + 7u] << 16);
+        } else {
+#pragma unroll
+            for (uint32_t b = 0; b < (uint32_t)kSlots / 4u; ++b)
+                out[i * (kSlots / 4u) + b] = make_uint4(e[4u * b], e[4u * b + 1u], e[4u * b + 2u], e[4u * b + 3u]);
+        }
+    }
+}
+
 // Every index the kernels derive from a descriptor stays inside its pool: root
 // entries name a node-5 below n5; a record that can be walked into has its walk
 // bits inside its child bits, and its first child plus its child count is at most
 // the child pool's size (the child of slot b is first + popcount(kids below b)).
-// Records are checked in parallel on the host; returns the first bad one.
-int check_desc(const wx_grid_desc *d, const char *who) {
+// Records are checked in parallel on the host; returns the first bad one. base receives
+// the entries' bases (GridDev::base: n5 in reverse, then n4) -- the least child index a
+// node's records walk into -- and compact whether every rank from there fits its entry.
+int check_desc(const wx_grid_desc *d, const char *who, std::vector<uint32_t> &base, bool &compact) {
+    base.assign((size_t)d->n5 + d->n4, 0u);
+    compact = true;
     for (uint32_t k = 0; k < d->n5; ++k) {
         const int32_t idx = d->root[4u * k + 3u];
         if (idx < 0 || (uint32_t)idx >= d->n5)
@@ -871,18 +858,27 @@ int check_desc(const wx_grid_desc *d, const char *who) {
         if (!L.n) continue;
         const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
         const uint64_t parts = std::min<uint64_t>(std::min<unsigned>(hw, 16u), (L.n + 65535u) / 65536u);
-        std::vector<uint64_t> bad(parts, ~0ull);
+        const uint64_t node_recs = L.kid_bits == 8u ? 4096u : 256u, nodes = L.n / node_recs;
+        std::vector<uint64_t> bad(parts, ~0ull), irregular(parts, 0u);
         auto scan = [&](uint64_t p) {
-            const uint64_t b = L.n * p / parts, e = L.n * (p + 1u) / parts;
             const uint32_t km = (1u << L.kid_bits) - 1u;
-            for (uint64_t i = b; i < e; ++i) {
-                const uint32_t w = L.rec[4u * i], first = L.rec[4u * i + 1u];
-                const uint32_t kids = w & km, walk = (w >> L.kid_bits) & km;
-                if (!walk) continue;
-                if ((walk & ~kids) || (uint64_t)first + (uint64_t)__builtin_popcount(kids) > L.child_pool) {
-                    bad[p] = i;
-                    return;
+            for (uint64_t node = nodes * p / parts; node < nodes * (p + 1u) / parts; ++node) {
+                uint64_t least = ~0ull, end = 0;
+                for (uint64_t i = node * node_recs; i < (node + 1u) * node_recs; ++i) {
+                    const uint32_t w = L.rec[4u * i], first = L.rec[4u * i + 1u];
+                    const uint32_t kids = w & km, walk = (w >> L.kid_bits) & km;
+                    if (!walk) continue;
+                    const uint64_t last = (uint64_t)first + (uint64_t)__builtin_popcount(kids);
+                    if ((walk & ~kids) || last > L.child_pool) {
+                        bad[p] = i;
+                        return;
+                    }
+                    least = std::min<uint64_t>(least, first);
+                    end = std::max(end, last);
                 }
+                if (least == ~0ull) continue;
+                base[L.kid_bits == 8u ? d->n5 - 1u - node : d->n5 + node] = (uint32_t)least;
+                if (end - least > node_recs * L.kid_bits) irregular[p] = 1u;
             }
         };
         if (parts <= 1u) {
@@ -896,6 +892,7 @@ int check_desc(const wx_grid_desc *d, const char *who) {
             if (b != ~0ull)
                 return set_error(WX_ERR_INVALID, std::string(who) + ": " + L.name + " record " +
                                                      std::to_string(b) + " walks into a child outside the pool");
+        for (uint64_t b : irregular) compact = compact && !b;
     }
     return WX_OK;
 }
@@ -921,10 +918,12 @@ int grid_new(const wx_grid_desc *d, const char *who, wx_grid **out) {
     // the traversal's fast quotient relies on |p| <= bound <= 2^100 after the bound test
     if (!(d->bound > 0.0f) || !(d->bound <= 0x1p100f))
         return set_error(WX_ERR_INVALID, w + ": bound must be in (0, 2^100]");
-    // the kernels address the node pools with 32-bit byte offsets (leaves with 64-bit indices)
+    // at most 4 GiB of records per node level
     if (d->n5 > (1u << 16) || d->n4 > (1u << 20))
         return set_error(WX_ERR_UNSUPPORTED, w + ": more than 65536 node-5 or 2^20 node-4 nodes");
-    if (int rc = check_desc(d, who)) return rc;
+    std::vector<uint32_t> base;
+    bool compact = true;
+    if (int rc = check_desc(d, who, base, compact)) return rc;
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) return set_error(WX_ERR_DEVICE, w + ": no HIP device");
     wx_grid *g = new (std::nothrow) wx_grid();
@@ -951,19 +950,56 @@ int grid_new(const wx_grid_desc *d, const char *who, wx_grid **out) {
             }
         }
     }
+    // the slot entries, made on the default stream after the copies and waited for, so the
+    // grid is complete for work on any stream
+    const uint64_t nrec[3] = {(uint64_t)d->n5 * 4096u, (uint64_t)d->n4 * 256u, base.size()};
+    const uint64_t rec_bytes[3] = {compact ? 16u : 32u, compact ? 32u : 64u, 4u};
+    hipError_t e = hipSuccess;
+    for (int k = 0; k < 3 && e == hipSuccess; ++k) {
+        const size_t n = std::max<size_t>(nrec[k] * rec_bytes[k], 16u);
+        e = hipMalloc(&g->entries[k], n);
+        if (e != hipSuccess) g->entries[k] = nullptr;
+        else g->bytes += n;
+    }
+    if (e != hipSuccess) {
+        wx_grid_destroy(g);
+        return set_error(e == hipErrorOutOfMemory ? WX_ERR_BUDGET : WX_ERR_DEVICE,
+                         w + ": hipMalloc: " + hipGetErrorString(e));
+    }
+    const uint32_t *dbase = static_cast<const uint32_t *>(g->entries[2]) + d->n5;
+    if (!base.empty()) e = hipMemcpy(g->entries[2], base.data(), base.size() * 4u, hipMemcpyHostToDevice);
+    for (int k = 0; k < 2 && e == hipSuccess; ++k) {
+        if (!nrec[k]) continue;
+        const uint4 *rec = static_cast<const uint4 *>(g->mem[1 + k]);
+        uint4 *out = static_cast<uint4 *>(g->entries[k]);
+        const dim3 blocks((uint32_t)std::min<uint64_t>((nrec[k] + 255u) / 256u, 8192u));
+        if (k == 0)
+            hipLaunchKernelGGL(k_expand<8>, blocks, dim3(256), 0, nullptr, rec, nrec[k], compact ? dbase - 1 : nullptr, -1,
+                               out);
+        else
+            hipLaunchKernelGGL(k_expand<16>, blocks, dim3(256), 0, nullptr, rec, nrec[k], compact ? dbase : nullptr, 1, out);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+    if (e != hipSuccess) {
+        wx_grid_destroy(g);
+        return hip_fail(e, (w + ": slot entries").c_str());
+    }
     g->dev.root = static_cast<const int4 *>(g->mem[0]);
-    g->dev.n5 = static_cast<const uint4 *>(g->mem[1]);
-    g->dev.n4 = static_cast<const uint4 *>(g->mem[2]);
+    g->dev.n5 = g->entries[0];
+    g->dev.n4 = g->entries[1];
     g->dev.leaf = static_cast<const uint32_t *>(g->mem[3]);
+    g->dev.base = dbase;
     g->dev.n5count = d->n5;
     g->dev.bound = d->bound;
     g->n5 = d->n5;
     g->n4 = d->n4;
     g->n3 = d->n3;
-    g->dev.root0 = d->n5 ? make_int4(d->root[0], d->root[1], d->root[2], d->root[3]) : make_int4(0, 0, 0, 0);
-    // WX_WIDE_LEAVES=1 takes the 64-bit leaf addressing at any size (to test it on small grids)
+    if (d->n5) g->dev.kx = d->root[0], g->dev.ky = d->root[1], g->dev.kz = d->root[2];
+    // WX_WIDE_LEAVES=1 takes the 64-bit pool addressing at any size (to test it on small grids)
     const char *wide = std::getenv("WX_WIDE_LEAVES");
-    g->dev.wide = (d->n3 > (1u << 24) || (wide && wide[0] == '1')) ? 1u : 0u;
+    const bool narrow = d->n3 <= (1u << 24) && !(wide && wide[0] == '1');
+    g->dev.form = !compact ? kIndexed : (d->n5 == 1u && base[0] == 0u && narrow ? kOneRoot : kTable);
     *out = g;
     return WX_OK;
 }
@@ -1035,6 +1071,8 @@ int wx_grid_destroy(wx_grid *g) {
     if (!g) return WX_OK;
     for (int k = 0; k < 4; ++k)
         if (g->mem[k]) (void)hipFree(g->mem[k]);
+    for (int k = 0; k < 3; ++k)
+        if (g->entries[k]) (void)hipFree(g->entries[k]);
     delete g;
     return WX_OK;
 }
@@ -1145,26 +1183,14 @@ int wx_autotune(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs,
         ms = acc / 3.f;
         return WX_OK;
     };
-    // the one-lane-per-ray shape, the compact shape for a lone primary camera request
-    // (census intervals), then a coordinate search over the persistent shape: waves, refill,
-    // chunk, XCD split
+    // the one-lane-per-ray shape, then a coordinate search over the persistent shape:
+    // waves, refill, chunk, XCD split
     {
         wx_tune c = default_tune();
         c.persistent = 0;
         float ms;
         rc = time_it(c, ms);
         if (rc == WX_OK && ms < bms) bms = ms, bt = c;
-    }
-    if (rc == WX_OK && n_reqs == 1u && n_grids == 1u && reqs[0].kind == WX_REQ_CAMERA &&
-        !(reqs[0].flags & WX_TRACE_SHADOW)) {
-        for (uint32_t k : {4u, 8u, 16u}) {
-            wx_tune c = default_tune();
-            c.persistent = 2;
-            c.refill = k;
-            float ms;
-            if ((rc = time_it(c, ms))) break;
-            if (ms < bms) bms = ms, bt = c;
-        }
     }
     wx_tune t = default_tune();
     t.persistent = 1;
