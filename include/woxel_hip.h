@@ -98,15 +98,19 @@ typedef struct wx_request {
 
 /* Launch shape of a traversal (see wx_autotune). */
 typedef struct wx_tune {
-    uint32_t persistent;   /* 0: one lane per ray, one workgroup per 256 ray slots;
-                              1: persistent waves refilled from a work queue (fields below);
+    uint32_t persistent;   /* 0: one lane per ray (a ray list of a million rays or more without
+                                 shadow rays also goes through refilled waves, for the runs of 64
+                                 whose directions have nothing in common);
+                              1: persistent waves whose idle lanes are refilled: one request in
+                                 equal shares, others from a work queue (fields below);
                               2, 3: as 0 (two shapes that measured slower than it: compacting
                                  workgroups, node-5 records in LDS) */
     uint32_t refill;       /* 1: refill a wave's idle lanes once at least this many are idle (1..64) */
-    uint32_t chunk;        /* work slots a wave takes from the queue at once (multiple of 64) */
-    uint32_t waves_per_cu; /* resident waves per CU launched (1..32) */
-    uint32_t xcd_split;    /* shape 1: nonzero = one queue region per XCD, stealing when drained;
-                              0 = one region. Shape 0 camera requests: 2 = each XCD takes one
+    uint32_t chunk;        /* 1, several requests: work slots a wave takes from the queue at once
+                              (multiple of 64) */
+    uint32_t waves_per_cu; /* 1: waves per CU launched (1..32) */
+    uint32_t xcd_split;    /* 1, several requests: nonzero = one queue region per XCD, stealing when
+                              drained; 0 = one region. Shape 0 camera requests: 2 = each XCD takes one
                               contiguous band of the image's 16x8 tiles, else the hardware's
                               round-robin of tiles over the XCDs */
 } wx_tune;
@@ -337,9 +341,9 @@ int wx_tune_set(const wx_tune *t);
  * requests and grids, and a shadow ray continues on-device in the lane of its
  * primary. The request table is copied to the device asynchronously on
  * `stream`; grids must stay alive until the work completes.
- * HIP graph capture: a call with one request on one grid in any shape but 1
- * launches one kernel whose arguments are all passed by value, and may be captured
- * and replayed. Other calls (several requests or grids, shape 1) stage tables and
+ * HIP graph capture: a call with one request on one grid launches kernels whose
+ * arguments are all passed by value, and may be captured and replayed (in shape 1
+ * without a shadow ray). Other calls (several requests or grids) stage tables and
  * queue counters in per-stream scratch memory that later calls reuse or grow, and
  * must not be captured. */
 int wx_trace_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs, uint32_t n_reqs,

@@ -131,3 +131,45 @@ def test_layouts_without_consecutive_children(wx, oracle_mod, cuda):
             wx.trace_batch([g], [wx.rays_request(0, t, out), wx.rays_request(0, t, out2)], tune)
             assert_hits_equal(wx.hits_to_numpy(out2), want, f"{name} batch {persistent}")
     assert wx.tune_get().as_dict() == old.as_dict()
+
+
+@pytest.mark.parametrize("n", [(1 << 20) - 1, (1 << 20) + 37])
+def test_long_ray_lists(wx, oracle_mod, cuda, n):
+    """Lists on both sides of the length at which scattered sets of 64 rays go to the
+    refilled waves: sets of one direction and scattered ones in turn, rays of the general
+    step and rays that meet the step cap among both."""
+    print(f"{n} rays", flush=True)
+    rng = np.random.default_rng(n)
+    org = np.array([(x, 0, 0) for x in range(0, 4096, 8)], np.int32)
+    masks = np.full((org.shape[0], 8), np.uint64(0xFF))
+    p = wx.Vdb345()
+    p.add_leaf_masks(org >> 3, masks)
+    p.add_spheres(np.array([[2000.0, 1500.0, 1800.0, 60.0], [700.0, 900.0, 2500.0, 45.0]]))
+    p.compute_sdf()
+    o = oracle_mod.Vdb()
+    o.add_leaf_masks(org, masks)
+    for s in ([2000.0, 1500.0, 1800.0, 60.0], [700.0, 900.0, 2500.0, 45.0]):
+        o.add_sphere(np.array(s[:3]), s[3])
+    o.compute_sdf()
+    g = wx.Grid(p)
+    m = (n + 63) // 64 * 64
+    eye = rng.uniform(-3000, 6000, (m, 3))
+    d = rng.uniform(-60, 60, (m, 3)) + np.where(rng.random((m, 1)) < 0.5, [[2000, 1500, 1800]], [[700, 900, 2500]]) - eye
+    rays = np.concatenate([eye, d], 1).reshape(-1, 64, 6)
+    rays[::3, :, :3] = rays[::3, :1, :3]  # one eye, neighbouring directions
+    rays[::3, :, 3:] = rays[::3, :1, 3:] + rng.uniform(-20, 20, rays[::3, :, 3:].shape)
+    rays = rays.reshape(m, 6)[:n].astype(np.float32)
+    rays[:, 3:] /= np.linalg.norm(rays[:, 3:], axis=1, keepdims=True)
+    k = rng.integers(0, n, 3000)
+    rays[k, 3 + rng.integers(0, 3, 3000)] = -0.0
+    k = rng.integers(0, n, 3000)
+    rays[k] = np.stack([np.full(3000, 0.5), 1.5 + k % 7, np.full(3000, 4.5), np.ones(3000), np.zeros(3000),
+                        np.zeros(3000)], 1)  # beside the wall: the step cap
+    t = cuda.from_numpy(rays).cuda()
+    ora, _ = o.trace_rays(rays, clip=True)
+    nan = np.isnan(ora["t"])
+    for simple in (False, True):
+        gpu = wx.hits_to_numpy(g.trace_rays(t, clip=True, simple=simple))
+        assert np.array_equal(np.isnan(gpu["t"]), nan)
+        assert_hits_equal(gpu[~nan], ora[~nan], f"{n} rays, simple={simple}")
+    assert {wx.HIT, wx.OOB, wx.MAXSTEPS} <= set(np.unique(gpu["state"]).tolist())

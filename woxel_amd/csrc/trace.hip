@@ -5,12 +5,12 @@
 //  * k_simple_*: one lane per ray, 8x8-pixel wave tiles (the reference's dispatch
 //    shape); camera tiles dealt round-robin over the XCDs, or in one band per XCD
 //    (wx_tune.xcd_split = 2: better L2 locality, worse balance -- measured slower);
-//  * k_persist*: persistent wave64 workers. A wave holds 64 rays; once `refill`
-//    lanes have finished, the idle lanes take the next slots of the wave's chunk
-//    of the work queue (chunks come from per-XCD queue regions, with stealing).
-//    Shadow rays continue in the lane of their primary. Every wave exits once
-//    the queue is drained and its lanes are idle; every ray ends within 1000
-//    steps, so the grid always drains.
+//  * k_persist1, k_persist_batch: wave64 workers that refill. Once `refill` lanes of a wave
+//    have finished, the idle lanes take new slots: of the wave's fixed share of the one
+//    request (also for the scattered sets of a long ray list in the one-lane shape), or of
+//    chunks of a batch's work queue (per-XCD regions, with stealing; shadow rays continue
+//    in the lane of their primary). Every wave exits once its slots are used up and its
+//    lanes are idle; every ray ends within 1000 steps, so the grid always drains.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -76,15 +76,30 @@ __global__ __launch_bounds__(128) void k_simple_camera(GridDev g, ReqDev q, uint
     if (kShadow) finish_with_shadow(g, q, r, pix, s_root_buf, root_lds);
 }
 
+// Whether a wave's rays (lanes with `in`, direction (x, y, z)) go the same way: at least
+// half of them within about 25 degrees of the first. A scan line, a panorama or a light's
+// rays do; of rays that have nothing to do with each other one in twenty does. Every lane
+// of the wave calls it.
+__device__ __forceinline__ bool rays_together(bool in, float x, float y, float z) {
+    auto lead = [](float v) { return __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(v))); };
+    const float x0 = lead(x), y0 = lead(y), z0 = lead(z);
+    const float c = x * x0 + y * y0 + z * z0;
+    const bool near = c > 0.0f && c * c > 0.81f * (x * x + y * y + z * z) * (x0 * x0 + y0 * y0 + z0 * z0);
+    return 2u * (uint32_t)__popcll(__ballot(in && near)) >= (uint32_t)__popcll(__ballot(in));
+}
+
+// split: only the waves whose rays go together trace theirs, k_persist1 the others'.
 template <bool kShadow>
-__global__ __launch_bounds__(128) void k_simple_rays(GridDev g, ReqDev q) {
+__global__ __launch_bounds__(128) void k_simple_rays(GridDev g, ReqDev q, uint32_t split) {
     __shared__ int4 s_root_buf[kRootLds];
     const bool root_lds = stage_root(g, s_root_buf);
     const uint32_t i = blockIdx.x * 128u + threadIdx.x;
+    const float *p = reinterpret_cast<const float *>(q.rays + std::min(i, q.w - 1u));
+    const float dx = p[3], dy = p[4], dz = p[5];
+    if (split && !rays_together(i < q.w, dx, dy, dz)) return;
     if (i >= q.w) return;
-    const float *p = reinterpret_cast<const float *>(q.rays + i);
     RayLane r;
-    lane_start(r, p[0], p[1], p[2], p[3], p[4], p[5], g.bound, (q.flags & WX_TRACE_CLIP) != 0u);
+    lane_start(r, p[0], p[1], p[2], dx, dy, dz, g.bound, (q.flags & WX_TRACE_CLIP) != 0u);
     lane_run(g, r, s_root_buf, root_lds);
     lane_write(r, p[0], p[1], p[2], q.out + i);
     if (kShadow) finish_with_shadow(g, q, r, i, s_root_buf, root_lds);
@@ -188,80 +203,81 @@ struct WaveQueue {
 // time on full lanes (direction, reciprocals, entry clip: as many instructions as two
 // steps), and idle lanes take from here.
 struct ReadyRays {
-    float w[9][64];  // position, direction, reciprocal direction
+    float w[12][64];  // position, direction, reciprocal direction, origin
     uint32_t pix[64];
 };
 
-// The lanes of a wave within a persistent kernel: steps them until at most `keep` run.
-// trip counts the wave's iterations, start is the trip before a lane's first.
-template <bool kFast, uint32_t kForm>
-__device__ __forceinline__ void persist_run(const GridDev &g, RayLane &r, bool &running, bool &capped, uint32_t &trip,
-                                            uint32_t start, uint32_t keep, const int4 *s_root, bool root_lds) {
-    do {
-        ++trip;
-        if (running) {
-            running = lane_look<kFast, kForm>(g, r, s_root, root_lds);
-            if (running) {
-                lane_advance<kFast>(r);
-                if (trip - start == kMaxSteps) capped = true, running = false;
-            }
-        }
-    } while ((uint32_t)__popcll(__ballot(running)) > keep);
+// The ray of slot s of a request; false when the slot has none (outside the image).
+template <uint32_t KIND>
+__device__ __forceinline__ bool slot_ray(const ReqDev &q, uint32_t s, uint32_t &pix, float *o, float *d) {
+    if (KIND == WX_REQ_CAMERA) {
+        uint32_t px, py;
+        if (!camera_pixel(q, s, px, py)) return false;
+        pix = py * q.w + px;
+        o[0] = q.ex, o[1] = q.ey, o[2] = q.ez;
+        camera_dir(q, px, py, d[0], d[1], d[2]);
+        return true;
+    }
+    if (s >= q.w) return false;
+    pix = s;
+    const float *p = reinterpret_cast<const float *>(q.rays + s);
+    o[0] = p[0], o[1] = p[1], o[2] = p[2], d[0] = p[3], d[1] = p[4], d[2] = p[5];
+    return true;
 }
 
-// One request (camera or ray list), no shadow rays: the single-request path. Once at
-// least `refill` lanes of a wave are idle, their records are written together and they
-// take new rays.
-template <uint32_t KIND>
-__global__ __launch_bounds__(256) void k_persist1(PersistArgs a, GridDev g, ReqDev q) {
+// One request (camera or ray list), no shadow rays, by n waves that each take every n-th
+// set of 64 slots and refill: once `refill` lanes are idle, their records are written
+// together and they take new rays. No counters in memory; rays that are not fast
+// (lane_fast) wait until the wave's others are done, so that the loop holds the fast step
+// of one grid form alone (64 VGPRs, eight waves per SIMD; 103 with the general step beside
+// it). With `split` the wave leaves out the sets whose rays go together: those lose by
+// refilling, which breaks up their lookups, and by a fixed share per wave (16.8 M panorama
+// rays: 2.05 ms one lane per ray, 2.56 refilled, 3.05 in fixed shares without refilling),
+// while scattered rays gain, as one lane per ray leaves nine lanes in ten idle (16.8 M:
+// 4.22 ms one lane per ray, 1.97 here).
+template <uint32_t KIND, uint32_t kForm>
+__global__ __launch_bounds__(256, 8) void k_persist1(GridDev g, ReqDev q, uint32_t total, uint32_t refill,
+                                                   uint32_t split) {
     __shared__ int4 s_root_buf[kRootLds];
     __shared__ ReadyRays s_ready[4];
+    __shared__ float s_org[3][256];
+    __shared__ uint32_t s_pix[256], s_start[256];
     const bool root_lds = stage_root(g, s_root_buf);
     const uint32_t lane = threadIdx.x & 63u;
     ReadyRays &ready = s_ready[threadIdx.x >> 6];
     const uint64_t lt = (1ull << lane) - 1ull;
-    const bool clip = (q.flags & WX_TRACE_CLIP) != 0u;
-    WaveQueue wq;
-    wq.init(a);
-    bool running = false, pending = false, capped = false;
-    uint32_t pix = 0, n_ready = 0, trip = 0, start = 0;
+    const bool clip = (q.flags & WX_TRACE_CLIP) != 0u, bounded = g.bound <= kFastBound;
+    const uint64_t stride = (uint64_t)gridDim.x * 256u, end = total;
+    const uint64_t first =
+        (uint64_t)blockIdx.x * 256u + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~63u));
+    uint64_t next = first;
+    bool running = false, pending = false, capped = false, slow = false;
+    uint32_t n_ready = 0, trip = 0, oldest = 0;
     RayLane r;
     for (;;) {
         if (pending && !running) {  // records of the rays that ended since the last refill
             lane_finish(r, capped);
-            if (KIND == WX_REQ_CAMERA) {
-                lane_write(r, q.ex, q.ey, q.ez, q.out + pix);
-            } else {
-                const float *p = reinterpret_cast<const float *>(q.rays + pix);
-                lane_write(r, p[0], p[1], p[2], q.out + pix);
-            }
+            lane_write(r, s_org[0][threadIdx.x], s_org[1][threadIdx.x], s_org[2][threadIdx.x], q.out + s_pix[threadIdx.x]);
             pending = false;
         }
         uint32_t n_idle = (uint32_t)__popcll(__ballot(!running));
         while (n_idle) {
-            while (!n_ready) {  // start the next 64 slots; rays that miss the box end here
-                wq.fetch(a, lane);
-                const uint32_t n = std::min(wq.end - wq.cur, 64u);
-                if (!n) break;
-                const uint32_t s = wq.cur + lane;
-                wq.cur += n;
+            while (!n_ready && next < end) {  // start the next 64 slots; rays that miss the box end here
+                const uint32_t s = (uint32_t)next + lane;
+                next += stride;
                 RayLane f;
                 f.state = WX_OOB;
-                uint32_t fp = s;
-                if (lane < n) {
-                    if (KIND == WX_REQ_CAMERA) {
-                        uint32_t px, py;
-                        if (camera_pixel(q, s, px, py)) {
-                            float dx, dy, dz;
-                            camera_dir(q, px, py, dx, dy, dz);
-                            fp = py * q.w + px;
-                            lane_start(f, q.ex, q.ey, q.ez, dx, dy, dz, g.bound, clip);
-                            if (lane_state(f) != kRun) lane_write(f, q.ex, q.ey, q.ez, q.out + fp);
-                        }
-                    } else if (s < q.w) {
-                        const float *p = reinterpret_cast<const float *>(q.rays + s);
-                        lane_start(f, p[0], p[1], p[2], p[3], p[4], p[5], g.bound, clip);
-                        if (lane_state(f) != kRun) lane_write(f, p[0], p[1], p[2], q.out + fp);
+                uint32_t fp = 0;
+                float o[3], d[3] = {0.0f, 0.0f, 0.0f};
+                const bool in = s < end && slot_ray<KIND>(q, s, fp, o, d);
+                if (KIND == WX_REQ_RAYS && split && rays_together(in, d[0], d[1], d[2])) continue;
+                if (in) {
+                    lane_start(f, o[0], o[1], o[2], d[0], d[1], d[2], g.bound, clip);
+                    if (lane_state(f) != kRun) {
+                        lane_write(f, o[0], o[1], o[2], q.out + fp);
+                    } else if (!(bounded && lane_fast(f))) {
+                        slow = true;
+                        f.state = WX_OOB;
                     }
                 }
                 const uint64_t m = __ballot(lane_state(f) == kRun);
@@ -270,6 +286,7 @@ __global__ __launch_bounds__(256) void k_persist1(PersistArgs a, GridDev g, ReqD
                     ready.w[0][k] = f.px, ready.w[1][k] = f.py, ready.w[2][k] = f.pz;
                     ready.w[3][k] = f.dx, ready.w[4][k] = f.dy, ready.w[5][k] = f.dz;
                     ready.w[6][k] = f.ix, ready.w[7][k] = f.iy, ready.w[8][k] = f.iz;
+                    ready.w[9][k] = o[0], ready.w[10][k] = o[1], ready.w[11][k] = o[2];
                     ready.pix[k] = fp;
                 }
                 n_ready = (uint32_t)__popcll(m);
@@ -283,8 +300,9 @@ __global__ __launch_bounds__(256) void k_persist1(PersistArgs a, GridDev g, ReqD
                 const uint32_t k = n_ready - 1u - rank;
                 lane_resume(r, ready.w[0][k], ready.w[1][k], ready.w[2][k], ready.w[3][k], ready.w[4][k],
                             ready.w[5][k], ready.w[6][k], ready.w[7][k], ready.w[8][k]);
-                pix = ready.pix[k];
-                start = trip;
+                for (uint32_t c = 0; c < 3u; ++c) s_org[c][threadIdx.x] = ready.w[9u + c][k];
+                s_pix[threadIdx.x] = ready.pix[k];
+                s_start[threadIdx.x] = trip;
                 capped = false;
                 running = pending = true;
             }
@@ -292,15 +310,37 @@ __global__ __launch_bounds__(256) void k_persist1(PersistArgs a, GridDev g, ReqD
             n_ready -= take;
             n_idle -= take;
         }
-        if (!__any(running)) break;  // every slot is started and no ray is left
-        const uint32_t keep = n_idle ? 0u : 64u - a.refill;  // idle lanes: the queue is drained
-        const bool fast = g.bound <= kFastBound && __ballot(running && !lane_fast(r)) == 0ull;
-        auto go = [&](auto step) { step(g, r, running, capped, trip, start, keep, s_root_buf, root_lds); };
-        if (fast && g.form == kOneRoot) go(persist_run<true, kOneRoot>);
-        else if (fast && g.form == kTable) go(persist_run<true, kTable>);
-        else if (fast) go(persist_run<true, kIndexed>);
-        else if (g.form != kIndexed) go(persist_run<false, kTable>);
-        else go(persist_run<false, kIndexed>);
+        if (!__any(running)) break;  // every slot is started and no fast ray is left
+        // no running ray started before trip `oldest`, so none meets the step cap before
+        // trip oldest + kMaxSteps
+        if (trip - oldest > kMaxSteps / 2u) {
+            uint32_t m = running ? trip - s_start[threadIdx.x] : 0u;
+            for (int d = 1; d < 64; d <<= 1) m = std::max(m, (uint32_t)__shfl_xor((int)m, d));
+            oldest = trip - (uint32_t)__builtin_amdgcn_readfirstlane((int)m);
+        }
+        const uint32_t keep = n_idle ? 0u : 64u - refill;  // idle lanes: there are no more slots
+        do {
+            ++trip;
+            if (running) {
+                running = opaque(lane_look<true, kForm>(g, r, s_root_buf, root_lds));
+                if (running) lane_advance<true>(r);
+            }
+            if (trip - oldest >= kMaxSteps && running && trip - s_start[threadIdx.x] == kMaxSteps)
+                capped = true, running = false;
+        } while ((uint32_t)__popcll(__ballot(running)) > keep);
+    }
+    if (!__any(slow)) return;
+    for (next = first; next < end; next += stride) {  // the rays that were left out, set by set
+        const uint32_t s = (uint32_t)next + lane;
+        uint32_t pix;
+        float o[3], d[3] = {0.0f, 0.0f, 0.0f};
+        const bool in = s < end && slot_ray<KIND>(q, s, pix, o, d);
+        if (KIND == WX_REQ_RAYS && split && rays_together(in, d[0], d[1], d[2])) continue;
+        if (!in) continue;
+        lane_start(r, o[0], o[1], o[2], d[0], d[1], d[2], g.bound, clip);
+        if (lane_state(r) != kRun || (bounded && lane_fast(r))) continue;
+        lane_loop<false, kForm == kIndexed ? kIndexed : kTable>(g, r, s_root_buf, root_lds);
+        lane_write(r, o[0], o[1], o[2], q.out + pix);
     }
 }
 
@@ -412,6 +452,15 @@ __global__ __launch_bounds__(256) void k_persist_batch(PersistArgs a) {
             }
         }
     }
+}
+
+template <uint32_t KIND>
+void launch_persist1(uint32_t blocks, hipStream_t stream, const GridDev &g, const ReqDev &q, uint32_t total,
+                     uint32_t refill, uint32_t split) {
+    const dim3 n(blocks), t(256);
+    if (g.form == kOneRoot) hipLaunchKernelGGL((k_persist1<KIND, kOneRoot>), n, t, 0, stream, g, q, total, refill, split);
+    else if (g.form == kTable) hipLaunchKernelGGL((k_persist1<KIND, kTable>), n, t, 0, stream, g, q, total, refill, split);
+    else hipLaunchKernelGGL((k_persist1<KIND, kIndexed>), n, t, 0, stream, g, q, total, refill, split);
 }
 
 int hip_fail(hipError_t e, const char *what) {
@@ -676,11 +725,12 @@ int upload_tables(wx_grid *const *grids, uint32_t n_grids, const ReqDev *q, cons
     return WX_OK;
 }
 
-// One launch over a validated batch, in the shape `t` selects. With a static
+// A batch, validated and launched in the shape `t` selects. may_split: a long ray list may
+// go to two kernels. With a static
 // staging the tables are built directly in the device's host staging area and no
 // memory is allocated.
 int launch_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs, uint32_t n_reqs,
-                 const wx_tune &t, hipStream_t stream, const Staging &stg = Staging()) {
+                 const wx_tune &t, hipStream_t stream, const Staging &stg = Staging(), bool may_split = true) {
     if (!tune_ok(t)) return set_error(WX_ERR_INVALID, "tune: out of range");
     std::vector<ReqDev> qv;
     std::vector<uint32_t> bv;
@@ -737,8 +787,19 @@ int launch_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs
                 else hipLaunchKernelGGL(k_simple_camera<false>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], band);
             } else {
                 dim3 grid((q[0].w + 127u) / 128u);
-                if (sh) hipLaunchKernelGGL(k_simple_rays<true>, grid, dim3(128), 0, stream, grids[0]->dev, q[0]);
-                else hipLaunchKernelGGL(k_simple_rays<false>, grid, dim3(128), 0, stream, grids[0]->dev, q[0]);
+                // a list with at least two sets of 64 rays for every wave the GPU holds goes to two
+                // kernels, each of which takes the sets that suit it (k_persist1): at 1 Mi rays
+                // scattered ones took 286 us against 346 in one kernel, a panorama 243 against 234;
+                // at half that scattered ones 251 against 193
+                const uint32_t sets = (q[0].w + 63u) / 64u, most = (uint32_t)cu_count() * 32u;
+                const uint32_t split = may_split && !sh && sets >= 2u * most ? 1u : 0u;
+                if (sh) hipLaunchKernelGGL(k_simple_rays<true>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], 0u);
+                else hipLaunchKernelGGL(k_simple_rays<false>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], split);
+                if (split) {
+                    const uint32_t per_wave = (sets + most - 1u) / most;
+                    launch_persist1<WX_REQ_RAYS>((sets + 4u * per_wave - 1u) / (4u * per_wave), stream, grids[0]->dev, q[0],
+                                                 q[0].w, 24u, 1u);
+                }
             }
         } else {
             BatchArgs b;
@@ -755,38 +816,30 @@ int launch_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs
         if (e != hipSuccess) return hip_fail(e, "batch: launch");
         return WX_OK;
     }
-    PersistArgs a;
-    std::memset(&a, 0, sizeof a);
-    a.n_grids = n_grids;
-    a.n_reqs = n_reqs;
-    a.total = (uint32_t)total;
-    a.regions = t.xcd_split ? kRegions : 1u;
-    a.refill = t.refill;
-    a.chunk = t.chunk;
-    const int cus = cu_count();
-    const uint32_t blocks = std::max<uint32_t>(1u, (uint32_t)cus * t.waves_per_cu / 4u);
     if (single) {
-        if (stg.is_static) {
-            a.ctr = reinterpret_cast<uint32_t *>(stg.dev + kOffCtr);
-        } else {
-            StreamScratch *S = nullptr;
-            int rc = scratch_for(stream, 1024, 0, &S);
-            if (rc) return rc;
-            a.ctr = reinterpret_cast<uint32_t *>(S->dev);
-        }
+        // as many waves as asked for at most, each with the same number of sets of 64 slots
+        const uint64_t sets = total / 64u, most = (uint64_t)cu_count() * t.waves_per_cu;
+        const uint64_t per_wave = (sets + most - 1u) / most;
+        const uint32_t blocks = (uint32_t)(((sets + per_wave - 1u) / per_wave + 3u) / 4u);
+        if (q[0].kind == WX_REQ_CAMERA)
+            launch_persist1<WX_REQ_CAMERA>(blocks, stream, grids[0]->dev, q[0], (uint32_t)total, t.refill, 0u);
+        else
+            launch_persist1<WX_REQ_RAYS>(blocks, stream, grids[0]->dev, q[0], q[0].w, t.refill, 0u);
     } else {
+        PersistArgs a;
+        std::memset(&a, 0, sizeof a);
+        a.n_grids = n_grids;
+        a.n_reqs = n_reqs;
+        a.total = (uint32_t)total;
+        a.regions = t.xcd_split ? kRegions : 1u;
+        a.refill = t.refill;
+        a.chunk = t.chunk;
         int rc = tables(&a.grids, &a.reqs, &a.begin, &a.ctr);
         if (rc) return rc;
-    }
-    // the queue counters start at zero: a fill kernel (no memset node, so the launch
-    // sequence stays valid inside a captured graph)
-    hipLaunchKernelGGL(k_zero, dim3(1), dim3(256), 0, stream, a.ctr, 16u * kRegions);
-    if (single) {
-        if (q[0].kind == WX_REQ_CAMERA)
-            hipLaunchKernelGGL(k_persist1<WX_REQ_CAMERA>, dim3(blocks), dim3(256), 0, stream, a, grids[0]->dev, q[0]);
-        else
-            hipLaunchKernelGGL(k_persist1<WX_REQ_RAYS>, dim3(blocks), dim3(256), 0, stream, a, grids[0]->dev, q[0]);
-    } else {
+        // the queue counters start at zero: a fill kernel (no memset node, so the launch
+        // sequence stays valid inside a captured graph)
+        hipLaunchKernelGGL(k_zero, dim3(1), dim3(256), 0, stream, a.ctr, 16u * kRegions);
+        const uint32_t blocks = std::max<uint32_t>(1u, (uint32_t)cu_count() * t.waves_per_cu / 4u);
         hipLaunchKernelGGL(k_persist_batch, dim3(blocks), dim3(256), 0, stream, a);
     }
     e = hipGetLastError();
@@ -901,7 +954,7 @@ int trace_one(wx_grid *g, const wx_request &in, uint32_t flags, hipStream_t stre
     wx_grid *gs[1] = {g};
     wx_tune t = current_tune();
     if (flags & WX_TRACE_SIMPLE) t.persistent = 0;
-    return launch_batch(gs, 1, &in, 1, t, stream);
+    return launch_batch(gs, 1, &in, 1, t, stream, Staging(), !(flags & WX_TRACE_SIMPLE));
 }
 
 }  // namespace
