@@ -25,8 +25,8 @@ struct GridDev {
     const void *n5;       // n5 x 32768 slot entries (below)
     const void *n4;       // n4 x 4096 slot entries
     const uint32_t *leaf; // n3 x 64 words
-    const uint32_t *base; // compact entries: base[i] = index of node-4 i's rank-0 leaf,
-                          // base[-1 - k] = index of node-5 k's rank-0 node-4
+    const uint32_t *base; // compact entries: base[i] + kWalk = index of node-4 i's rank-0 leaf,
+                          // base[-1 - k] + kWalk = index of node-5 k's rank-0 node-4
     uint32_t n5count;
     float bound;
     uint32_t form;        // kOneRoot, kTable or kIndexed
@@ -79,12 +79,11 @@ __device__ __forceinline__ int32_t f2i(float x) {
     return r;
 }
 
-// min(|a|, |b|, |c|, d) of numbers that are no NaN (the C functions would quiet signalling
+// min(|a|, |b|, |c|) of numbers that are no NaN (the C functions would quiet signalling
 // ones first, one instruction each).
-__device__ __forceinline__ float min4_abs(float a, float b, float c, float d) {
+__device__ __forceinline__ float min3_abs(float a, float b, float c) {
     float r;
     asm("v_min3_f32 %0, |%1|, |%2|, |%3|" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(r), "v"(d));
     return r;
 }
 
@@ -99,11 +98,11 @@ struct RayLane {
     float dx, dy, dz, ix, iy, iz, px, py, pz;
     float ax, ay, az;     // last nudge per axis
     uint32_t qx, qy, qz;  // last looked-up voxel, biased (voxel_bits)
-    uint32_t e5, e4;      // last node-5 / node-4 entry
+    uint32_t e5, e4;      // last node-5 / node-4 entry, as 4 bytes (an entry of 2 bytes in the upper half)
     uint32_t b5, b4;      // base of the last node-5 (not in kOneRoot, where it is 0) / node-4 looked up
     int32_t i5;           // node-5 index of the last root lookup, -1: none (not in kOneRoot)
-    uint32_t n5, miss, w5;  // node-5 lookups with root misses; root misses; node-5 walks
-    uint32_t n4, w4, n3;    // node-4 lookups; node-4 walks; leaf lookups
+    uint32_t c5, c4;      // node-5 (with root misses) / node-4 lookups | those that walked on << 15
+    uint32_t miss, n3;    // root misses; leaf lookups
     float fx, fy, fz;       // floor of the position last looked up
     float size;             // step size found there, 0: a hit
     uint32_t state;       // kRun or the final state
@@ -153,7 +152,7 @@ __device__ __forceinline__ void lane_resume(RayLane &r, float px, float py, floa
     r.ix = ix, r.iy = iy, r.iz = iz;
     r.ax = 0.0f, r.ay = 0.0f, r.az = 0.0f;
     r.s01 = 0, r.s23 = 0, r.lk = 0, r.state = kRun;
-    r.n5 = 0, r.miss = 0, r.w5 = 0, r.n4 = 0, r.w4 = 0, r.n3 = 0, r.qx = 0, r.qy = 0, r.qz = 0;
+    r.c5 = 0, r.c4 = 0, r.miss = 0, r.n3 = 0, r.qx = 0, r.qy = 0, r.qz = 0;
     r.e5 = 0, r.e4 = 0, r.b5 = 0, r.b4 = 0, r.i5 = -1;  // nothing cached
 }
 
@@ -253,27 +252,51 @@ __device__ __forceinline__ int32_t root_find(const GridDev &g, uint32_t x, uint3
     return -1;
 }
 
+// a's bits where the mask is set, b's elsewhere (in C the compiler masks both operands first);
+// acc | (a ^ b) and acc | (~a & b).
+__device__ __forceinline__ uint32_t bits_of(uint32_t mask, uint32_t a, uint32_t b) {
+    uint32_t r;
+    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "s"(mask), "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ uint32_t or_xor(uint32_t acc, uint32_t a, uint32_t b) {
+    return (uint32_t)__builtin_amdgcn_bitop3_b32((int)a, (int)b, (int)acc, 0xBE);
+}
+__device__ __forceinline__ uint32_t or_andn(uint32_t acc, uint32_t a, uint32_t b) {
+    return (uint32_t)__builtin_amdgcn_bitop3_b32((int)acc, (int)a, (int)b, 0xF2);
+}
+
+// a && b as the compiler cannot see through it: a flag in a scalar mask, not branches threaded
+// past the code that follows.
+__device__ __forceinline__ bool opaque_and(bool a, bool b) {
+    uint64_t m = __builtin_amdgcn_ballot_w64(a) & __builtin_amdgcn_ballot_w64(b);
+    asm volatile("" : "+s"(m));
+    return __builtin_amdgcn_inverse_ballot_w64(m);
+}
+
 // The lookup of one iteration (raycast.comp.wgsl:344-494): the step size at voxel (x, y, z).
 // Each level is one region of the lanes that need it, and no region nests in another: a
 // wave alone on its SIMD pays about 25 ns for a divergent region, six VALU instructions.
+// Large frames are bound by VALU issue (95 % of it on the 1080p sphere frame), so the regions
+// are written for their instruction count: offsets by bit-field inserts of shifted
+// coordinates, whose unwanted bits the last insert drops, and an entry's walk mark left in
+// an index and taken off its base instead.
 template <uint32_t kForm>
 __device__ __forceinline__ float lane_lookup(const GridDev &g, RayLane &r, uint32_t x, uint32_t y, uint32_t z,
                                              const int4 *s_root, bool root_lds) {
     // get_vdb_leaf_from_leaf (:360-396): the lookup starts at the deepest cached node that
     // still contains the voxel; a level whose entry was no walk is looked up again
-    constexpr uint32_t W = kForm == kIndexed ? kWalk32 : kWalk;
-    constexpr int kWBit = kForm == kIndexed ? 31 : 15, kUp = 31 - kWBit;  // an entry << kUp is the size's float
-    const uint32_t diff = (x ^ r.qx) | (y ^ r.qy) | (z ^ r.qz);
+    const uint32_t diff = or_xor(or_xor(x ^ r.qx, y, r.qy), z, r.qz);
     r.qx = x, r.qy = y, r.qz = z;
-    uint32_t bits = 0;
-    if ((diff | (~r.e5 & W)) >= 128u) {  // get_vdb_leaf_from_nothing / _node5 (:398-444)
+    if (or_andn(diff, r.e5, kWalk32) >= 128u) {  // get_vdb_leaf_from_nothing / _node5 (:398-444)
         bool miss;
+        uint32_t raw = 0;
         if (kForm == kOneRoot) {  // every slot lies inside the node, so a miss may read one too
             const uint32_t kx = kVoxelBias + ((uint32_t)g.kx << 12), ky = kVoxelBias + ((uint32_t)g.ky << 12),
                            kz = kVoxelBias + ((uint32_t)g.kz << 12);
-            const uint32_t off = (x & 0xF80u) << 4 | ((y >> 1) & 0x7C0u) | ((z >> 6) & 0x3Eu);
-            miss = ((x ^ kx) | (y ^ ky) | (z ^ kz)) >= 4096u;
-            r.e5 = pool_at<uint16_t, true, 16>(g.n5, 0u, off);
+            const uint32_t off = bits_of(0x3Eu, z >> 6, bits_of(0x7C0u, y >> 1, x << 4)) & 0xFFFEu;
+            raw = pool_at<uint16_t, true, 16>(g.n5, 0u, off);
+            miss = or_xor(or_xor(x ^ kx, y, ky), z, kz) >= 4096u;
         } else {
             const uint32_t slot = (x & 0xF80u) << 3 | (y & 0xF80u) >> 2 | (z & 0xF80u) >> 7;
             if (diff >= 4096u || r.i5 < 0) {
@@ -282,40 +305,46 @@ __device__ __forceinline__ float lane_lookup(const GridDev &g, RayLane &r, uint3
             }
             miss = r.i5 < 0;
             if (!miss)
-                r.e5 = kForm == kTable ? pool_at<uint16_t, false, 16>(g.n5, (uint32_t)r.i5, slot * 2u)
-                                       : pool_at<uint32_t, false, 17>(g.n5, (uint32_t)r.i5, slot * 4u);
+                raw = kForm == kTable ? pool_at<uint16_t, false, 16>(g.n5, (uint32_t)r.i5, slot * 2u)
+                                      : pool_at<uint32_t, false, 17>(g.n5, (uint32_t)r.i5, slot * 4u);
         }
-        if (miss) r.e5 = __float_as_uint(4096.0f) >> kUp;  // distance 1 at depth 0 (:412)
-        r.n5 += 1u;
+        constexpr int kUp = kForm == kIndexed ? 0 : 16;
+        if (miss) raw = __float_as_uint(4096.0f) >> kUp;  // distance 1 at depth 0 (:412)
+        r.c5 += kForm == kIndexed ? (raw >> 31 << 15) + 1u : (raw & kWalk) + 1u;
         r.miss += miss ? 1u : 0u;
-        r.w5 += r.e5 >> kWBit;
-        bits = r.e5 << kUp;
+        r.e5 = raw << kUp;
     }
-    if (((r.e5 & W) != 0u) & ((diff | (~r.e4 & W)) >= 8u)) {  // get_vdb_leaf_from_node4 (:446-475)
-        const uint32_t off = (x & 0x78u) << 6 | (y & 0x78u) << 2 | ((z >> 2) & 0x1Eu);
-        if (kForm == kOneRoot) {  // e5's kWalk is taken off the bases, not off the offset
+    const bool in4 = (int32_t)r.e5 < 0;
+    const uint32_t y2 = y << 2, z2 = z << 2;
+    if (in4 & (or_andn(diff, r.e4, kWalk32) >= 8u)) {  // get_vdb_leaf_from_node4 (:446-475)
+        if (kForm == kOneRoot) {
+            const uint32_t off = bits_of(0x1Eu, z >> 2, bits_of(0x1E0u, y2, x << 6));
             const char *n4 = static_cast<const char *>(g.n4) - ((size_t)kWalk << 13);
-            r.e4 = pool_at<uint16_t, true, 13>(n4, r.e5, off);
-            r.b4 = pool_at<uint32_t, true, 2>(g.base - kWalk, r.e5, 0u);
-        } else if (kForm == kTable) {
-            const uint32_t i4 = (r.e5 & ~kWalk) + r.b5;
-            r.e4 = pool_at<uint16_t, false, 13>(g.n4, i4, off);
-            r.b4 = g.base[i4];
+            const uint32_t raw = pool_at<uint16_t, true, 0>(n4, 0u, bits_of(0x1FFEu, off, r.e5 >> 3));
+            r.b4 = pool_at<uint32_t, true, 0>(g.base - kWalk, 0u, r.e5 >> 14);
+            r.c4 += (raw & kWalk) + 1u;
+            r.e4 = raw << 16;
         } else {
-            r.e4 = pool_at<uint32_t, false, 14>(g.n4, r.e5 & ~kWalk32, off * 2u);
+            const uint32_t off = (x & 0x78u) << 6 | (y & 0x78u) << 2 | ((z >> 2) & 0x1Eu);
+            if (kForm == kTable) {
+                const uint32_t i4 = (r.e5 >> 16) + r.b5;
+                r.e4 = (uint32_t)pool_at<uint16_t, false, 13>(g.n4, i4, off) << 16;
+                r.b4 = g.base[i4];
+            } else {
+                r.e4 = pool_at<uint32_t, false, 14>(g.n4, r.e5 & ~kWalk32, off * 2u);
+            }
+            r.c4 += (r.e4 >> 31 << 15) + 1u;
         }
-        r.n4 += 1u;
-        r.w4 += r.e4 >> kWBit;
-        bits = r.e4 << kUp;
     }
-    if ((r.e5 & r.e4 & W) != 0u) {  // get_vdb_leaf_from_node3 (:477-494)
+    float size = __uint_as_float(in4 ? r.e4 : r.e5);
+    if (in4 & ((int32_t)r.e4 < 0)) {  // get_vdb_leaf_from_node3 (:477-494)
         // word (off >> 3) of 64 per leaf holds 8 4-bit slots, off = x<<6 | y<<3 | z
-        const uint32_t leaf = kForm == kIndexed ? r.e4 & ~kWalk32 : r.b4 + (r.e4 & ~kWalk);
-        const uint32_t w = pool_at<uint32_t, kForm == kOneRoot, 8>(g.leaf, leaf, (x & 7u) << 5 | (y & 7u) << 2);
+        const uint32_t leaf = kForm == kIndexed ? r.e4 & ~kWalk32 : r.b4 + (r.e4 >> 16);
+        const uint32_t w = pool_at<uint32_t, kForm == kOneRoot, 8>(g.leaf, leaf, bits_of(0x1Cu, y2, x << 5) & 0xFCu);
         r.n3 += 1u;
-        bits = __float_as_uint((float)((w >> ((z & 7u) << 2)) & 15u));
+        size = (float)__builtin_amdgcn_ubfe(w, z2, 4u);  // the shift takes 5 bits: (z & 7) * 4
     }
-    return __uint_as_float(bits);
+    return size;
 }
 
 // First half of an iteration of the hdda_ray loop (raycast.comp.wgsl:92-103): looks the
@@ -332,16 +361,11 @@ __device__ __forceinline__ bool lane_look(const GridDev &g, RayLane &r, const in
                                     (uint32_t)f2i(r.fz) + kVoxelBias, s_root, root_lds);
     // :96-98 hit (distance 0), then :101-103 any(bound < |p|) (NaN components compare
     // false either way)
-    const bool out = g.bound < fmaxf(fmaxf(fabsf(r.px), fabsf(r.py)), fabsf(r.pz));
-    if (!kFast) return !(out | (r.size == 0.0f));
-    bool run = true;
-    if (out | (min4_abs(r.px, r.py, r.pz, r.size) < 0x1p-64f)) {  // one test for the ends and the tiny p
-        run = !(out | (r.size == 0.0f));
-        if (run) {  // a negative quotient that underflows has floor -0, not -1
-            if (fabsf(r.px) < 0x1p-64f && r.px / r.size == 0.0f) r.fx = 0.0f;
-            if (fabsf(r.py) < 0x1p-64f && r.py / r.size == 0.0f) r.fy = 0.0f;
-            if (fabsf(r.pz) < 0x1p-64f && r.pz / r.size == 0.0f) r.fz = 0.0f;
-        }
+    const bool run = opaque_and(!(g.bound < fmaxf(fmaxf(fabsf(r.px), fabsf(r.py)), fabsf(r.pz))), r.size != 0.0f);
+    if (kFast && min3_abs(r.px, r.py, r.pz) < 0x1p-64f) {  // a negative quotient that underflows has floor -0, not -1
+        if (fabsf(r.px) < 0x1p-64f && r.px / r.size == 0.0f) r.fx = 0.0f;
+        if (fabsf(r.py) < 0x1p-64f && r.py / r.size == 0.0f) r.fy = 0.0f;
+        if (fabsf(r.pz) < 0x1p-64f && r.pz / r.size == 0.0f) r.fz = 0.0f;
     }
     return run;
 }
@@ -392,19 +416,11 @@ __device__ __forceinline__ void lane_advance(RayLane &r) {
 
 // The state and the record words of a lane whose ray ended, or met the step cap.
 __device__ __forceinline__ void lane_finish(RayLane &r, bool capped) {
-    const uint32_t l5 = r.n5 - r.miss, s1 = l5 - r.w5, s2 = r.n4 - r.w4;
-    r.s01 = r.miss | s1 << 16;
-    r.s23 = s2 | r.n3 << 16;
-    r.lk = l5 | r.n4 << 10;
+    const uint32_t l5 = (r.c5 & 0x7FFFu) - r.miss, n4 = r.c4 & 0x7FFFu;
+    r.s01 = r.miss | (l5 - (r.c5 >> 15)) << 16;
+    r.s23 = (n4 - (r.c4 >> 15)) | r.n3 << 16;
+    r.lk = l5 | n4 << 10;
     r.state = capped ? WX_MAXSTEPS : (r.size == 0.0f ? WX_HIT : WX_OOB);
-}
-
-// b as the compiler cannot see through it: a flag in a scalar mask, not branches threaded
-// past the code that follows.
-__device__ __forceinline__ bool opaque(bool b) {
-    uint64_t m = __builtin_amdgcn_ballot_w64(b);
-    asm volatile("" : "+s"(m));
-    return __builtin_amdgcn_inverse_ballot_w64(m);
 }
 
 // The rays of a wave whose lanes start together, to their end: the trip count, and with it
@@ -413,12 +429,12 @@ __device__ __forceinline__ bool opaque(bool b) {
 template <bool kFast, uint32_t kForm>
 __device__ __forceinline__ void lane_loop(const GridDev &g, RayLane &r, const int4 *s_root, bool root_lds) {
     if (lane_state(r) != kRun) return;
-    bool run = opaque(lane_look<kFast, kForm>(g, r, s_root, root_lds));
+    bool run = lane_look<kFast, kForm>(g, r, s_root, root_lds);
     if (run) {
         uint32_t looks = 1;
         do {
             lane_advance<kFast>(r);
-            run = opaque(lane_look<kFast, kForm>(g, r, s_root, root_lds));
+            run = lane_look<kFast, kForm>(g, r, s_root, root_lds);
         } while (run && ++looks < kMaxSteps);
         if (run) lane_advance<kFast>(r);
     }

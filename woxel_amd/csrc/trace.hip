@@ -322,7 +322,7 @@ __global__ __launch_bounds__(256, 8) void k_persist1(GridDev g, ReqDev q, uint32
         do {
             ++trip;
             if (running) {
-                running = opaque(lane_look<true, kForm>(g, r, s_root_buf, root_lds));
+                running = lane_look<true, kForm>(g, r, s_root_buf, root_lds);
                 if (running) lane_advance<true>(r);
             }
             if (trip - oldest >= kMaxSteps && running && trip - s_start[threadIdx.x] == kMaxSteps)
@@ -848,8 +848,9 @@ int launch_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs
 }
 
 // Slot entries of the node pools (lane.hpp) from the layout's records: one record per
-// lane, its 8 (node-5) or 16 (node-4) slots written as 16-byte words. base[node] is taken
-// off the child indices of compact (2-byte) entries; base NULL makes 4-byte entries. Bound
+// lane, its 8 (node-5) or 16 (node-4) slots written as 16-byte words. base[node],
+// which is kWalk less than the node's first child, is taken off the child indices of compact
+// (2-byte) entries; base NULL makes 4-byte entries. Bound
 // by the entries written.
 template <int kSlots>
 __global__ __launch_bounds__(256) void k_expand(const uint4 *rec, uint64_t n, const uint32_t *base, int base_step,
@@ -866,7 +867,7 @@ __global__ __launch_bounds__(256) void k_expand(const uint4 *rec, uint64_t n, co
             const uint32_t size = __float_as_uint((float)(uint32_t)((dist >> (b * kBits)) & kMask) * kVoxels);
             const uint32_t child = q.y - off + (uint32_t)__builtin_popcount(q.x & ((1u << b) - 1u));
             const bool walk = (q.x >> (kSlots + b)) & 1u;
-            e[b] = base ? (walk ? kWalk | child : size >> 16) : (walk ? kWalk32 | child : size);
+            e[b] = base ? (walk ? child : size >> 16) : (walk ? kWalk32 | child : size);  // base holds kWalk off
         }
         if (base) {
 #pragma unroll
@@ -888,9 +889,9 @@ __global__ __launch_bounds__(256) void k_expand(const uint4 *rec, uint64_t n, co
 // the child pool's size (the child of slot b is first + popcount(kids below b)).
 // Records are checked in parallel on the host; returns the first bad one. base receives
 // the entries' bases (GridDev::base: n5 in reverse, then n4) -- the least child index a
-// node's records walk into -- and compact whether every rank from there fits its entry.
+// node's records walk into, less kWalk -- and compact whether every rank from there fits its entry.
 int check_desc(const wx_grid_desc *d, const char *who, std::vector<uint32_t> &base, bool &compact) {
-    base.assign((size_t)d->n5 + d->n4, 0u);
+    base.assign((size_t)d->n5 + d->n4, 0u - kWalk);
     compact = true;
     for (uint32_t k = 0; k < d->n5; ++k) {
         const int32_t idx = d->root[4u * k + 3u];
@@ -930,7 +931,7 @@ int check_desc(const wx_grid_desc *d, const char *who, std::vector<uint32_t> &ba
                     end = std::max(end, last);
                 }
                 if (least == ~0ull) continue;
-                base[L.kid_bits == 8u ? d->n5 - 1u - node : d->n5 + node] = (uint32_t)least;
+                base[L.kid_bits == 8u ? d->n5 - 1u - node : d->n5 + node] = (uint32_t)least - kWalk;
                 if (end - least > node_recs * L.kid_bits) irregular[p] = 1u;
             }
         };
@@ -1052,7 +1053,7 @@ int grid_new(const wx_grid_desc *d, const char *who, wx_grid **out) {
     // WX_WIDE_LEAVES=1 takes the 64-bit pool addressing at any size (to test it on small grids)
     const char *wide = std::getenv("WX_WIDE_LEAVES");
     const bool narrow = d->n3 <= (1u << 24) && !(wide && wide[0] == '1');
-    g->dev.form = !compact ? kIndexed : (d->n5 == 1u && base[0] == 0u && narrow ? kOneRoot : kTable);
+    g->dev.form = !compact ? kIndexed : (d->n5 == 1u && base[0] == 0u - kWalk && narrow ? kOneRoot : kTable);
     *out = g;
     return WX_OK;
 }
