@@ -54,18 +54,19 @@ __device__ __forceinline__ void finish_with_shadow(const GridDev &g, const ReqDe
     lane_write(r, ox, oy, oz, q.shadow + pix);
 }
 
-// 128-lane workgroups of two 8x8 wave tiles (16x8 pixels): a finished workgroup frees
-// its slots for the next one sooner than a 16x16 one (measured faster).
+// 128-lane workgroups of two wave tiles (8x8 pixels at 64 rays per wave: 16x8 pixels): a
+// finished workgroup frees its slots for the next one sooner than a 16x16 one (measured
+// faster). lg: rays_per_wave_log2.
 template <bool kShadow>
-__global__ __launch_bounds__(128) void k_simple_camera(GridDev g, ReqDev q, uint32_t band) {
+__global__ __launch_bounds__(128) void k_simple_camera(GridDev g, ReqDev q, uint32_t lg, uint32_t band) {
     __shared__ int4 s_root_buf[kRootLds];
     const bool root_lds = stage_root(g, s_root_buf);
     uint32_t bx, by;
     tile_of_block(band != 0u, bx, by);
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t px = bx * 16u + wave * 8u + (lane & 7u);
-    const uint32_t py = by * 8u + (lane >> 3);
-    if (px >= q.w || py >= q.h) return;
+    const uint32_t lw = (lg + 1u) >> 1, px = ((bx * 2u + wave) << lw) + (lane & ((1u << lw) - 1u));
+    const uint32_t py = (by << (lg >> 1)) + (lane >> lw);
+    if (lane >> lg || px >= q.w || py >= q.h) return;
     float dx, dy, dz;
     camera_dir(q, px, py, dx, dy, dz);
     RayLane r;
@@ -90,14 +91,14 @@ __device__ __forceinline__ bool rays_together(bool in, float x, float y, float z
 
 // split: only the waves whose rays go together trace theirs, k_persist1 the others'.
 template <bool kShadow>
-__global__ __launch_bounds__(128) void k_simple_rays(GridDev g, ReqDev q, uint32_t split) {
+__global__ __launch_bounds__(128) void k_simple_rays(GridDev g, ReqDev q, uint32_t lg, uint32_t split) {
     __shared__ int4 s_root_buf[kRootLds];
     const bool root_lds = stage_root(g, s_root_buf);
-    const uint32_t i = blockIdx.x * 128u + threadIdx.x;
+    const uint32_t lane = threadIdx.x & 63u, i = ((blockIdx.x * 2u + (threadIdx.x >> 6)) << lg) + lane;
     const float *p = reinterpret_cast<const float *>(q.rays + std::min(i, q.w - 1u));
     const float dx = p[3], dy = p[4], dz = p[5];
     if (split && !rays_together(i < q.w, dx, dy, dz)) return;
-    if (i >= q.w) return;
+    if (lane >> lg || i >= q.w) return;
     RayLane r;
     lane_start(r, p[0], p[1], p[2], dx, dy, dz, g.bound, (q.flags & WX_TRACE_CLIP) != 0u);
     lane_run(g, r, s_root_buf, root_lds);
@@ -111,12 +112,12 @@ struct BatchArgs {
     const GridDev *grids;
     const ReqDev *reqs;
     const uint32_t *begin;
-    uint32_t n_grids, n_reqs, total, pad;
+    uint32_t n_grids, n_reqs, total, lg;
 };
 
 __global__ __launch_bounds__(128) void k_simple_batch(BatchArgs a) {
-    const uint32_t slot = blockIdx.x * 128u + threadIdx.x;
-    if (slot >= a.total) return;  // whole waves: every request has a multiple of 64 slots
+    const uint32_t lane = threadIdx.x & 63u, slot = ((blockIdx.x * 2u + (threadIdx.x >> 6)) << a.lg) + lane;
+    if (lane >> a.lg || slot >= a.total) return;
     // so the 64 slots of a wave belong to one request: find it once per wave
     const uint32_t wslot = (uint32_t)__builtin_amdgcn_readfirstlane((int)(slot & ~63u));
     uint32_t lo = 0, hi = a.n_reqs;  // slot -> request: binary search over the prefix
@@ -781,20 +782,22 @@ int launch_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs
         if (one) {
             const bool sh = (q[0].flags & WX_TRACE_SHADOW) != 0u;
             if (q[0].kind == WX_REQ_CAMERA) {
-                dim3 grid((q[0].w + 15u) / 16u, (q[0].h + 7u) / 8u, 1);
+                const uint32_t lg = rays_per_wave_log2(total), lw = 1u + ((lg + 1u) >> 1), lh = lg >> 1;
+                dim3 grid((q[0].w + (1u << lw) - 1u) >> lw, (q[0].h + (1u << lh) - 1u) >> lh, 1);
                 const uint32_t band = t.xcd_split == 2u ? 1u : 0u;  // XCD-banded tile order
-                if (sh) hipLaunchKernelGGL(k_simple_camera<true>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], band);
-                else hipLaunchKernelGGL(k_simple_camera<false>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], band);
+                if (sh) hipLaunchKernelGGL(k_simple_camera<true>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], lg, band);
+                else hipLaunchKernelGGL(k_simple_camera<false>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], lg, band);
             } else {
-                dim3 grid((q[0].w + 127u) / 128u);
+                const uint32_t lg = rays_per_wave_log2(total), per_group = 2u << lg;
+                dim3 grid((q[0].w + per_group - 1u) / per_group);
                 // a list with at least two sets of 64 rays for every wave the GPU holds goes to two
                 // kernels, each of which takes the sets that suit it (k_persist1): at 1 Mi rays
                 // scattered ones took 286 us against 346 in one kernel, a panorama 243 against 234;
                 // at half that scattered ones 251 against 193
                 const uint32_t sets = (q[0].w + 63u) / 64u, most = (uint32_t)cu_count() * 32u;
                 const uint32_t split = may_split && !sh && sets >= 2u * most ? 1u : 0u;
-                if (sh) hipLaunchKernelGGL(k_simple_rays<true>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], 0u);
-                else hipLaunchKernelGGL(k_simple_rays<false>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], split);
+                if (sh) hipLaunchKernelGGL(k_simple_rays<true>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], lg, 0u);
+                else hipLaunchKernelGGL(k_simple_rays<false>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], lg, split);
                 if (split) {
                     const uint32_t per_wave = (sets + most - 1u) / most;
                     launch_persist1<WX_REQ_RAYS>((sets + 4u * per_wave - 1u) / (4u * per_wave), stream, grids[0]->dev, q[0],
@@ -810,7 +813,9 @@ int launch_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs
             b.n_grids = n_grids;
             b.n_reqs = n_reqs;
             b.total = (uint32_t)total;
-            hipLaunchKernelGGL(k_simple_batch, dim3((uint32_t)((total + 127u) / 128u)), dim3(128), 0, stream, b);
+            b.lg = rays_per_wave_log2(total);
+            hipLaunchKernelGGL(k_simple_batch, dim3((uint32_t)((total + (2u << b.lg) - 1u) >> (b.lg + 1u))), dim3(128), 0,
+                               stream, b);
         }
         e = hipGetLastError();
         if (e != hipSuccess) return hip_fail(e, "batch: launch");
