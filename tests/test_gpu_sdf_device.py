@@ -151,3 +151,25 @@ def test_empty_tree(wx, cuda):
     v = wx.Vdb345()
     assert v.compute_sdf(device=True) == 0
     assert v.count_nodes() == [0, 0, 0]
+
+
+@pytest.mark.parametrize("fill", [0.002, 0.1, 0.97])
+@pytest.mark.parametrize("span", [3, 40, 600])
+def test_random_leaves(wx, cuda, span, fill):
+    """Leaves of random voxels around the corner of eight root nodes: neighbours of every
+    kind on every side (missing, solid, partly known), packed close and far apart."""
+    say(f"device SDF: random leaves, span {span}, fill {fill}")
+    rng = np.random.default_rng(span + int(1000 * fill))
+    keys = np.unique(rng.integers(-span, span, (900, 3)), axis=0).astype(np.int32)
+    on = rng.random((len(keys), 512)) < fill
+    on[rng.random(len(keys)) < 0.1] = True
+    on[np.arange(len(keys)), rng.integers(0, 512, len(keys))] = True  # no empty mask
+    masks = np.packbits(on, axis=1, bitorder="little").view(np.uint64)
+
+    def make():
+        v = wx.Vdb345()
+        v.add_leaf_masks(keys, masks)
+        return v
+
+    host, dev, _ = build_pair(make)
+    same_layout(host, dev)

@@ -7,9 +7,9 @@
 // offsets (-1, dy, dz), (0, -1, dz), (0, 0, -1) (or their negatives backward); in
 // the neighbouring nodes, whatever those hold at that moment. Two facts make
 // this parallel without changing a value:
-//  * slot (x, y, z) only reads in-node slots of smaller t = 4x + 2y + z (larger
-//    t backward), so the slots of one t are independent -- a node is a sweep of
-//    7 (D - 1) + 1 wavefronts (D = 8, 16, 32);
+//  * a row (x, y) of slots along z only reads in-node rows of smaller t = 2x + y
+//    (larger t backward), and its own chain along z is a prefix minimum, so the rows
+//    of one t are independent -- a node is a sweep of 3 (D - 1) + 1 steps (D = 8, 16, 32);
 //  * the host's level schedule groups the nodes so that every neighbour a node
 //    must see updated sits in an earlier group and every neighbour it must see
 //    untouched in a later one -- one launch per group, one workgroup per node.
@@ -38,37 +38,66 @@ namespace {
 
 constexpr uint8_t kUnknown = 255;  // the start value (the reference's MAX - 1)
 
-// One node swept by one workgroup (one wave). The node and a one-slot halo around
-// it are staged in LDS first, coded as 0 where a read gives 1 (a solid slot, a slot
-// of a missing node) and as the current value elsewhere: the neighbours a node
-// reads hold still while it is swept (the schedule), so the sweep runs from LDS
-// alone.
+// One node swept by one workgroup. The node and a one-slot halo around it are staged in
+// LDS first, coded as 0 where a read gives 1 (a solid slot, a slot of a missing node) and as
+// the current value elsewhere: the neighbours a node reads hold still while it is swept (the
+// schedule), so the sweep runs from LDS alone. The backward pass stages the node mirrored
+// along every axis, which makes it a forward pass.
+//
+// The sweep goes row by row, not slot by slot: row (x, y) needs the rows (x - 1, y - 1 .. y + 1)
+// and (x, y - 1), so the rows of one 2x + y are independent -- 3 D - 2 steps instead of the
+// 7 D - 6 of slots in order of 4x + 2y + z. Within a row a new value is
+//   v[z] = min(b[z], v[z - 1] + 1),  b[z] = min(v[z], 1 + min of the 12 slots of other rows),
+// a prefix minimum of b[z] - z. Sixteen lanes take a row, D / 8 slots each: lane 0 the slot
+// z = -1 (the neighbour's, which starts the prefix), lanes 1..8 the row, lane 9 z = D; the
+// shifts along z are DPP row shifts. A read of 255 (unknown) gives 256, which is below no
+// value; a slot at 0 keeps it.
+// Bound by the chain of steps: LDS read, about 15 dependent instructions, LDS write, in about
+// 500 clocks; slot by slot a launch took 13.8 us for leaves, 61 us for node-4s, 411 us for a
+// node-5.
 //
 // Leaves (LOG 3) may also emit their packed layout words: 64 words of eight 4-bit
 // codes, one word per lane, with *bad set when a code does not fit 4 bits.
 template <int LOG>
-struct NodeLds {
-    static constexpr int D = 1 << LOG, P = D + 2;
-    static constexpr uint32_t PS = (uint32_t)P * P * P;
-    uint8_t pad[PS];
-    int32_t nb[27];
+struct SweepShape {
+    static constexpr int D = 1 << LOG, P = D + 2, E = D / 8;  // E slots per lane
+    static constexpr int kStride = D + 8;                      // bytes of a row in LDS: slot z at 4 + z
+    static constexpr int kThreads = 8 * D;                     // at most D / 2 rows have one 2x + y
 };
 
+// The shift by n lanes up (row_shr) within 16; lanes without a source keep x.
+template <int kCtrl>
+__device__ __forceinline__ int dpp(int x) {
+    return __builtin_amdgcn_update_dpp(x, x, kCtrl, 0xF, 0xF, false);
+}
+constexpr int kRowShl1 = 0x101, kRowShr1 = 0x111, kRowShr2 = 0x112, kRowShr4 = 0x114, kRowShr8 = 0x118;
+
+// 0xFF in byte k where bit k of b is set.
+__device__ __forceinline__ uint64_t byte_mask(uint32_t b) {
+    const uint64_t one = (uint64_t)(b * 0x01010101u) * 0x100000001ull & 0x8040201008040201ull;
+    const uint64_t top = (one + 0x7F7F7F7F7F7F7F7Full) & 0x8080808080808080ull;
+    return top | (top - (top >> 7));
+}
+
 template <int LOG>
-__device__ __forceinline__ void sweep_node(NodeLds<LOG> &L, uint32_t n, const uint64_t *solid, uint8_t *val,
-                                           const int32_t *nb, int forward, uint32_t *nib, uint32_t *bad) {
-    constexpr int D = 1 << LOG, P = D + 2;
-    constexpr uint32_t S = (uint32_t)D * D * D, W = S / 64, T = 7 * (D - 1) + 1, PS = (uint32_t)P * P * P;
-    uint8_t *pad = L.pad;
-    int32_t *s_nb = L.nb;
+__global__ __launch_bounds__(8 << LOG) void k_sdf_nodes(const uint64_t *solid, uint8_t *val, const int32_t *nb,
+                                                        const uint32_t *group, int forward, uint32_t *nib,
+                                                        uint32_t *bad) {
+    using Sh = SweepShape<LOG>;
+    constexpr int D = Sh::D, P = Sh::P, E = Sh::E, RS = Sh::kStride, H = D / 8;
+    constexpr uint32_t S = (uint32_t)D * D * D, kThreads = Sh::kThreads;
+    __shared__ __align__(8) uint8_t pad[P * P * RS];
+    __shared__ int32_t s_nb[27];
+    const uint32_t n = group[blockIdx.x];
+    const uint8_t *bits = reinterpret_cast<const uint8_t *>(solid);
     // the neighbour row is loaded alongside the leaf's solid words (independent loads)
     const int32_t nb_own = threadIdx.x < 27u ? nb[(size_t)n * 27 + threadIdx.x] : -1;  // entry 13 is n itself
     if constexpr (LOG == 3) {
         // a leaf without an inactive voxel has nothing to sweep: every slot is solid (0)
-        const uint64_t *m = solid + (size_t)n * W;
+        const uint64_t *m = solid + (size_t)n * 8u;
         uint64_t all = ~0ull;
 #pragma unroll
-        for (uint32_t k = 0; k < W; ++k) all &= m[k];
+        for (uint32_t k = 0; k < 8u; ++k) all &= m[k];
         if (all == ~0ull) {
             reinterpret_cast<uint64_t *>(val + (size_t)n * S)[threadIdx.x] = 0;
             if (nib) nib[(size_t)n * 64u + threadIdx.x] = 0;
@@ -77,110 +106,124 @@ __device__ __forceinline__ void sweep_node(NodeLds<LOG> &L, uint32_t n, const ui
     }
     if (threadIdx.x < 27u) s_nb[threadIdx.x] = nb_own;
     __syncthreads();
-    // kG slots per lane at a time: their solid words and values are independent loads,
-    // all in flight together (a slot's value is read even where the solid bit wins); a
-    // leaf's 1,000 padded slots take one round
-    constexpr uint32_t kG = 16;
-    for (uint32_t base = 0; base < PS; base += 64u * kG) {
-        int32_t m[kG];
-        uint32_t c[kG];
-        uint64_t sw[kG];
-        uint8_t v[kG];
+    // staged eight slots of a row at a time, with the row's halo slots by its first and last eight
+    constexpr uint32_t kItems = (uint32_t)(P * P * H), kRounds = (kItems + kThreads - 1u) / kThreads;
+    constexpr uint32_t kG = kRounds < 4u ? kRounds : 4u;  // rounds with their loads in flight together
+    for (uint32_t base = 0; base < kItems; base += kG * kThreads) {
+        uint64_t v[kG];
+        uint32_t b[kG], lo[kG], hi[kG];
 #pragma unroll
         for (uint32_t k = 0; k < kG; ++k) {
-            const uint32_t i = base + k * 64u + threadIdx.x;
-            m[k] = -1, c[k] = 0, sw[k] = 0, v[k] = 0;
-            if (i < PS) {
-                int cx = (int)(i / (P * P)) - 1, cy = (int)((i / P) % P) - 1, cz = (int)(i % P) - 1;
-                const int ox = cx < 0 ? -1 : (cx >= D ? 1 : 0);
-                const int oy = cy < 0 ? -1 : (cy >= D ? 1 : 0);
-                const int oz = cz < 0 ? -1 : (cz >= D ? 1 : 0);
-                cx &= D - 1, cy &= D - 1, cz &= D - 1;
-                m[k] = s_nb[(ox + 1) * 9 + (oy + 1) * 3 + (oz + 1)];
-                c[k] = ((uint32_t)cx << (2 * LOG)) | ((uint32_t)cy << LOG) | (uint32_t)cz;
-                if (m[k] >= 0) {
-                    sw[k] = solid[(size_t)m[k] * W + (c[k] >> 6)];
-                    v[k] = val[(size_t)m[k] * S + c[k]];
+            const uint32_t i = base + k * kThreads + threadIdx.x;
+            v[k] = 0, b[k] = 0xFFu, lo[k] = 0, hi[k] = 0;
+            if (i < kItems) {
+                const uint32_t row = i / H, h = i % H, X = row / P, Y = row % P;
+                const uint32_t ox = X == 0u ? 0u : (X == P - 1u ? 2u : 1u), oy = Y == 0u ? 0u : (Y == P - 1u ? 2u : 1u);
+                const int32_t *m = s_nb + ox * 9u + oy * 3u;
+                const uint32_t c = ((X - 1u) & (D - 1u)) << (2 * LOG) | ((Y - 1u) & (D - 1u)) << LOG;
+                if (m[1] >= 0) {
+                    const size_t at = (size_t)m[1] * S + c + h * 8u;
+                    v[k] = *reinterpret_cast<const uint64_t *>(val + at);
+                    b[k] = bits[at >> 3];
+                }
+                if (h == 0u && m[0] >= 0) {
+                    const size_t at = (size_t)m[0] * S + c + D - 1u;
+                    lo[k] = (bits[at >> 3] & 0x80u) ? 0u : val[at];
+                }
+                if (h == H - 1u && m[2] >= 0) {
+                    const size_t at = (size_t)m[2] * S + c;
+                    hi[k] = (bits[at >> 3] & 1u) ? 0u : val[at];
                 }
             }
         }
 #pragma unroll
         for (uint32_t k = 0; k < kG; ++k) {
-            const uint32_t i = base + k * 64u + threadIdx.x;
-            if (i < PS) pad[i] = (m[k] < 0 || ((sw[k] >> (c[k] & 63u)) & 1ull)) ? (uint8_t)0 : v[k];
+            const uint32_t i = base + k * kThreads + threadIdx.x;
+            if (i < kItems) {
+                const uint32_t row = i / H, h = i % H;
+                uint64_t w = v[k] & ~byte_mask(b[k]);
+                uint8_t *r = pad + (forward ? row : P * P - 1u - row) * RS + 4;
+                if (!forward) w = __builtin_bswap64(w);
+                uint32_t *d = reinterpret_cast<uint32_t *>(r + (forward ? h : H - 1u - h) * 8u);
+                d[0] = (uint32_t)w, d[1] = (uint32_t)(w >> 32);
+                if (h == 0u) r[forward ? -1 : D] = (uint8_t)lo[k];
+                if (h == H - 1u) r[forward ? D : -1] = (uint8_t)hi[k];
+            }
         }
     }
     __syncthreads();
-    // the 13 neighbours in padded offsets: (sgn, dy, dz), (0, sgn, dz), (0, 0, sgn), dy, dz in -1..1
-    const int sgn = forward ? -1 : 1;
-    int off[13];
+    const uint32_t g = threadIdx.x >> 4, j = threadIdx.x & 15u;
+    const int z0 = ((int)(j < 9u ? j : 9u) - 1) * E;  // the lane's first slot; lanes past 9 repeat its reads
+    auto load = [&](const uint8_t *p, int *o) {
+        uint32_t w;
+        if constexpr (E == 1) w = *p;
+        else if constexpr (E == 2) w = *reinterpret_cast<const uint16_t *>(p);
+        else w = *reinterpret_cast<const uint32_t *>(p);
 #pragma unroll
-    for (int k = 0; k < 9; ++k) off[k] = sgn * P * P + (k / 3 - 1) * P + (k % 3 - 1);
+        for (int e = 0; e < E; ++e) o[e] = (int)((w >> (8 * e)) & 255u);
+    };
+    for (int t = 0; t < 3 * D - 2; ++t) {
+        const int x_lo = t < D ? 0 : (t - D + 2) >> 1, x = x_lo + (int)g, y = t - 2 * x;
+        if (x < D && y >= 0) {
+            uint8_t *own = pad + ((x + 1) * P + y + 1) * RS + 4 + z0;
+            int v[E], m[E], q[E];
+            load(own - RS, m);  // (x, y - 1), then (x - 1, y - 1 .. y + 1)
 #pragma unroll
-    for (int k = 0; k < 3; ++k) off[9 + k] = sgn * P + (k - 1);
-    off[12] = sgn;
-    // Columns (x, y) of slots (x, y, 0..D-1): lane l owns columns c = l + 64 j (x = c >> LOG,
-    // y = c & (D - 1)), and on wavefront t updates slot z = t - 4x - 2y of each of them where
-    // that lies in 0..D-1 (the slots of one wavefront are independent). The 13 reads are
-    // independent too, and
-    //   min(v, min over k of (1 if w_k == 0, 255 if w_k == 255, else w_k + 1))
-    // is min(v, min_k w_k + 1) unless every w_k is 255 (then v): a solid read gives 1, and a
-    // slot already at 0 or 1 keeps its value.
-    constexpr uint32_t C = (uint32_t)D * D / 64u;
-    for (int tt = 0; tt < (int)T; ++tt) {
-        const int t = forward ? tt : (int)T - 1 - tt;
+            for (int k = -1; k <= 1; ++k) {
+                load(own + (k - P) * RS, q);
 #pragma unroll
-        for (uint32_t j = 0; j < C; ++j) {
-            const uint32_t col = threadIdx.x + 64u * j, x = col >> LOG, y = col & (D - 1u);
-            const int z = t - (int)(4u * x + 2u * y);
-            if (z >= 0 && z < D) {
-                const int p = (int)((x + 1u) * P * P + (y + 1u) * P + 1u) + z;
-                uint32_t mw = pad[p + off[0]];
+                for (int e = 0; e < E; ++e) m[e] = min(m[e], q[e]);
+            }
+            load(own, v);
+            const int before = dpp<kRowShr1>(m[E - 1]), after = dpp<kRowShl1>(m[0]);
+            int c[E];
 #pragma unroll
-                for (int k = 1; k < 13; ++k) {
-                    const uint32_t w = pad[p + off[k]];
-                    mw = w < mw ? w : mw;
-                }
-                const uint32_t v = pad[p];
-                if (mw < (uint32_t)kUnknown && mw + 1u < v) pad[p] = (uint8_t)(mw + 1u);
+            for (int e = 0; e < E; ++e) {
+                const int w = min(min(e ? m[e ? e - 1 : 0] : before, m[e]), e < E - 1 ? m[e < E - 1 ? e + 1 : e] : after);
+                c[e] = min(v[e], w + 1) - e;
+                if (j == 0u) c[e] = e == E - 1 ? v[e] - e : 1024;  // the slot before the row stays
+                if (e) c[e] = min(c[e], c[e ? e - 1 : 0]);
+            }
+            // inclusive prefix over the lanes, each lane's slots E further than the last's
+            int T = c[E - 1] - (int)j * E;
+            T = min(T, dpp<kRowShr1>(T));
+            T = min(T, dpp<kRowShr2>(T));
+            T = min(T, dpp<kRowShr4>(T));
+            T = min(T, dpp<kRowShr8>(T));
+            uint32_t w = 0;
+            if constexpr (E == 1) {
+                w = (uint32_t)(T + (int)j);
+            } else {
+                const int prev = dpp<kRowShr1>(T) + (int)j * E;
+#pragma unroll
+                for (int e = 0; e < E; ++e) w |= (uint32_t)(min(c[e], prev) + e) << (8 * e);
+            }
+            if (j - 1u < 8u) {
+                if constexpr (E == 1) *own = (uint8_t)w;
+                else if constexpr (E == 2) *reinterpret_cast<uint16_t *>(own) = (uint16_t)w;
+                else *reinterpret_cast<uint32_t *>(own) = w;
             }
         }
-        __syncthreads();
+        // a workgroup of one wave keeps its LDS accesses in order without waiting for them
+        if constexpr (kThreads == 64u) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        else __syncthreads();
     }
-    // column c is slots c D .. c D + D - 1, stored eight at a time (solid slots go back as 0; their
-    // value is never read, the solid bit answers first); a leaf lane's column is also its layout word
-#pragma unroll
-    for (uint32_t j = 0; j < C; ++j) {
-        const uint32_t col = threadIdx.x + 64u * j, x = col >> LOG, y = col & (D - 1u);
-        const int base = (int)((x + 1u) * P * P + (y + 1u) * P + 1u);
-        uint64_t *dst = reinterpret_cast<uint64_t *>(val + (size_t)n * S + (size_t)col * D);
-#pragma unroll
-        for (int h = 0; h < D / 8; ++h) {
-            uint64_t bytes = 0;
-            uint32_t word = 0, over = 0;
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const uint32_t v = pad[base + 8 * h + k];
-                bytes |= (uint64_t)v << (8 * k);
-                over |= v > 15u ? 1u : 0u;
-                word |= (v & 15u) << (4 * k);
-            }
-            dst[h] = bytes;
-            if (LOG == 3 && nib) {
-                nib[(size_t)n * 64u + threadIdx.x] = word;
-                if (over) atomicOr(bad, 1u);
-            }
+    // solid slots go back as 0; their value is never read, the solid bit answers first
+    for (uint32_t i = threadIdx.x; i < (uint32_t)(D * D * H); i += kThreads) {
+        const uint32_t col = i / H, h = i % H, row = ((col >> LOG) + 1u) * P + (col & (D - 1u)) + 1u;
+        const uint32_t *r = reinterpret_cast<const uint32_t *>(pad + (forward ? row : P * P - 1u - row) * RS + 4 +
+                                                               (forward ? h : H - 1u - h) * 8u);
+        uint64_t bytes = (uint64_t)r[1] << 32 | r[0];
+        if (!forward) bytes = __builtin_bswap64(bytes);
+        reinterpret_cast<uint64_t *>(val + (size_t)n * S)[i] = bytes;
+        if (LOG == 3 && nib) {
+            uint64_t w = bytes & 0x0F0F0F0F0F0F0F0Full;
+            if (w != bytes) atomicOr(bad, 1u);
+            w = (w | w >> 4) & 0x00FF00FF00FF00FFull;
+            w = (w | w >> 8) & 0x0000FFFF0000FFFFull;
+            nib[(size_t)n * 64u + i] = (uint32_t)(w | w >> 16);
         }
     }
-}
-
-// One workgroup per node of one schedule group (one launch per group).
-template <int LOG>
-__global__ __launch_bounds__(64) void k_sdf_nodes(const uint64_t *solid, uint8_t *val, const int32_t *nb,
-                                                  const uint32_t *group, int forward, uint32_t *nib,
-                                                  uint32_t *bad) {
-    __shared__ NodeLds<LOG> L;
-    sweep_node<LOG>(L, group[blockIdx.x], solid, val, nb, forward, nib, bad);
 }
 
 // ---- the leaves' neighbour table and level schedules, built on the device ----
@@ -698,7 +741,7 @@ bool run_level(wx::SdfLevelJob &J, Ctx &c, std::string &err) {
     std::unique_ptr<Scheduler> sch;  // outlives the sweeps, which read its groups
     const uint64_t *sp = nullptr;     // the solid masks the sweeps read: solid, or the tree's device copy
     auto sweep = [&](const uint32_t *group, uint32_t n, int fw) {
-        hipLaunchKernelGGL(k_sdf_nodes<LOG>, dim3(n), dim3(64), 0, c.stream, sp,
+        hipLaunchKernelGGL(k_sdf_nodes<LOG>, dim3(n), dim3(SweepShape<LOG>::kThreads), 0, c.stream, sp,
                            static_cast<uint8_t *>(val.p), static_cast<const int32_t *>(nb.p), group,
                            fw,
                            fw ? nullptr : static_cast<uint32_t *>(nib.p), static_cast<uint32_t *>(bad.p));
