@@ -55,6 +55,17 @@ def test_device_noise_matches_host(wx, cuda, lo, hi, f0, occ):
     same_layout(h, d)
 
 
+@pytest.mark.parametrize("lo,hi", [((0, 0, 0), (1, 1, 1)), ((-9, 3, 70), (60, 44, 99))])
+@pytest.mark.parametrize("occ", [1e-6, 0.37, 0.5, 0.999999])
+def test_device_threshold_matches_host(wx, cuda, lo, hi, occ):
+    """The sample picked as the threshold, at both ends of the samples and among equal ones."""
+    say(f"device noise threshold {lo} {hi} occupancy {occ}")
+    for seed in (0, 1, 2 ** 63 + 5):
+        th = wx.Vdb345().add_noise(seed, lo, hi, 0.11, occ, threads=2)
+        td = wx.Vdb345().add_noise(seed, lo, hi, 0.11, occ, device=True)
+        assert np.float32(th).view(np.uint32) == np.float32(td).view(np.uint32)
+
+
 def test_device_noise_merges_into_existing_leaves(wx, cuda):
     say("device noise over a sphere set")
     sp = scenes.sphere_set(3, count=60, domain=256, rmin=4, rmax=30)

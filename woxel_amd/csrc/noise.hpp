@@ -117,6 +117,25 @@ struct Params {
     int32_t lo[3], hi[3];
 };
 
+// The threshold is a quantile of the noise at kSamples seeded points of [lo, hi): a 64-bit
+// xorshift sequence, three numbers a point.
+constexpr uint32_t kSamples = 65536;
+
+WX_NOISE_FN uint64_t sample_next(uint64_t &st) {
+    st ^= st << 13;
+    st ^= st >> 7;
+    st ^= st << 17;
+    return st;
+}
+
+WX_NOISE_FN float sample(const Params &p, uint64_t &st) {
+    int32_t q[3];
+    for (int a = 0; a < 3; ++a) q[a] = p.lo[a] + (int32_t)(sample_next(st) % (uint64_t)(p.hi[a] - p.lo[a]));
+    return noise3(p.seed, p.f0, (float)q[0], (float)q[1], (float)q[2]);
+}
+
+WX_NOISE_FN uint64_t sample_start(uint64_t seed) { return seed * 0x9E3779B97F4A7C15ull + 1; }
+
 // Leaf class from its centre value: 0 = no active voxel, 1 = every voxel active,
 // 2 = decided voxel by voxel. b = the leaf's first voxel.
 WX_NOISE_FN int leaf_class(const Params &p, const int32_t b[3], bool &inside_box) {

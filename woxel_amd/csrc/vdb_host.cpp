@@ -473,7 +473,7 @@ bool HostVdb::add_spheres(const double *sp, size_t n, const int32_t lo[3], const
 }
 
 bool HostVdb::noise_params(uint64_t seed, const int32_t lo[3], const int32_t hi[3], float base_freq,
-                           float occupancy, wxnoise::Params &p, std::string &err) const {
+                           float occupancy, wxnoise::Params &p, size_t &rank, std::string &err) const {
     if (finalized_) { err = "add_noise: grid already finalized"; return false; }
     for (int i = 0; i < 3; ++i)
         if (lo[i] < -kCoordLimit || hi[i] > kCoordLimit || lo[i] >= hi[i]) {
@@ -488,21 +488,7 @@ bool HostVdb::noise_params(uint64_t seed, const int32_t lo[3], const int32_t hi[
     p.f0 = base_freq;
     for (int a = 0; a < 3; ++a) p.lo[a] = lo[a], p.hi[a] = hi[a];
     // threshold = the (1 - occupancy) quantile of seeded samples
-    std::vector<float> smp(65536);
-    uint64_t st = seed * 0x9E3779B97F4A7C15ull + 1;
-    auto next = [&] {
-        st ^= st << 13;
-        st ^= st >> 7;
-        st ^= st << 17;
-        return st;
-    };
-    for (float &v : smp) {
-        int32_t q[3];
-        for (int a = 0; a < 3; ++a) q[a] = lo[a] + (int32_t)(next() % (uint64_t)(hi[a] - lo[a]));
-        v = wxnoise::noise3(p.seed, base_freq, (float)q[0], (float)q[1], (float)q[2]);
-    }
-    std::sort(smp.begin(), smp.end());
-    p.thr = smp[(size_t)((1.0f - occupancy) * (float)(smp.size() - 1))];
+    rank = (size_t)((1.0f - occupancy) * (float)(wxnoise::kSamples - 1u));
     p.bound = wxnoise::leaf_bound(base_freq);
     return true;
 }
@@ -510,7 +496,13 @@ bool HostVdb::noise_params(uint64_t seed, const int32_t lo[3], const int32_t hi[
 bool HostVdb::add_noise(uint64_t seed, const int32_t lo[3], const int32_t hi[3], float base_freq, float occupancy,
                         int threads, float *threshold, std::string &err) {
     wxnoise::Params prm;
-    if (!noise_params(seed, lo, hi, base_freq, occupancy, prm, err)) return false;
+    size_t rank = 0;
+    if (!noise_params(seed, lo, hi, base_freq, occupancy, prm, rank, err)) return false;
+    std::vector<float> smp(wxnoise::kSamples);
+    uint64_t st = wxnoise::sample_start(seed);
+    for (float &v : smp) v = wxnoise::sample(prm, st);
+    std::nth_element(smp.begin(), smp.begin() + (ptrdiff_t)rank, smp.end());
+    prm.thr = smp[rank];
     if (threshold) *threshold = prm.thr;
     const int32_t l0[3] = {lo[0] >> 3, lo[1] >> 3, lo[2] >> 3};
     const int32_t l1[3] = {(hi[0] - 1) >> 3, (hi[1] - 1) >> 3, (hi[2] - 1) >> 3};

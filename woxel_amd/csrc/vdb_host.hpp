@@ -115,10 +115,10 @@ class HostVdb {
     // is active (quantile of 65536 seeded samples); *threshold receives t.
     bool add_noise(uint64_t seed, const int32_t lo[3], const int32_t hi[3], float base_freq, float occupancy,
                    int threads, float *threshold, std::string &err);
-    // The checked parameters and threshold of that isosurface (for a generator
-    // elsewhere, the device one: same voxels).
+    // The checked parameters of that isosurface, without its threshold, and the rank of the
+    // sample that is the threshold (for a generator elsewhere, the device one: same voxels).
     bool noise_params(uint64_t seed, const int32_t lo[3], const int32_t hi[3], float base_freq, float occupancy,
-                      wxnoise::Params &p, std::string &err) const;
+                      wxnoise::Params &p, size_t &rank, std::string &err) const;
     // Append leaves the caller guarantees are new: keys unique and absent from the
     // tree, masks non-zero. No hashing; the key index is rebuilt on the next lookup.
     bool append_new_leaves(const int32_t *keys, const uint64_t *masks, size_t n, std::string &err);
