@@ -65,10 +65,11 @@ struct SweepShape {
     static constexpr int kThreads = 8 * D;                     // at most D / 2 rows have one 2x + y
 };
 
-// The shift by n lanes up (row_shr) within 16; lanes without a source keep x.
+// x of the lane n below (row_shr) or above (row_shl) within 16, 0 where there is none: the
+// form that is part of the instruction that uses it.
 template <int kCtrl>
-__device__ __forceinline__ int dpp(int x) {
-    return __builtin_amdgcn_update_dpp(x, x, kCtrl, 0xF, 0xF, false);
+__device__ __forceinline__ uint32_t dpp(uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kCtrl, 0xF, 0xF, true);
 }
 constexpr int kRowShl1 = 0x101, kRowShr1 = 0x111, kRowShr2 = 0x112, kRowShr4 = 0x114, kRowShr8 = 0x118;
 
@@ -86,7 +87,7 @@ __global__ __launch_bounds__(8 << LOG) void k_sdf_nodes(const uint64_t *solid, u
     using Sh = SweepShape<LOG>;
     constexpr int D = Sh::D, P = Sh::P, E = Sh::E, RS = Sh::kStride, H = D / 8;
     constexpr uint32_t S = (uint32_t)D * D * D, kThreads = Sh::kThreads;
-    __shared__ __align__(8) uint8_t pad[P * P * RS];
+    __shared__ __align__(8) uint8_t pad[P * P * RS + 4];
     __shared__ int32_t s_nb[27];
     const uint32_t n = group[blockIdx.x];
     const uint8_t *bits = reinterpret_cast<const uint8_t *>(solid);
@@ -154,56 +155,60 @@ __global__ __launch_bounds__(8 << LOG) void k_sdf_nodes(const uint64_t *solid, u
     __syncthreads();
     const uint32_t g = threadIdx.x >> 4, j = threadIdx.x & 15u;
     const int z0 = ((int)(j < 9u ? j : 9u) - 1) * E;  // the lane's first slot; lanes past 9 repeat its reads
-    auto load = [&](const uint8_t *p, int *o) {
+    auto load = [&](const uint8_t *p, uint32_t *o) {
         uint32_t w;
         if constexpr (E == 1) w = *p;
         else if constexpr (E == 2) w = *reinterpret_cast<const uint16_t *>(p);
         else w = *reinterpret_cast<const uint32_t *>(p);
 #pragma unroll
-        for (int e = 0; e < E; ++e) o[e] = (int)((w >> (8 * e)) & 255u);
+        for (int e = 0; e < E; ++e) o[e] = (w >> (8 * e)) & 255u;
     };
-    for (int t = 0; t < 3 * D - 2; ++t) {
-        const int x_lo = t < D ? 0 : (t - D + 2) >> 1, x = x_lo + (int)g, y = t - 2 * x;
-        if (x < D && y >= 0) {
-            uint8_t *own = pad + ((x + 1) * P + y + 1) * RS + 4 + z0;
-            int v[E], m[E], q[E];
-            load(own - RS, m);  // (x, y - 1), then (x - 1, y - 1 .. y + 1)
+    // a group takes the rows x = g and x = g + D / 2 one after the other, from step 2 g on; at
+    // other steps, and on lanes without a slot of the row, it writes to a spare place
+    int i = -2 * (int)g;
+    const uint8_t *at = pad + g * P * RS + 4 + z0;  // row (x - 1, y - 1)
+    uint8_t *spare = pad + P * P * RS;
+    for (int t = 0; t < 3 * D - 2; ++t, ++i) {
+        const bool on = (uint32_t)i < 2u * D;
+        uint8_t *own = pad + (at - pad) + (P + 1) * RS;
+        uint32_t v[E], m[E], q[E];
+        load(at + P * RS, m);  // (x, y - 1), then (x - 1, y - 1 .. y + 1)
 #pragma unroll
-            for (int k = -1; k <= 1; ++k) {
-                load(own + (k - P) * RS, q);
+        for (int k = 0; k < 3; ++k) {
+            load(at + k * RS, q);
 #pragma unroll
-                for (int e = 0; e < E; ++e) m[e] = min(m[e], q[e]);
-            }
-            load(own, v);
-            const int before = dpp<kRowShr1>(m[E - 1]), after = dpp<kRowShl1>(m[0]);
-            int c[E];
-#pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const int w = min(min(e ? m[e ? e - 1 : 0] : before, m[e]), e < E - 1 ? m[e < E - 1 ? e + 1 : e] : after);
-                c[e] = min(v[e], w + 1) - e;
-                if (j == 0u) c[e] = e == E - 1 ? v[e] - e : 1024;  // the slot before the row stays
-                if (e) c[e] = min(c[e], c[e ? e - 1 : 0]);
-            }
-            // inclusive prefix over the lanes, each lane's slots E further than the last's
-            int T = c[E - 1] - (int)j * E;
-            T = min(T, dpp<kRowShr1>(T));
-            T = min(T, dpp<kRowShr2>(T));
-            T = min(T, dpp<kRowShr4>(T));
-            T = min(T, dpp<kRowShr8>(T));
-            uint32_t w = 0;
-            if constexpr (E == 1) {
-                w = (uint32_t)(T + (int)j);
-            } else {
-                const int prev = dpp<kRowShr1>(T) + (int)j * E;
-#pragma unroll
-                for (int e = 0; e < E; ++e) w |= (uint32_t)(min(c[e], prev) + e) << (8 * e);
-            }
-            if (j - 1u < 8u) {
-                if constexpr (E == 1) *own = (uint8_t)w;
-                else if constexpr (E == 2) *reinterpret_cast<uint16_t *>(own) = (uint16_t)w;
-                else *reinterpret_cast<uint32_t *>(own) = w;
-            }
+            for (int e = 0; e < E; ++e) m[e] = min(m[e], q[e]);
         }
+        load(own, v);
+        uint8_t *dst = on && j - 1u < 8u ? own : spare;
+        if (on) at += i == D - 1 ? (D / 2 * P - (D - 1)) * RS : RS;
+        const uint32_t before = dpp<kRowShr1>(m[E - 1]), after = dpp<kRowShl1>(m[0]);
+        // the prefix minimum as a maximum of 1024 + slot - value, which 0 never is
+        uint32_t c[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const uint32_t w = min(min(m[e], e ? m[e ? e - 1 : 0] : before), e < E - 1 ? m[e < E - 1 ? e + 1 : e] : after);
+            uint32_t b = min(v[e], w + 1u);
+            if (j == 0u) b = e == E - 1 ? v[e] : 512u;  // the slot before the row stays
+            c[e] = 1024u + (uint32_t)e + j * E - b;
+            if (e) c[e] = max(c[e], c[e ? e - 1 : 0]);
+        }
+        uint32_t T = c[E - 1];
+        T = max(T, dpp<kRowShr1>(T));
+        T = max(T, dpp<kRowShr2>(T));
+        T = max(T, dpp<kRowShr4>(T));
+        T = max(T, dpp<kRowShr8>(T));
+        uint32_t w = 0;
+        if constexpr (E == 1) {
+            w = 1024u + j - T;
+        } else {
+            const uint32_t prev = dpp<kRowShr1>(T);
+#pragma unroll
+            for (int e = 0; e < E; ++e) w |= (1024u + (uint32_t)e + j * E - max(c[e], prev)) << (8 * e);
+        }
+        if constexpr (E == 1) *dst = (uint8_t)w;
+        else if constexpr (E == 2) *reinterpret_cast<uint16_t *>(dst) = (uint16_t)w;
+        else *reinterpret_cast<uint32_t *>(dst) = w;
         // a workgroup of one wave keeps its LDS accesses in order without waiting for them
         if constexpr (kThreads == 64u) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         else __syncthreads();
