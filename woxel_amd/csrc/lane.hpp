@@ -14,6 +14,7 @@
 #include <cstdint>
 
 #include "../../include/woxel_hip.h"
+#include "device_arena.hpp"
 
 namespace wxk {
 
@@ -489,6 +490,7 @@ __device__ __forceinline__ void camera_ray(const float *u, const float *mv, cons
 // of the records, and the addresses the kernels take.
 struct wx_grid {
     wxk::GridDev dev;
+    wx::DeviceArena arena;  // holds every pool below
     void *mem[4] = {nullptr, nullptr, nullptr, nullptr};
     void *entries[3] = {nullptr, nullptr, nullptr};  // node-5, node-4, bases
     uint64_t bytes = 0;

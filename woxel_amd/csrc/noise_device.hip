@@ -13,6 +13,7 @@
 #include <vector>
 
 #define WX_NOISE_FN __host__ __device__ inline
+#include "device_arena.hpp"
 #include "noise.hpp"
 #include "pinned_copy.hpp"
 #include "wave.hpp"
@@ -198,18 +199,16 @@ __global__ __launch_bounds__(1024) void k_noise_threshold(const uint32_t *sample
     if (threadIdx.x == 0u) *out = __uint_as_float((best >> 31) ? best & 0x7FFFFFFFu : ~best);
 }
 
-// The threshold of p (the sample of this rank) on the device.
-int device_threshold(uint64_t seed, wxnoise::Params &p, size_t rank, hipStream_t st) {
-    constexpr uint32_t kStates = wxnoise::kSamples / kPerState;
+// The threshold of p (the sample of this rank) on the device, in `mem` of kThresholdBytes.
+constexpr uint32_t kStates = wxnoise::kSamples / kPerState;
+constexpr size_t kThresholdBytes = kStates * 8u + wxnoise::kSamples * 4u + 4u;
+int device_threshold(uint64_t seed, wxnoise::Params &p, size_t rank, void *mem, hipStream_t st) {
     std::vector<uint64_t> states(kStates);
     uint64_t s = wxnoise::sample_start(seed);
     for (uint64_t &v : states) {
         v = s;
         for (uint32_t k = 0; k < 3u * kPerState; ++k) wxnoise::sample_next(s);
     }
-    void *mem = nullptr;
-    if (hipMalloc(&mem, kStates * 8u + wxnoise::kSamples * 4u + 4u) != hipSuccess)
-        return set_error(WX_ERR_BUDGET, "wx_vdb_add_noise_device: hipMalloc of the samples failed");
     uint64_t *ds = static_cast<uint64_t *>(mem);
     uint32_t *dv = reinterpret_cast<uint32_t *>(ds + kStates);
     float *dt = reinterpret_cast<float *>(dv + wxnoise::kSamples);
@@ -221,7 +220,6 @@ int device_threshold(uint64_t seed, wxnoise::Params &p, size_t rank, hipStream_t
     }
     if (e == hipSuccess) e = hipMemcpyAsync(&p.thr, dt, 4, hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
-    (void)hipFree(mem);
     return e == hipSuccess ? WX_OK : set_error(WX_ERR_DEVICE, "wx_vdb_add_noise_device: threshold failed");
 }
 
@@ -279,7 +277,6 @@ extern "C" int wx_vdb_add_noise_device(wx_vdb *v, uint64_t seed, const int32_t l
         size_t rank = 0;
         if (!v->tree.noise_params(seed, lo, hi, base_freq, occupancy, p, rank, err))
             return set_error(v->tree.finalized() ? WX_ERR_STATE : WX_ERR_INVALID, "wx_vdb_add_noise_device: " + err);
-        if (int rc = device_threshold(seed, p, rank, static_cast<hipStream_t>(stream))) return rc;
         LeafBox bx;
         uint64_t n[3];
         for (int a = 0; a < 3; ++a) {
@@ -302,19 +299,24 @@ extern "C" int wx_vdb_add_noise_device(wx_vdb *v, uint64_t seed, const int32_t l
         // otherwise they merge like add_leaf_masks
         const bool fresh = v->tree.leaf_count() == 0;
         hipStream_t st = static_cast<hipStream_t>(stream);
-        DevBuf counter, keys, masks, todo, skeys, smasks, dk, dk2, idx, idx2, tmp;
+        wx::DeviceArena mem;
         size_t tmp_bytes = 0;
         if (hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, (const uint64_t *)nullptr, (uint64_t *)nullptr,
                                                (const uint32_t *)nullptr, (uint32_t *)nullptr, (uint64_t)slab, 0, 64,
                                                st) != hipSuccess)
             return set_error(WX_ERR_DEVICE, "wx_vdb_add_noise_device: sort set-up failed");
-        if (hipMalloc(&counter.p, 8) != hipSuccess || hipMalloc(&keys.p, slab * 12) != hipSuccess ||
-            hipMalloc(&todo.p, slab * 4) != hipSuccess ||
-            hipMalloc(&masks.p, slab * 64) != hipSuccess || hipMalloc(&skeys.p, slab * 12) != hipSuccess ||
-            hipMalloc(&smasks.p, slab * 64) != hipSuccess || hipMalloc(&dk.p, slab * 8) != hipSuccess ||
-            hipMalloc(&dk2.p, slab * 8) != hipSuccess || hipMalloc(&idx.p, slab * 4) != hipSuccess ||
-            hipMalloc(&idx2.p, slab * 4) != hipSuccess || hipMalloc(&tmp.p, tmp_bytes ? tmp_bytes : 16) != hipSuccess)
+        auto piece = [](size_t n) { return wx::DeviceArena::piece(n); };
+        if (mem.allocate(piece(8) + piece(kThresholdBytes) + piece(slab * 64) + piece(slab * 12) + 3 * piece(slab * 4) +
+                         2 * piece(slab * 8) + piece(tmp_bytes)) != hipSuccess)
             return set_error(WX_ERR_BUDGET, "wx_vdb_add_noise_device: hipMalloc of the slab buffers failed");
+        uint32_t *const dcnt = mem.take<uint32_t>(8);
+        if (int rc = device_threshold(seed, p, rank, mem.take<void>(kThresholdBytes), st)) return rc;
+        uint8_t *const masks = mem.take<uint8_t>(slab * 64);
+        int32_t *const keys = mem.take<int32_t>(slab * 12);
+        uint32_t *const todo = mem.take<uint32_t>(slab * 4), *const idx = mem.take<uint32_t>(slab * 4),
+                        *const idx2 = mem.take<uint32_t>(slab * 4);
+        uint64_t *const dk = mem.take<uint64_t>(slab * 8), *const dk2 = mem.take<uint64_t>(slab * 8);
+        void *const tmp = mem.take<void>(tmp_bytes);
         // each slab's sorted leaves stay on the device until the last slab: the tree then
         // grows once, by the exact count (no regrowth, no zero fill), and they come down
         // through pinned staging
@@ -335,14 +337,11 @@ extern "C" int wx_vdb_add_noise_device(wx_vdb *v, uint64_t seed, const int32_t l
             p0 = p1;
             // counters[0]: output slots, counters[1]: candidates to decide voxel by voxel
             uint32_t cnt[2] = {0, 0};
-            uint32_t *dcnt = static_cast<uint32_t *>(counter.p);
             if (hipMemcpyAsync(dcnt, cnt, 8, hipMemcpyHostToDevice, st) != hipSuccess)
                 return set_error(WX_ERR_DEVICE, "wx_vdb_add_noise_device: counter reset failed");
             const uint64_t lanes = (count + kPerLane - 1u) / kPerLane;
             hipLaunchKernelGGL(k_noise_classify, dim3((uint32_t)((lanes + 255u) / 256u)), dim3(256), 0, st, p, bx, first,
-                               count, dcnt,
-                               static_cast<int32_t *>(keys.p), static_cast<uint8_t *>(masks.p),
-                               static_cast<uint32_t *>(todo.p), dcnt + 1);
+                               count, dcnt, keys, masks, todo, dcnt + 1);
             if (hipGetLastError() != hipSuccess ||
                 hipMemcpyAsync(cnt, dcnt, 8, hipMemcpyDeviceToHost, st) != hipSuccess ||
                 hipStreamSynchronize(st) != hipSuccess)
@@ -353,8 +352,7 @@ extern "C" int wx_vdb_add_noise_device(wx_vdb *v, uint64_t seed, const int32_t l
             if (cnt[1]) {
                 const uint32_t waves = (cnt[1] + kPerLane - 1u) / kPerLane;
                 hipLaunchKernelGGL(k_noise_voxels, dim3((waves + 3u) / 4u), dim3(256), 0, st, p, bx, first,
-                                   static_cast<const uint32_t *>(todo.p), cnt[1], dcnt,
-                                   static_cast<int32_t *>(keys.p), static_cast<uint8_t *>(masks.p));
+                                   todo, cnt[1], dcnt, keys, masks);
                 if (hipGetLastError() != hipSuccess ||
                     hipMemcpyAsync(&found, dcnt, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
                     hipStreamSynchronize(st) != hipSuccess)
@@ -369,17 +367,15 @@ extern "C" int wx_vdb_add_noise_device(wx_vdb *v, uint64_t seed, const int32_t l
                 return set_error(WX_ERR_BUDGET, "wx_vdb_add_noise_device: hipMalloc of the slab's leaves failed");
             // the slab's leaves into DFS order (they were appended in no particular order)
             hipLaunchKernelGGL(k_dfs_keys, dim3((found + 255u) / 256u), dim3(256), 0, st,
-                               static_cast<const int32_t *>(keys.p), found, static_cast<uint64_t *>(dk.p),
-                               static_cast<uint32_t *>(idx.p));
+                               keys, found, dk, idx);
             size_t tb = tmp_bytes;
             if (hipGetLastError() != hipSuccess ||
-                hipcub::DeviceRadixSort::SortPairs(tmp.p, tb, static_cast<const uint64_t *>(dk.p),
-                                                   static_cast<uint64_t *>(dk2.p), static_cast<const uint32_t *>(idx.p),
-                                                   static_cast<uint32_t *>(idx2.p), (uint64_t)found, 0, 64, st) != hipSuccess)
+                hipcub::DeviceRadixSort::SortPairs(tmp, tb, static_cast<const uint64_t *>(dk), dk2,
+                                                   static_cast<const uint32_t *>(idx), idx2, (uint64_t)found, 0, 64,
+                                                   st) != hipSuccess)
                 return set_error(WX_ERR_DEVICE, "wx_vdb_add_noise_device: sort failed");
             hipLaunchKernelGGL(k_gather_leaves, dim3((found + 3u) / 4u), dim3(256), 0, st,
-                               static_cast<const uint32_t *>(idx2.p), found, static_cast<const int32_t *>(keys.p),
-                               static_cast<const uint8_t *>(masks.p), static_cast<int32_t *>(o->keys.p),
+                               idx2, found, keys, masks, static_cast<int32_t *>(o->keys.p),
                                static_cast<uint8_t *>(o->masks.p));
             if (hipGetLastError() != hipSuccess) return set_error(WX_ERR_DEVICE, "wx_vdb_add_noise_device: gather failed");
             total_found += found;
@@ -388,7 +384,9 @@ extern "C" int wx_vdb_add_noise_device(wx_vdb *v, uint64_t seed, const int32_t l
         if (hipStreamSynchronize(st) != hipSuccess)
             return set_error(WX_ERR_DEVICE, "wx_vdb_add_noise_device: kernel failed");
         if (total_found) {
-            wx::PinnedCopier dl(st);
+            size_t largest = 0;
+            for (const auto &o : outs) largest = std::max(largest, (size_t)o->n * 64);
+            wx::PinnedCopier dl(st, largest);
             if (!dl.ok()) return set_error(WX_ERR_DEVICE, "wx_vdb_add_noise_device: pinned staging allocation failed");
             if (fresh) {
                 const size_t base = v->tree.leaf_count();
@@ -409,8 +407,10 @@ extern "C" int wx_vdb_add_noise_device(wx_vdb *v, uint64_t seed, const int32_t l
                 // order, for the device SDF replay (skipped, not an error, without room)
                 if (base == 0) {
                     void *all = nullptr;
-                    bool kept = hipMalloc(&all, total_found * 64) == hipSuccess;
-                    for (size_t k = 0, off = 0; kept && k < outs.size(); off += outs[k]->n, ++k)
+                    const bool whole = outs.size() == 1;  // one slab's masks are all
+                    if (whole) std::swap(all, outs[0]->masks.p);
+                    bool kept = whole || hipMalloc(&all, total_found * 64) == hipSuccess;
+                    for (size_t k = 0, off = 0; kept && !whole && k < outs.size(); off += outs[k]->n, ++k)
                         kept = hipMemcpyAsync(static_cast<char *>(all) + off * 64, outs[k]->masks.p,
                                               (size_t)outs[k]->n * 64, hipMemcpyDeviceToDevice, st) == hipSuccess;
                     kept = hipStreamSynchronize(st) == hipSuccess && kept;

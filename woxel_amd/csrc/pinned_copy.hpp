@@ -20,8 +20,9 @@ class PinnedCopier {
     // Copies below this size take a plain hipMemcpy (the pinned buffers are not worth it).
     static constexpr size_t kMin = 32ull << 20;
 
-    // Copies are ordered on `stream` (0: a stream of the copier's own).
-    explicit PinnedCopier(hipStream_t stream = nullptr) {
+    // Copies are ordered on `stream` (0: a stream of the copier's own). `largest`: bytes of the
+    // largest copy it will make, below which no second buffer and no larger one is pinned.
+    explicit PinnedCopier(hipStream_t stream = nullptr, size_t largest = ~size_t(0)) {
         const unsigned hc = std::thread::hardware_concurrency();
         threads_ = (int)std::min(16u, std::max(1u, hc));
         if (!stream) {
@@ -30,8 +31,9 @@ class PinnedCopier {
         } else {
             st_ = stream;
         }
-        for (int i = 0; i < 2 && ok_; ++i)
-            ok_ = hipHostMalloc(reinterpret_cast<void **>(&buf_[i]), kPiece, hipHostMallocDefault) == hipSuccess &&
+        const size_t piece = std::min(kPiece, std::max<size_t>(largest, 1u));
+        for (int i = 0; i < (largest > kPiece ? 2 : 1) && ok_; ++i)
+            ok_ = hipHostMalloc(reinterpret_cast<void **>(&buf_[i]), piece, hipHostMallocDefault) == hipSuccess &&
                   hipEventCreateWithFlags(&ev_[i], hipEventDisableTiming) == hipSuccess;
     }
     ~PinnedCopier() {

@@ -28,6 +28,7 @@
 #include <thread>
 #include <vector>
 
+#include "device_arena.hpp"
 #include "pinned_copy.hpp"
 #include "wave.hpp"
 #include "wx_internal.hpp"
@@ -462,44 +463,73 @@ struct LevelTrace {
 };
 
 template <typename T>
-bool upload(DevBuf &b, const T *src, size_t n, hipStream_t st, std::string &err) {
-    const size_t bytes = (n ? n : 1) * sizeof(T);
-    if (hipMalloc(&b.p, bytes) != hipSuccess) {
-        b.p = nullptr;
-        err = "device SDF: hipMalloc of " + std::to_string(bytes) + " bytes failed";
-        return false;
-    }
-    if (n && hipMemcpyAsync(b.p, src, n * sizeof(T), hipMemcpyHostToDevice, st) != hipSuccess) {
+bool upload(T *dst, const T *src, size_t n, hipStream_t st, std::string &err) {
+    if (n && hipMemcpyAsync(dst, src, n * sizeof(T), hipMemcpyHostToDevice, st) != hipSuccess) {
         err = "device SDF: upload failed";
         return false;
     }
     return true;
 }
 
-// The leaves' neighbour table on the device (from J.keys, DFS order) into nb.
-bool build_neighbours(wx::SdfLevelJob &J, Ctx &c, DevBuf &nb, std::string &err) {
-    const uint32_t n = J.nodes;
+// Slots of the hash table of n keys.
+uint64_t key_slots(uint32_t n) {
     uint64_t cap = 64;
     while (cap < 2ull * n) cap <<= 1;
-    DevBuf keys, kt, vt;
-    if (!J.keys || !upload(keys, J.keys, (size_t)n * 3, c.stream, err)) {
-        if (!J.keys) err = "device SDF: no neighbour table and no node keys";
-        return false;
+    return cap;
+}
+
+// Device buffers of one level's replay, from one allocation.
+struct LevelMem {
+    wx::DeviceArena arena;
+    uint64_t *solid = nullptr;                       // masks to upload (not the ones already on the device)
+    uint8_t *val = nullptr;
+    int32_t *nb = nullptr;
+    uint32_t *order[2] = {nullptr, nullptr};         // node-5s, node-4s: the schedules; leaves: the device schedule's
+    uint32_t *indeg[2] = {nullptr, nullptr};         // leaves
+    int32_t *keys = nullptr, *vt = nullptr;          // leaves: their keys and the hash table
+    uint64_t *kt = nullptr;
+    uint32_t *bad = nullptr;
+
+    bool allocate(const wx::SdfLevelJob &J, size_t S, bool own_masks, std::string &err) {
+        const bool host = !J.nb.empty();
+        const size_t n = J.nodes, cap = host ? 0 : key_slots(J.nodes);
+        const size_t sz[] = {own_masks ? n * S / 8 : 0, n * S, n * 27 * 4, n * 4, n * 4, host ? 0 : n * 4, host ? 0 : n * 4,
+                             host ? 0 : n * 12, cap * 8, cap * 4, 4};
+        size_t all = 0;
+        for (size_t b : sz) all += wx::DeviceArena::piece(b);
+        if (arena.allocate(all) != hipSuccess) {
+            err = "device SDF: hipMalloc of " + std::to_string(all) + " bytes failed";
+            return false;
+        }
+        size_t k = 0;
+        solid = arena.take<uint64_t>(sz[k++]);
+        val = arena.take<uint8_t>(sz[k++]);
+        nb = arena.take<int32_t>(sz[k++]);
+        for (uint32_t *&p : order) p = arena.take<uint32_t>(sz[k++]);
+        for (uint32_t *&p : indeg) p = arena.take<uint32_t>(sz[k++]);
+        keys = arena.take<int32_t>(sz[k++]);
+        kt = arena.take<uint64_t>(sz[k++]);
+        vt = arena.take<int32_t>(sz[k++]);
+        bad = arena.take<uint32_t>(sz[k++]);
+        return true;
     }
-    if (hipMalloc(&kt.p, cap * 8) != hipSuccess || hipMalloc(&vt.p, cap * 4) != hipSuccess ||
-        hipMalloc(&nb.p, (size_t)n * 27 * 4) != hipSuccess) {
-        err = "device SDF: hipMalloc of the neighbour tables failed";
+};
+
+// The leaves' neighbour table on the device (from J.keys, DFS order) into m.nb.
+bool build_neighbours(wx::SdfLevelJob &J, Ctx &c, LevelMem &m, std::string &err) {
+    const uint32_t n = J.nodes;
+    const uint64_t cap = key_slots(n);
+    if (!J.keys || !upload(m.keys, J.keys, (size_t)n * 3, c.stream, err)) {
+        if (!J.keys) err = "device SDF: no neighbour table and no node keys";
         return false;
     }
     const uint32_t blocks = (n + 255u) / 256u;
     const uint64_t nb_blocks = ((uint64_t)n * 27u + 255u) / 256u;
-    hipLaunchKernelGGL(k_fill_u64, dim3(4096), dim3(256), 0, c.stream, static_cast<uint64_t *>(kt.p), cap, kEmptyKey);
-    hipLaunchKernelGGL(k_key_put, dim3(blocks), dim3(256), 0, c.stream, static_cast<const int32_t *>(keys.p), n,
-                       static_cast<uint64_t *>(kt.p), static_cast<int32_t *>(vt.p), cap - 1u);
-    hipLaunchKernelGGL(k_neighbours, dim3((uint32_t)nb_blocks), dim3(256), 0, c.stream,
-                       static_cast<const int32_t *>(keys.p), n, static_cast<const uint64_t *>(kt.p),
-                       static_cast<const int32_t *>(vt.p), cap - 1u, static_cast<int32_t *>(nb.p));
-    // the tables (keys, kt, vt) are freed when this returns: wait for their readers
+    hipLaunchKernelGGL(k_fill_u64, dim3(4096), dim3(256), 0, c.stream, m.kt, cap, kEmptyKey);
+    hipLaunchKernelGGL(k_key_put, dim3(blocks), dim3(256), 0, c.stream, m.keys, n, m.kt, m.vt, cap - 1u);
+    hipLaunchKernelGGL(k_neighbours, dim3((uint32_t)nb_blocks), dim3(256), 0, c.stream, m.keys, n, m.kt, m.vt, cap - 1u,
+                       m.nb);
+    // the schedule reads the table on a stream of its own
     if (hipGetLastError() != hipSuccess || hipStreamSynchronize(c.stream) != hipSuccess) {
         err = "device SDF: neighbour table failed";
         c.status = WX_ERR_DEVICE;
@@ -529,23 +559,18 @@ class Scheduler {
     }
 
     // Allocates, computes the in-degrees and starts the rounds (nb must be complete).
-    bool start(uint32_t n, const DevBuf &nb, std::string &err) {
+    bool start(uint32_t n, const LevelMem &m, std::string &err) {
         n_ = n;
         if (hipGetDevice(&dev_) != hipSuccess || hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking) != hipSuccess) {
             err = "device SDF: schedule stream failed";
             return false;
         }
-        for (int p = 0; p < 2; ++p)
-            if (hipMalloc(&indeg_[p].p, (size_t)n * 4) != hipSuccess || hipMalloc(&order_[p].p, (size_t)n * 4) != hipSuccess) {
-                err = "device SDF: hipMalloc of the schedule buffers failed";
-                return false;
-            }
         if (!grow(4096, 0, err)) return false;
-        s_.nb = static_cast<const int32_t *>(nb.p);
+        s_.nb = m.nb;
         s_.n = n;
         for (int p = 0; p < 2; ++p) {
-            s_.indeg[p] = static_cast<uint32_t *>(indeg_[p].p);
-            s_.order[p] = static_cast<uint32_t *>(order_[p].p);
+            s_.indeg[p] = m.indeg[p];
+            s_.order[p] = m.order[p];
             hipLaunchKernelGGL(k_indegree, dim3((n + 255u) / 256u), dim3(256), 0, stream_, s_.nb, n, p == 0 ? 1 : 0,
                                s_.indeg[p], s_.order[p], &s_.rs[p][0].y);
         }
@@ -578,19 +603,18 @@ class Scheduler {
     bool grow(uint64_t want, uint64_t used, std::string &err) {
         uint64_t nc = cap_ ? cap_ : 4096;
         while (nc < want) nc *= 2;
-        for (int p = 0; p < 2; ++p) {
-            DevBuf nr;
-            if (hipMalloc(&nr.p, (nc + 1) * sizeof(uint2)) != hipSuccess ||
-                hipMemsetAsync(nr.p, 0, (nc + 1) * sizeof(uint2), stream_) != hipSuccess ||
-                (used && hipMemcpyAsync(nr.p, rs_[p].p, used * sizeof(uint2), hipMemcpyDeviceToDevice, stream_) !=
-                             hipSuccess) ||
-                hipStreamSynchronize(stream_) != hipSuccess) {  // the old records are freed below
-                err = "device SDF: schedule records: allocation or copy failed";
-                return false;
-            }
-            std::swap(rs_[p].p, nr.p);
-            s_.rs[p] = static_cast<uint2 *>(rs_[p].p);
+        DevBuf nr;  // both passes' records, one after the other
+        bool ok = hipMalloc(&nr.p, 2 * (nc + 1) * sizeof(uint2)) == hipSuccess &&
+                  hipMemsetAsync(nr.p, 0, 2 * (nc + 1) * sizeof(uint2), stream_) == hipSuccess;
+        uint2 *rs[2] = {static_cast<uint2 *>(nr.p), static_cast<uint2 *>(nr.p) + (nc + 1)};
+        for (int p = 0; p < 2 && used && ok; ++p)
+            ok = hipMemcpyAsync(rs[p], s_.rs[p], used * sizeof(uint2), hipMemcpyDeviceToDevice, stream_) == hipSuccess;
+        if (!ok || (used && hipStreamSynchronize(stream_) != hipSuccess)) {  // the old records are freed below
+            err = "device SDF: schedule records: allocation or copy failed";
+            return false;
         }
+        std::swap(rs_.p, nr.p);
+        for (int p = 0; p < 2; ++p) s_.rs[p] = rs[p];
         cap_ = nc;
         return true;
     }
@@ -644,7 +668,7 @@ class Scheduler {
     uint32_t n_ = 0;
     int dev_ = 0;
     hipStream_t stream_ = nullptr;
-    DevBuf indeg_[2], order_[2], rs_[2];
+    DevBuf rs_;
     uint64_t cap_ = 0;
     Schedule s_{};
     std::thread th_;
@@ -694,85 +718,65 @@ bool run_level(wx::SdfLevelJob &J, Ctx &c, std::string &err) {
     constexpr size_t S = (size_t)1 << (3 * LOG), W = S / 64;
     if (!J.nodes) return true;
     LevelTrace tr(LOG);
-    DevBuf solid, val, nb, ord0, ord1, nib, bad;
+    LevelMem mem;
+    DevBuf nib;
     const bool words = LOG == 3 && J.words;  // leaves leave as packed layout words, kept on the device
+    // masks a device generator left on this device are read where they are
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    const bool resident = J.nb.empty() && J.solid_dev && J.solid_dev_device == dev;
+    if (!mem.allocate(J, S, !resident, err)) return false;
     if (words) {
-        const uint32_t zero = 0;
-        if (hipMalloc(&nib.p, (size_t)J.nodes * 256) != hipSuccess || hipMalloc(&bad.p, 4) != hipSuccess) {
+        if (hipMalloc(&nib.p, (size_t)J.nodes * 256) != hipSuccess) {
             err = "device SDF: hipMalloc of the leaf words failed";
             return false;
         }
-        if (hipMemcpyAsync(bad.p, &zero, 4, hipMemcpyHostToDevice, c.stream) != hipSuccess ||
-            hipStreamSynchronize(c.stream) != hipSuccess) {
+        if (hipMemsetAsync(mem.bad, 0, 4, c.stream) != hipSuccess) {
             err = "device SDF: flag reset failed";
             return false;
         }
     }
     // every slot starts unknown (255): filled on the device instead of copied
-    auto make_val = [&] {
-        if (hipMalloc(&val.p, J.nodes * S) != hipSuccess) {
-            val.p = nullptr;
-            err = "device SDF: hipMalloc of the distance array failed";
-            return false;
-        }
-        if (hipMemsetAsync(val.p, kUnknown, J.nodes * S, c.stream) != hipSuccess) {
-            err = "device SDF: fill failed";
-            return false;
-        }
-        return true;
-    };
+    if (hipMemsetAsync(mem.val, kUnknown, J.nodes * S, c.stream) != hipSuccess) {
+        err = "device SDF: fill failed";
+        return false;
+    }
     // the solid masks come from pageable host memory; a large set goes through pinned
     // staging on a stream of the copier's own (host threads fill one buffer while the DMA
     // drains the other) and is on the device when this returns
     const size_t solid_bytes = J.nodes * W * sizeof(uint64_t);
     const bool staged = solid_bytes >= wx::PinnedCopier::kMin;
     auto staged_masks = [&](std::string &e) {
-        if (hipMalloc(&solid.p, solid_bytes) != hipSuccess) {
-            solid.p = nullptr;
-            e = "device SDF: hipMalloc of the solid masks failed";
-            return false;
-        }
         wx::PinnedCopier cp;
-        if (!cp.ok() || !cp.to_device(solid.p, J.solid, solid_bytes)) {
+        if (!cp.ok() || !cp.to_device(mem.solid, J.solid, solid_bytes)) {
             e = "device SDF: upload of the solid masks failed";
             return false;
         }
         return true;
     };
-    auto prepare = [&] {
-        if (!make_val()) return false;
-        return staged ? staged_masks(err) : upload(solid, J.solid, J.nodes * W, c.stream, err);
-    };
+    auto masks = [&] { return staged ? staged_masks(err) : upload(mem.solid, J.solid, J.nodes * W, c.stream, err); };
     std::unique_ptr<Scheduler> sch;  // outlives the sweeps, which read its groups
-    const uint64_t *sp = nullptr;     // the solid masks the sweeps read: solid, or the tree's device copy
+    const uint64_t *sp = resident ? static_cast<const uint64_t *>(J.solid_dev) : mem.solid;  // the masks the sweeps read
     auto sweep = [&](const uint32_t *group, uint32_t n, int fw) {
-        hipLaunchKernelGGL(k_sdf_nodes<LOG>, dim3(n), dim3(SweepShape<LOG>::kThreads), 0, c.stream, sp,
-                           static_cast<uint8_t *>(val.p), static_cast<const int32_t *>(nb.p), group,
-                           fw,
-                           fw ? nullptr : static_cast<uint32_t *>(nib.p), static_cast<uint32_t *>(bad.p));
+        hipLaunchKernelGGL(k_sdf_nodes<LOG>, dim3(n), dim3(SweepShape<LOG>::kThreads), 0, c.stream, sp, mem.val, mem.nb,
+                           group, fw, fw ? nullptr : static_cast<uint32_t *>(nib.p), mem.bad);
         ++c.launches;
     };
     if (!J.nb.empty()) {  // neighbour table and schedules from the host, one launch per group
-        if (!prepare() || !upload(nb, J.nb.data(), J.nb.size(), c.stream, err) ||
-            !upload(ord1, J.order[1].data(), J.order[1].size(), c.stream, err) ||
-            !upload(ord0, J.order[0].data(), J.order[0].size(), c.stream, err))
+        if (!masks() || !upload(mem.nb, J.nb.data(), J.nb.size(), c.stream, err) ||
+            !upload(mem.order[1], J.order[1].data(), J.order[1].size(), c.stream, err) ||
+            !upload(mem.order[0], J.order[0].data(), J.order[0].size(), c.stream, err))
             return false;
-        sp = static_cast<const uint64_t *>(solid.p);
         tr.phase("uploads");
         for (int fw = 1; fw >= 0; --fw) {  // forward pass, then backward
             const std::vector<uint32_t> &st = J.start[fw];
-            const uint32_t *ord = static_cast<const uint32_t *>(fw ? ord1.p : ord0.p);
             for (size_t g = 0; g + 1 < st.size(); ++g)
-                if (st[g + 1] > st[g]) sweep(ord + st[g], st[g + 1] - st[g], fw);
+                if (st[g + 1] > st[g]) sweep(mem.order[fw] + st[g], st[g + 1] - st[g], fw);
         }
     } else {  // the schedule on the device, its rounds overlapping the upload and the forward sweeps
         sch.reset(new Scheduler);
         // a large mask set goes up on a thread of its own while the neighbour table is built
         // and the rounds start (it has its own stream; the sweeps are launched after the join)
-        int dev = 0;
-        (void)hipGetDevice(&dev);
-        // masks a device generator left on this device are read where they are
-        const bool resident = J.solid_dev && J.solid_dev_device == dev;
         std::string up_err;
         bool up_ok = true;
         std::thread up;
@@ -786,10 +790,10 @@ bool run_level(wx::SdfLevelJob &J, Ctx &c, std::string &err) {
                     up_err = "device SDF: upload of the solid masks failed (host resources)";
                 }
             });
-        bool ok = build_neighbours(J, c, nb, err);
+        bool ok = build_neighbours(J, c, mem, err);
         if (ok) {
             tr.phase("neighbours");
-            ok = sch->start(J.nodes, nb, err);
+            ok = sch->start(J.nodes, mem, err);
         }
         if (up.joinable()) up.join();
         if (!ok) return false;
@@ -798,8 +802,7 @@ bool run_level(wx::SdfLevelJob &J, Ctx &c, std::string &err) {
             return false;
         }
         tr.phase("rounds started");
-        if (!(staged || resident ? make_val() : prepare())) return false;
-        sp = resident ? static_cast<const uint64_t *>(J.solid_dev) : static_cast<const uint64_t *>(solid.p);
+        if (!staged && !resident && !masks()) return false;
         tr.phase(resident ? "masks resident" : "masks up");
         if (!sweep_pass(*sch, 0, (uint32_t)J.nodes, sweep, c, err)) return false;
         tr.phase("forward queued");
@@ -809,8 +812,8 @@ bool run_level(wx::SdfLevelJob &J, Ctx &c, std::string &err) {
     uint32_t over = 0;
     tr.phase("launched");
     if (hipGetLastError() != hipSuccess ||
-        (words ? hipMemcpyAsync(&over, bad.p, 4, hipMemcpyDeviceToHost, c.stream)
-               : hipMemcpyAsync(J.val, val.p, J.nodes * S, hipMemcpyDeviceToHost, c.stream)) != hipSuccess ||
+        (words ? hipMemcpyAsync(&over, mem.bad, 4, hipMemcpyDeviceToHost, c.stream)
+               : hipMemcpyAsync(J.val, mem.val, J.nodes * S, hipMemcpyDeviceToHost, c.stream)) != hipSuccess ||
         hipStreamSynchronize(c.stream) != hipSuccess) {
         err = "device SDF: kernel or download failed";
         c.status = WX_ERR_DEVICE;
@@ -822,8 +825,6 @@ bool run_level(wx::SdfLevelJob &J, Ctx &c, std::string &err) {
         return false;
     }
     if (words) {  // the words stay where the device grid will be built
-        int dev = 0;
-        (void)hipGetDevice(&dev);
         J.kept.reset(new HipWords(nib.p, dev));
         nib.p = nullptr;
     }

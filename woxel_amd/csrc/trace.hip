@@ -991,40 +991,31 @@ int grid_new(const wx_grid_desc *d, const char *who, wx_grid **out) {
     const size_t sz[4] = {(size_t)d->n5 * 16u, (size_t)d->n5 * 4096u * 16u, (size_t)d->n4 * 256u * 16u,
                           (size_t)d->n3 * 64u * 4u};
     const void *src[4] = {d->root, d->n5_records, d->n4_records, d->leaves};
-    for (int k = 0; k < 4; ++k) {
-        size_t n = sz[k] ? sz[k] : 16;
-        hipError_t e = hipMalloc(&g->mem[k], n);
-        if (e != hipSuccess) {
-            g->mem[k] = nullptr;
-            wx_grid_destroy(g);
-            return set_error(e == hipErrorOutOfMemory ? WX_ERR_BUDGET : WX_ERR_DEVICE,
-                             w + ": hipMalloc: " + hipGetErrorString(e));
-        }
-        g->bytes += n;
-        if (sz[k] && src[k]) {
-            e = hipMemcpy(g->mem[k], src[k], sz[k], hipMemcpyHostToDevice);
-            if (e != hipSuccess) {
-                wx_grid_destroy(g);
-                return hip_fail(e, (w + ": hipMemcpy").c_str());
-            }
-        }
-    }
-    // the slot entries, made on the default stream after the copies and waited for, so the
-    // grid is complete for work on any stream
     const uint64_t nrec[3] = {(uint64_t)d->n5 * 4096u, (uint64_t)d->n4 * 256u, base.size()};
     const uint64_t rec_bytes[3] = {compact ? 16u : 32u, compact ? 32u : 64u, 4u};
-    hipError_t e = hipSuccess;
-    for (int k = 0; k < 3 && e == hipSuccess; ++k) {
-        const size_t n = std::max<size_t>(nrec[k] * rec_bytes[k], 16u);
-        e = hipMalloc(&g->entries[k], n);
-        if (e != hipSuccess) g->entries[k] = nullptr;
-        else g->bytes += n;
+    size_t n[7], all = 0;
+    for (int k = 0; k < 7; ++k) {
+        n[k] = std::max<size_t>(k < 4 ? sz[k] : nrec[k - 4] * rec_bytes[k - 4], 16u);
+        g->bytes += n[k];
+        all += wx::DeviceArena::piece(n[k]);
     }
+    hipError_t e = g->arena.allocate(all);
     if (e != hipSuccess) {
         wx_grid_destroy(g);
         return set_error(e == hipErrorOutOfMemory ? WX_ERR_BUDGET : WX_ERR_DEVICE,
                          w + ": hipMalloc: " + hipGetErrorString(e));
     }
+    for (int k = 0; k < 7; ++k) (k < 4 ? g->mem[k] : g->entries[k - 4]) = g->arena.take<void>(n[k]);
+    for (int k = 0; k < 4; ++k) {
+        if (!sz[k] || !src[k]) continue;
+        e = hipMemcpy(g->mem[k], src[k], sz[k], hipMemcpyHostToDevice);
+        if (e != hipSuccess) {
+            wx_grid_destroy(g);
+            return hip_fail(e, (w + ": hipMemcpy").c_str());
+        }
+    }
+    // the slot entries, made on the default stream after the copies and waited for, so the
+    // grid is complete for work on any stream
     const uint32_t *dbase = static_cast<const uint32_t *>(g->entries[2]) + d->n5;
     if (!base.empty()) e = hipMemcpy(g->entries[2], base.data(), base.size() * 4u, hipMemcpyHostToDevice);
     for (int k = 0; k < 2 && e == hipSuccess; ++k) {
@@ -1110,13 +1101,9 @@ int wx_vdb_grid_create(const wx_vdb *v, float bound, wx_grid **out) {
     wx_grid *g = nullptr;
     if (int rc = wx::grid_new(&d, "wx_vdb_grid_create", &g)) return rc;
     if (on_device && d.n3) {
-        // copied on a stream of its own and waited for, so the grid is complete for work
-        // on any stream when this returns
-        hipStream_t st = nullptr;
-        hipError_t e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
-        if (e == hipSuccess) e = hipMemcpyAsync(g->mem[3], dw->data(), (size_t)d.n3 * 256u, hipMemcpyDeviceToDevice, st);
-        if (e == hipSuccess) e = hipStreamSynchronize(st);
-        if (st) (void)hipStreamDestroy(st);
+        // waited for, so the grid is complete for work on any stream when this returns
+        hipError_t e = hipMemcpyAsync(g->mem[3], dw->data(), (size_t)d.n3 * 256u, hipMemcpyDeviceToDevice, nullptr);
+        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
         if (e != hipSuccess) {
             wx_grid_destroy(g);
             return hip_fail(e, "wx_vdb_grid_create: device copy of the leaf words");
@@ -1128,10 +1115,6 @@ int wx_vdb_grid_create(const wx_vdb *v, float bound, wx_grid **out) {
 
 int wx_grid_destroy(wx_grid *g) {
     if (!g) return WX_OK;
-    for (int k = 0; k < 4; ++k)
-        if (g->mem[k]) (void)hipFree(g->mem[k]);
-    for (int k = 0; k < 3; ++k)
-        if (g->entries[k]) (void)hipFree(g->entries[k]);
     delete g;
     return WX_OK;
 }
