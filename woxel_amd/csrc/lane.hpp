@@ -442,19 +442,21 @@ __device__ __forceinline__ void lane_finish(RayLane &r, bool capped) {
 
 // The rays of a wave whose lanes start together, to their end: the trip count, and with it
 // the step cap, is a scalar. The loop starts with the second half of an iteration, so that
-// leaving it is the only region between a lookup and the step after it.
+// leaving it is the only region between a lookup and the step after it; whether a ray left
+// it at its end or at the cap is asked again behind it, not carried through it (three scalar
+// instructions a step: 3837x2157 noise frame 467 -> 461 us, 1080p spheres 287 -> 284).
 template <bool kFast, uint32_t kForm>
 __device__ __forceinline__ void lane_loop(const GridDev &g, RayLane &r, const int4 *s_root, bool root_lds) {
     if (lane_state(r) != kRun) return;
-    bool run = lane_look<kFast, kForm>(g, r, s_root, root_lds);
-    if (run) {
+    if (lane_look<kFast, kForm>(g, r, s_root, root_lds)) {
         uint32_t looks = 1;
         do {
             lane_advance<kFast>(r);
-            run = lane_look<kFast, kForm>(g, r, s_root, root_lds);
-        } while (run && ++looks < kMaxSteps);
-        if (run) lane_advance<kFast>(r);
+            if (!lane_look<kFast, kForm>(g, r, s_root, root_lds)) break;
+        } while (++looks < kMaxSteps);
     }
+    const bool run = !(g.bound < fmaxf(fmaxf(fabsf(r.px), fabsf(r.py)), fabsf(r.pz))) & (r.size != 0.0f);
+    if (run) lane_advance<kFast>(r);
     lane_finish(r, run);
 }
 
