@@ -53,3 +53,21 @@ def test_frames(wx, cuda, scene, w, h):
         f = g.render_camera(cam, w, h, shade, 0.5, f32=True).cpu().numpy()
         rf, _ = lay.render_camera(cam.as_array(), w, h, shade, 0.5)
         assert np.array_equal(f.view(np.uint32), rf.view(np.uint32)), mode
+
+
+@pytest.mark.parametrize("n_grids,n_reqs", [(1, 2), (12, 24), (12, 25), (13, 24), (13, 25)])
+def test_batch_tables(wx, cuda, scene, n_grids, n_reqs):
+    """Both sides of the counts up to which a batch's tables are kernel arguments."""
+    print(f"{n_reqs} requests on {n_grids} grids", flush=True)
+    _, o = scene
+    g = [scene[0]] * n_grids
+    reqs, outs, want = [], [], []
+    for k in range(n_reqs):
+        w, h = 9 + 3 * k, 31 - k
+        cam = wx.camera_basis((300 - 9 * k, 250, -260 + 5 * k), (40, 35, 30), (0, 1, 0), w / h, 40.0, float(w))
+        outs.append(cuda.empty((w * h, 32), dtype=cuda.uint8, device="cuda"))
+        reqs.append(wx.camera_request((7 * k + n_grids - 1) % n_grids, cam, w, h, outs[-1], clip=True))
+        want.append(o.trace_camera(cam.as_array(), w, h, 0.5, clip=True)[0])
+    wx.trace_batch(g, reqs)
+    for k, (t, ora) in enumerate(zip(outs, want)):
+        assert_hits_equal(wx.hits_to_numpy(t), ora, f"request {k}")

@@ -114,8 +114,19 @@ struct BatchArgs {
     const uint32_t *begin;
     uint32_t n_grids, n_reqs, total, lg;
 };
+// The same with the tables among the kernel's arguments, which take 4 KiB at most: up to
+// 24 requests on 12 grids need no copy before the launch.
+constexpr uint32_t kInlineGrids = 12u, kInlineReqs = 24u;
+struct BatchInline {
+    ReqDev reqs[kInlineReqs];
+    GridDev grids[kInlineGrids];
+    uint32_t begin[kInlineReqs + 1u];
+    uint32_t n_reqs, total, lg;
+};
+static_assert(sizeof(BatchInline) <= 3968, "kernel arguments");
 
-__global__ __launch_bounds__(128) void k_simple_batch(BatchArgs a) {
+template <typename Tables>
+__global__ __launch_bounds__(128) void k_simple_batch(Tables a) {
     const uint32_t lane = threadIdx.x & 63u, slot = ((blockIdx.x * 2u + (threadIdx.x >> 6)) << a.lg) + lane;
     if (lane >> a.lg || slot >= a.total) return;
     // so the 64 slots of a wave belong to one request: find it once per wave
@@ -805,17 +816,29 @@ int launch_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs
                 }
             }
         } else {
-            BatchArgs b;
-            std::memset(&b, 0, sizeof b);
-            uint32_t *ctr = nullptr;
-            int rc = tables(&b.grids, &b.reqs, &b.begin, &ctr);
-            if (rc) return rc;
-            b.n_grids = n_grids;
-            b.n_reqs = n_reqs;
-            b.total = (uint32_t)total;
-            b.lg = rays_per_wave_log2(total);
-            hipLaunchKernelGGL(k_simple_batch, dim3((uint32_t)((total + (2u << b.lg) - 1u) >> (b.lg + 1u))), dim3(128), 0,
-                               stream, b);
+            const uint32_t lg = rays_per_wave_log2(total);
+            const dim3 grid((uint32_t)((total + (2u << lg) - 1u) >> (lg + 1u)));
+            if (n_reqs <= kInlineReqs && n_grids <= kInlineGrids) {
+                BatchInline b;
+                std::memcpy(b.reqs, q, sizeof(ReqDev) * n_reqs);
+                std::memcpy(b.begin, begin, 4u * (n_reqs + 1u));
+                for (uint32_t i = 0; i < n_grids; ++i) b.grids[i] = grids[i]->dev;
+                b.n_reqs = n_reqs;
+                b.total = (uint32_t)total;
+                b.lg = lg;
+                hipLaunchKernelGGL(k_simple_batch<BatchInline>, grid, dim3(128), 0, stream, b);
+            } else {
+                BatchArgs b;
+                std::memset(&b, 0, sizeof b);
+                uint32_t *ctr = nullptr;
+                int rc = tables(&b.grids, &b.reqs, &b.begin, &ctr);
+                if (rc) return rc;
+                b.n_grids = n_grids;
+                b.n_reqs = n_reqs;
+                b.total = (uint32_t)total;
+                b.lg = lg;
+                hipLaunchKernelGGL(k_simple_batch<BatchArgs>, grid, dim3(128), 0, stream, b);
+            }
         }
         e = hipGetLastError();
         if (e != hipSuccess) return hip_fail(e, "batch: launch");
