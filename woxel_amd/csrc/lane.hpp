@@ -272,9 +272,7 @@ __device__ __forceinline__ int32_t root_find(const GridDev &g, uint32_t x, uint3
 // a's bits where the mask is set, b's elsewhere (in C the compiler masks both operands first);
 // acc | (a ^ b) and acc | (~a & b).
 __device__ __forceinline__ uint32_t bits_of(uint32_t mask, uint32_t a, uint32_t b) {
-    uint32_t r;
-    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "s"(mask), "v"(a), "v"(b));
-    return r;
+    return (uint32_t)__builtin_amdgcn_bitop3_b32((int)mask, (int)a, (int)b, 0xCA);
 }
 __device__ __forceinline__ uint32_t or_xor(uint32_t acc, uint32_t a, uint32_t b) {
     return (uint32_t)__builtin_amdgcn_bitop3_b32((int)a, (int)b, (int)acc, 0xBE);
@@ -379,7 +377,7 @@ __device__ __forceinline__ bool lane_look(const GridDev &g, RayLane &r, const in
     // :96-98 hit (distance 0), then :101-103 any(bound < |p|) (NaN components compare
     // false either way)
     const bool run = opaque_and(!(g.bound < fmaxf(fmaxf(fabsf(r.px), fabsf(r.py)), fabsf(r.pz))), r.size != 0.0f);
-    if (kFast && min3_abs(r.px, r.py, r.pz) < 0x1p-64f) {  // a negative quotient that underflows has floor -0, not -1
+    if (kFast && fminf(fminf(fabsf(r.px), fabsf(r.py)), fabsf(r.pz)) < 0x1p-64f) {  // a negative quotient that underflows has floor -0, not -1
         if (fabsf(r.px) < 0x1p-64f && r.px / r.size == 0.0f) r.fx = 0.0f;
         if (fabsf(r.py) < 0x1p-64f && r.py / r.size == 0.0f) r.fy = 0.0f;
         if (fabsf(r.pz) < 0x1p-64f && r.pz / r.size == 0.0f) r.fz = 0.0f;
