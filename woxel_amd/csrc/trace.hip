@@ -1,6 +1,6 @@
 // HDDA + grid-SDF traversal kernels for gfx950, and the device-side C ABI.
 //
-// The per-lane traversal (RayLane, lane_step) lives in lane.hpp. The launch shapes
+// The per-lane traversal (RayLane, lane_look, lane_advance) lives in lane.hpp. The launch shapes
 // (wx_tune.persistent) share it:
 //  * k_simple_*: one lane per ray, 8x8-pixel wave tiles (the reference's dispatch
 //    shape); camera tiles dealt round-robin over the XCDs, or in one band per XCD
