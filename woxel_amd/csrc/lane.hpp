@@ -15,6 +15,7 @@
 
 #include "../../include/woxel_hip.h"
 #include "device_arena.hpp"
+#include "launch_shape.hpp"
 
 namespace wxk {
 
@@ -129,22 +130,6 @@ __device__ __forceinline__ T pool_at(const void *pool, uint32_t idx, uint32_t of
     const char *base = static_cast<const char *>(pool);
     if (kNarrow) return *reinterpret_cast<const T *>(base + ((idx << kShift) | off));
     return *reinterpret_cast<const T *>(base + (((uint64_t)idx << kShift) | off));
-}
-
-// How many rays a wave of the one-lane-per-ray shapes takes, as a power of two: 64, or fewer
-// in launches too small to fill the GPU, whose time is that of their longest waves. A wave
-// alone on its SIMD pays 50 clocks for a region of a step even to skip it, with 6 to 8 more
-// for each instruction inside and 129 or more for a load, and it enters a region when one of
-// its rays needs it, so fewer rays mean shorter steps and fewer of them; up to 4 waves per
-// SIMD (4096) hardly slow each other. 8 rays (4x2 pixels) were slower than 4 and 16 at most sizes.
-// Measured, 64 rays against this rule: 64x36 pixels of the ball 50.4 -> 41.4 us, of an
-// isosurface 77.1 -> 63.9, 160x90 pixels of 1000 spheres 112 -> 106, 448x252 164 -> 156;
-// 500 scattered rays 50.5 -> 43.0, 8000 66.5 -> 60.9, 128000 75.2 -> 77.0; panoramas of 8192
-// and 131072 rays 85.5 -> 74.2 and 129 -> 117.
-inline uint32_t rays_per_wave_log2(uint64_t rays) {
-    uint32_t lg = 0;
-    while (lg < 6u && (rays >> lg) > 4096u) ++lg;
-    return lg == 3u ? 4u : lg;
 }
 
 // Workgroup -> image tile under XCD-aware dispatch. The hardware hands workgroup b

@@ -799,17 +799,14 @@ int launch_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs
                 if (sh) hipLaunchKernelGGL(k_simple_camera<true>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], lg, band);
                 else hipLaunchKernelGGL(k_simple_camera<false>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], lg, band);
             } else {
-                const uint32_t lg = rays_per_wave_log2(total), per_group = 2u << lg;
-                dim3 grid((q[0].w + per_group - 1u) / per_group);
-                // a list with at least two sets of 64 rays for every wave the GPU holds goes to two
-                // kernels, each of which takes the sets that suit it (k_persist1): at 1 Mi rays
-                // scattered ones took 286 us against 346 in one kernel, a panorama 243 against 234;
-                // at half that scattered ones 251 against 193
-                const uint32_t sets = (q[0].w + 63u) / 64u, most = (uint32_t)cu_count() * 32u;
-                const uint32_t split = may_split && !sh && sets >= 2u * most ? 1u : 0u;
+                // split: the sets of 64 rays that scatter go to k_persist1, the others stay
+                const ListShape list = list_shape(q[0].w, (uint32_t)cu_count());
+                const uint32_t lg = list.lg, split = list.split && may_split && !sh ? 1u : 0u;
+                dim3 grid((q[0].w + (2u << lg) - 1u) >> (lg + 1u));
                 if (sh) hipLaunchKernelGGL(k_simple_rays<true>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], lg, 0u);
                 else hipLaunchKernelGGL(k_simple_rays<false>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], lg, split);
                 if (split) {
+                    const uint32_t sets = (q[0].w + 63u) / 64u, most = (uint32_t)cu_count() * 32u;
                     const uint32_t per_wave = (sets + most - 1u) / most;
                     launch_persist1<WX_REQ_RAYS>((sets + 4u * per_wave - 1u) / (4u * per_wave), stream, grids[0]->dev, q[0],
                                                  q[0].w, 24u, 1u);
