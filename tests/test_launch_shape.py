@@ -54,6 +54,14 @@ def test_split_lists_take_whole_sets(shape, cus):
 
 
 @pytest.mark.parametrize("cus", CUS)
+def test_small_waves_only_where_they_fit(shape, cus):
+    """A wave takes fewer than 64 rays only while four waves per SIMD hold them all."""
+    ns = lengths(cus)
+    for n, (lg, _) in zip(ns, shape([(n, cus) for n in ns])):
+        assert lg == 6 or n >> lg <= 16 * cus, (n, cus, lg)
+
+
+@pytest.mark.parametrize("cus", CUS)
 def test_every_ray_is_traced_once(shape, cus):
     """The two kernels' rules on a list of mixed directions: k_simple_rays takes 2^lg rays a wave
     and, in a split list, votes over the 64 from its first; k_persist1 votes over sets of 64."""

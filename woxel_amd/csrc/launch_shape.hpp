@@ -11,14 +11,14 @@ namespace wxk {
 // alone on its SIMD pays 50 clocks for a region of a step even to skip it, with 6 to 8 more
 // for each instruction inside and 129 or more for a load, and it enters a region when one of
 // its rays needs it, so fewer rays mean shorter steps and fewer of them; up to 4 waves per
-// SIMD (4096) hardly slow each other. 8 rays (4x2 pixels) were slower than 4 and 16 at most sizes.
-// Measured, 64 rays against this rule: 64x36 pixels of the ball 50.4 -> 41.4 us, of an
-// isosurface 77.1 -> 63.9, 160x90 pixels of 1000 spheres 112 -> 106, 448x252 164 -> 156;
-// 500 scattered rays 50.5 -> 43.0, 8000 66.5 -> 60.9, 128000 75.2 -> 77.0; panoramas of 8192
-// and 131072 rays 85.5 -> 74.2 and 129 -> 117.
-inline uint32_t rays_per_wave_log2(uint64_t rays) {
+// SIMD (16 per compute unit) hardly slow each other. 8 rays (4x2 pixels) were slower than 4
+// and 16 at most sizes. Measured on 256 compute units, 64 rays against this rule: 64x36
+// pixels of the ball 50.4 -> 41.4 us, of an isosurface 77.1 -> 63.9, 160x90 pixels of 1000
+// spheres 112 -> 106, 448x252 164 -> 156; 500 scattered rays 50.5 -> 43.0, 8000 66.5 -> 60.9,
+// 128000 75.2 -> 77.0; panoramas of 8192 and 131072 rays 85.5 -> 74.2 and 129 -> 117.
+inline uint32_t rays_per_wave_log2(uint64_t rays, uint32_t cus) {
     uint32_t lg = 0;
-    while (lg < 6u && (rays >> lg) > 4096u) ++lg;
+    while (lg < 6u && (rays >> lg) > 16u * cus) ++lg;
     return lg == 3u ? 4u : lg;
 }
 
@@ -34,7 +34,7 @@ struct ListShape {
 inline ListShape list_shape(uint64_t rays, uint32_t cus) {
     ListShape s;
     s.split = (rays + 63u) / 64u >= 2u * cus * 32u;
-    s.lg = s.split ? 6u : rays_per_wave_log2(rays);
+    s.lg = s.split ? 6u : rays_per_wave_log2(rays, cus);
     return s;
 }
 

@@ -590,8 +590,10 @@ bool tune_ok(const wx_tune &t) {
            t.waves_per_cu >= 1 && t.waves_per_cu <= 32 && t.xcd_split <= 2;
 }
 
+}  // namespace
+
 // CUs of the current device (queried once per device; thread-safe).
-int cu_count() {
+int wx::cu_count() {
     static std::mutex mu;
     static std::map<int, int> cus;
     int dev = 0;
@@ -604,9 +606,6 @@ int cu_count() {
     cus[dev] = n;
     return n;
 }
-
-}  // namespace
-
 
 namespace {
 
@@ -789,31 +788,32 @@ int launch_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs
         return WX_OK;
     };
     hipError_t e;
+    const uint32_t cus = (uint32_t)wx::cu_count();
     if (t.persistent != 1u) {  // the one-lane shape
         if (one) {
             const bool sh = (q[0].flags & WX_TRACE_SHADOW) != 0u;
             if (q[0].kind == WX_REQ_CAMERA) {
-                const uint32_t lg = rays_per_wave_log2(total), lw = 1u + ((lg + 1u) >> 1), lh = lg >> 1;
+                const uint32_t lg = rays_per_wave_log2(total, cus), lw = 1u + ((lg + 1u) >> 1), lh = lg >> 1;
                 dim3 grid((q[0].w + (1u << lw) - 1u) >> lw, (q[0].h + (1u << lh) - 1u) >> lh, 1);
                 const uint32_t band = t.xcd_split == 2u ? 1u : 0u;  // XCD-banded tile order
                 if (sh) hipLaunchKernelGGL(k_simple_camera<true>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], lg, band);
                 else hipLaunchKernelGGL(k_simple_camera<false>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], lg, band);
             } else {
                 // split: the sets of 64 rays that scatter go to k_persist1, the others stay
-                const ListShape list = list_shape(q[0].w, (uint32_t)cu_count());
+                const ListShape list = list_shape(q[0].w, cus);
                 const uint32_t lg = list.lg, split = list.split && may_split && !sh ? 1u : 0u;
                 dim3 grid((q[0].w + (2u << lg) - 1u) >> (lg + 1u));
                 if (sh) hipLaunchKernelGGL(k_simple_rays<true>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], lg, 0u);
                 else hipLaunchKernelGGL(k_simple_rays<false>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], lg, split);
                 if (split) {
-                    const uint32_t sets = (q[0].w + 63u) / 64u, most = (uint32_t)cu_count() * 32u;
+                    const uint32_t sets = (q[0].w + 63u) / 64u, most = cus * 32u;
                     const uint32_t per_wave = (sets + most - 1u) / most;
                     launch_persist1<WX_REQ_RAYS>((sets + 4u * per_wave - 1u) / (4u * per_wave), stream, grids[0]->dev, q[0],
                                                  q[0].w, 24u, 1u);
                 }
             }
         } else {
-            const uint32_t lg = rays_per_wave_log2(total);
+            const uint32_t lg = rays_per_wave_log2(total, cus);
             const dim3 grid((uint32_t)((total + (2u << lg) - 1u) >> (lg + 1u)));
             if (n_reqs <= kInlineReqs && n_grids <= kInlineGrids) {
                 BatchInline b;
@@ -843,7 +843,7 @@ int launch_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs
     }
     if (single) {
         // as many waves as asked for at most, each with the same number of sets of 64 slots
-        const uint64_t sets = total / 64u, most = (uint64_t)cu_count() * t.waves_per_cu;
+        const uint64_t sets = total / 64u, most = (uint64_t)cus * t.waves_per_cu;
         const uint64_t per_wave = (sets + most - 1u) / most;
         const uint32_t blocks = (uint32_t)(((sets + per_wave - 1u) / per_wave + 3u) / 4u);
         if (q[0].kind == WX_REQ_CAMERA)
@@ -864,7 +864,7 @@ int launch_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs
         // the queue counters start at zero: a fill kernel (no memset node, so the launch
         // sequence stays valid inside a captured graph)
         hipLaunchKernelGGL(k_zero, dim3(1), dim3(256), 0, stream, a.ctr, 16u * kRegions);
-        const uint32_t blocks = std::max<uint32_t>(1u, (uint32_t)cu_count() * t.waves_per_cu / 4u);
+        const uint32_t blocks = std::max<uint32_t>(1u, cus * t.waves_per_cu / 4u);
         hipLaunchKernelGGL(k_persist_batch, dim3(blocks), dim3(256), 0, stream, a);
     }
     e = hipGetLastError();

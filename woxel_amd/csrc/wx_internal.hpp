@@ -16,6 +16,9 @@ namespace wx {
 int set_error(int code, const std::string &msg);
 int ok();
 
+// Compute units of the current device.
+int cu_count();
+
 // Frees the batch scratch kept for `stream` (a hipStream_t about to be destroyed).
 void drop_stream_scratch(void *stream);
 
