@@ -1,0 +1,57 @@
+"""Edges of the rules that choose a path, each against the oracle or the general path, bit for bit."""
+import numpy as np
+import pytest
+
+from test_gpu_trace import assert_hits_equal
+
+pytestmark = pytest.mark.gpu
+
+
+def same_but_nan(gpu, ora, what):
+    """Every byte of the records, but for t where it is NaN on both sides (its bits are the hardware's)."""
+    nan = np.isnan(ora["t"])
+    assert np.array_equal(np.isnan(gpu["t"]), nan), what
+    gpu, ora = gpu.copy(), ora.copy()
+    gpu["t"][nan] = ora["t"][nan] = 0.0
+    assert_hits_equal(gpu, ora, what)
+
+
+@pytest.mark.parametrize("past", [-1, 0, 1])
+def test_general_step_in_long_lists(wx, oracle_mod, cuda, past):
+    """Lists one ray short of the length at which scattered sets of 64 go to the refilled waves,
+    and past it; rays of the general step that run on (a start of -0) and that turn NaN (a
+    direction component of -0) in scattered and in kept sets."""
+    n = 64 * 64 * cuda.cuda.get_device_properties(0).multi_processor_count - 64 + past
+    print(f"general step, {n} rays", flush=True)
+    rng = np.random.default_rng(abs(past) + 3)
+    sp = np.array([[2000.0, 1500.0, 1800.0, 60.0], [700.0, 900.0, 2500.0, 45.0], [300.0, 200.0, 250.0, 90.0]])
+    p = wx.Vdb345()
+    p.add_spheres(sp)
+    p.compute_sdf()
+    o = oracle_mod.Vdb()
+    for s in sp:
+        o.add_sphere(s[:3], s[3])
+    o.compute_sdf()
+    m = (n + 63) // 64 * 64
+    eye = rng.uniform(-3000, 4000, (m, 3))
+    d = sp[rng.integers(0, 3, m), :3] + rng.uniform(-60, 60, (m, 3)) - eye
+    rays = np.concatenate([eye, d], 1).reshape(-1, 64, 6)
+    rays[::3, :, :3] = rays[::3, :1, :3]  # one eye, neighbouring directions
+    rays[::3, :, 3:] = rays[::3, :1, 3:] + rng.uniform(-20, 20, rays[::3, :, 3:].shape)
+    rays = rays.reshape(m, 6)[:n]
+    rays[:, 3:] /= np.linalg.norm(rays[:, 3:], axis=1, keepdims=True)
+    rays = rays.astype(np.float32)
+    zero = rng.choice(n, 8000, replace=False)
+    rays[zero, rng.integers(0, 3, 8000)] = -0.0
+    nan = rng.integers(0, n, 3000)
+    rays[nan, 3 + rng.integers(0, 3, 3000)] = -0.0
+    t = cuda.from_numpy(rays).cuda()
+    g = wx.Grid(p)
+    for clip in (False, True):
+        ora, _ = o.trace_rays(rays, clip=clip)
+        gpu = wx.hits_to_numpy(g.trace_rays(t, clip=clip))
+        same_but_nan(gpu, ora, f"{n} rays, clip={clip}")
+        ran = zero[~np.isnan(ora["t"][zero]) & (ora["steps"][zero].sum(1) > 3)]
+        scattered = (ran // 64) % 3 != 0
+        assert scattered.sum() > 1000 and (~scattered).sum() > 500
+        assert (ora["state"][ran] == wx.HIT).sum() > 50
