@@ -55,3 +55,41 @@ def test_general_step_in_long_lists(wx, oracle_mod, cuda, past):
         scattered = (ran // 64) % 3 != 0
         assert scattered.sum() > 1000 and (~scattered).sum() > 500
         assert (ora["state"][ran] == wx.HIT).sum() > 50
+
+
+@pytest.mark.parametrize("bound", [4096.0, 2.0 ** 21])
+def test_degenerate_rays_in_every_shape(wx, oracle_mod, cuda, bound):
+    """Zeros, infinities, denormals and NaNs, quiet and signalling, in any component: every
+    shape gives the oracle's records (t where it is NaN aside), with and without the clip."""
+    print(f"degenerate rays, bound {bound}", flush=True)
+    rng = np.random.default_rng(5)
+    n = 64 * 300
+    sp = np.array([[40.0, 30.0, 45.0, 22.0], [90.0, 60.0, 20.0, 14.0], [-45.0, 40.0, 30.0, 19.0]])
+    r = np.concatenate([rng.uniform(-120, 120, (n, 3)), rng.standard_normal((n, 3))], 1).astype(np.float32)
+    odd = np.array([0.0, -0.0, np.inf, -np.inf, np.nan, 1e-40, -1e-39, 3e38, -3e38, 2.0 ** -64, -2.0 ** -66], np.float32)
+    m = rng.random(r.shape) < 0.12
+    r[m] = rng.choice(odd, m.sum())
+    bits = r.view(np.uint32)
+    m = np.isnan(r)
+    bits[m] = (rng.integers(0, 2, m.sum()).astype(np.uint32) << 31) | 0x7F800000 | rng.integers(1, 1 << 23, m.sum()).astype(np.uint32)
+    t = cuda.from_numpy(r).cuda()
+    tune = wx.tune_get()
+    for roots in (2, 3):
+        p = wx.Vdb345()
+        p.add_spheres(sp[:roots])
+        p.compute_sdf()
+        o = oracle_mod.Vdb()
+        for s in sp[:roots]:
+            o.add_sphere(s[:3], s[3])
+        o.compute_sdf()
+        g = wx.Grid(p, bound)
+        for clip in (False, True):
+            ora, _ = o.trace_rays(r, bound=bound, clip=clip)
+            for persistent in (0, 1):
+                print(f"{roots} spheres, clip {clip}, shape {persistent}", flush=True)
+                tune.persistent = persistent
+                for grids in ([g], [g, g]):
+                    out = [cuda.empty((n, 32), dtype=cuda.uint8, device="cuda") for _ in grids]
+                    wx.trace_batch(grids, [wx.rays_request(k, t, out[k], clip=clip) for k in range(len(grids))], tune)
+                    for x in out:
+                        same_but_nan(wx.hits_to_numpy(x), ora, f"{roots} {clip} {persistent} {len(grids)}")

@@ -164,9 +164,9 @@ __device__ __forceinline__ void lane_resume(RayLane &r, float px, float py, floa
 __device__ __forceinline__ void lane_start(RayLane &r, float ox, float oy, float oz, float dx, float dy, float dz,
                                            float B, bool clip) {
     // canonicalized: quiet a signalling NaN so that a max over |p| ignores it like the
-    // comparisons of the bound test do (every other value passes unchanged)
-    lane_resume(r, __builtin_canonicalizef(ox), __builtin_canonicalizef(oy), __builtin_canonicalizef(oz), dx, dy, dz,
-                1.0f / dx, 1.0f / dy, 1.0f / dz);  // :88
+    // comparisons of the bound test and of the clip below do (every other value passes unchanged)
+    ox = __builtin_canonicalizef(ox), oy = __builtin_canonicalizef(oy), oz = __builtin_canonicalizef(oz);
+    lane_resume(r, ox, oy, oz, dx, dy, dz, 1.0f / dx, 1.0f / dy, 1.0f / dz);  // :88
     if (clip && (B < fabsf(ox) || B < fabsf(oy) || B < fabsf(oz))) {
         float tn = -__builtin_inff(), tf = __builtin_inff();
         float a = (-B - ox) * r.ix, b = (B - ox) * r.ix;
