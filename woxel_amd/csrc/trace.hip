@@ -334,8 +334,8 @@ __global__ __launch_bounds__(256, 8) void k_persist1(GridDev g, ReqDev q, uint32
         do {
             ++trip;
             if (running) {
-                running = lane_look<true, kForm>(g, r, s_root_buf, root_lds);
-                if (running) lane_advance<true>(r);
+                running = lane_look<kFast, kForm>(g, r, s_root_buf, root_lds);
+                if (running) lane_advance<kFast>(r);
             }
             if (trip - oldest >= kMaxSteps && running && trip - s_start[threadIdx.x] == kMaxSteps)
                 capped = true, running = false;
@@ -351,7 +351,7 @@ __global__ __launch_bounds__(256, 8) void k_persist1(GridDev g, ReqDev q, uint32
         if (!in) continue;
         lane_start(r, o[0], o[1], o[2], d[0], d[1], d[2], g.bound, clip);
         if (lane_state(r) != kRun || (bounded && lane_fast(r))) continue;
-        lane_loop<false, kForm == kIndexed ? kIndexed : kTable>(g, r, s_root_buf, root_lds);
+        lane_loop<kGeneral, kForm == kIndexed ? kIndexed : kTable>(g, r, s_root_buf, root_lds);
         lane_write(r, o[0], o[1], o[2], q.out + pix);
     }
 }
@@ -434,9 +434,9 @@ __global__ __launch_bounds__(256) void k_persist_batch(PersistArgs a) {
                     if (on) advance(r);
                     if (!on || it == kMaxSteps) lane_finish(r, on);
                 };
-                if (g.form == kIndexed) step(lane_look<false, kIndexed>, lane_advance<false>);
-                else if (__ballot(slow) == 0ull) step(lane_look<true, kTable>, lane_advance<true>);
-                else step(lane_look<false, kTable>, lane_advance<false>);
+                if (g.form == kIndexed) step(lane_look<kGeneral, kIndexed>, lane_advance<kGeneral>);
+                else if (__ballot(slow) == 0ull) step(lane_look<kFast, kTable>, lane_advance<kFast>);
+                else step(lane_look<kGeneral, kTable>, lane_advance<kGeneral>);
             }
             if (lane_state(r) != kRun) {
                 const ReqDev &q = a.reqs[req];
