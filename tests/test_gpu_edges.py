@@ -1,4 +1,6 @@
 """Edges of the rules that choose a path, each against the oracle or the general path, bit for bit."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -93,3 +95,57 @@ def test_degenerate_rays_in_every_shape(wx, oracle_mod, cuda, bound):
                     wx.trace_batch(grids, [wx.rays_request(k, t, out[k], clip=clip) for k in range(len(grids))], tune)
                     for x in out:
                         same_but_nan(wx.hits_to_numpy(x), ora, f"{roots} {clip} {persistent} {len(grids)}")
+
+
+def far_layout(wx, p):
+    """The tree's layout with every second node-4 record finding its leaves in a copy further on."""
+    lay = p.layout_arrays()
+    n5, n4, n3 = lay["n"]
+    rec4 = lay["n4"].copy()
+    rec4[::2, 1] += n3 + 5000
+    leaves = np.concatenate([lay["leaves"], np.zeros((5000, 64), np.uint32), lay["leaves"]])
+    return lay["root"], lay["n5"], rec4, leaves
+
+
+def grid_of(wx, root, n5, n4, leaves, bound=4096.0):
+    keep = [np.ascontiguousarray(root, np.int32)] + [np.ascontiguousarray(a, np.uint32) for a in (n5, n4, leaves)]
+    d = wx.GridDesc()
+    d.n5, d.n4, d.n3, d.bound = keep[1].size // 16384, keep[2].size // 1024, keep[3].size // 64, bound
+    d.root = keep[0].ctypes.data_as(C.POINTER(C.c_int32))
+    d.n5_records, d.n4_records, d.leaves = [a.ctypes.data_as(C.POINTER(C.c_uint32)) for a in keep[1:]]
+    return wx.Grid.from_desc(d)
+
+
+def test_persistent_batches_of_every_form(wx, cuda):
+    """Batches with shadow rays on one grid of each form and on grids of all forms together:
+    the persistent shape gives the records of the one-lane shape, request by request."""
+    print("persistent batches", flush=True)
+    sp = np.array([[400.0, 300.0, 450.0, 120.0], [700.0, 600.0, 260.0, 90.0]])
+    trees = []
+    for shift in (0.0, -500.0):  # one node-5, eight
+        p = wx.Vdb345()
+        p.add_spheres(sp + [shift, shift, shift, 0.0])
+        p.compute_sdf()
+        trees.append(p)
+    every = [wx.Grid(trees[0]), wx.Grid(trees[1]), grid_of(wx, *far_layout(wx, trees[0])), wx.Grid(trees[0], 2.0 ** 20 + 1)]
+    w, h = 161, 93
+    for grids in ([every[0]], [every[1]], [every[2]], [every[3]], every):
+        print(f"{len(grids)} grids", flush=True)
+        got = {}
+        for persistent in (0, 1):
+            out = [cuda.zeros((w * h, 32), dtype=cuda.uint8, device="cuda") for _ in range(8)]
+            reqs = []
+            for k in range(4):
+                g = k % len(grids)
+                shift = 500.0 if grids[g] is every[1] else 0.0
+                cam = wx.camera_basis((1200 - 90 * k - shift, 900 - shift, -700 - shift), (500 - shift, 450 - shift, 380 - shift),
+                                      (0, 1, 0), w / h, 45.0, float(w))
+                reqs.append(wx.camera_request(g, cam, w, h, out[2 * k], shadow_out=out[2 * k + 1],
+                                              light=(900.0 - shift, 2000.0 - shift, 300.0 - shift)))
+            wx.trace_batch(grids, reqs, wx.Tune(persistent=persistent, refill=16, chunk=128, waves_per_cu=16, xcd_split=1))
+            got[persistent] = [x.cpu().numpy() for x in out]
+        hits = 0
+        for a, b in zip(got[0], got[1]):
+            assert np.array_equal(a, b)
+            hits += int((a.view(wx.HIT_DTYPE)["state"] == wx.HIT).sum())
+        assert hits > 1000

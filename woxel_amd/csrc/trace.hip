@@ -357,21 +357,30 @@ __global__ __launch_bounds__(256, 8) void k_persist1(GridDev g, ReqDev q, uint32
 }
 
 // Any batch: many requests and grids, shadow rays continued in the lane of
-// their primary. Ray origins live in LDS (one per lane). A lane keeps its
-// request's grid index in a register and reads that grid's descriptor from LDS
-// on each step; the 128-byte request record is read when a ray starts or ends.
-__global__ __launch_bounds__(256) void k_persist_batch(PersistArgs a) {
-    __shared__ GridDev s_grid[kMaxGridsLds];
+// their primary. Ray origins live in LDS (one per lane); the 128-byte request record is read
+// when a ray starts or ends. kForm is the form of the batch's only grid, whose descriptor is
+// then an argument, or kMixed: lanes trace different grids, keep theirs as an index and
+// read its descriptor from LDS on each step. The general step alone: lanes here are at
+// different depths and enter every region of a step, so the fast step gained less than the
+// registers of both lost (112, four waves per SIMD; 96 with one, five for one grid). Measured
+// against both steps and per-lane descriptors for one grid: a shadowed 1080p request
+// 2800 -> 2440 us, 12 of 640x360 1445 -> 1330 (16 waves per CU), on eight node-5s 3340 -> 2890.
+constexpr uint32_t kMixed = 3u;
+template <uint32_t kForm>
+__global__ __launch_bounds__(256, kForm == kMixed ? 4 : 5) void k_persist_batch(PersistArgs a, GridDev one) {
+    constexpr bool mixed = kForm == kMixed;
+    __shared__ GridDev s_grid[mixed ? kMaxGridsLds : 1u];
     __shared__ uint32_t s_begin[kMaxReqsLds + 1];
     __shared__ float s_org[3][256];
-    for (uint32_t i = threadIdx.x; i < a.n_grids; i += 256u) s_grid[i] = a.grids[i];
+    if (mixed)
+        for (uint32_t i = threadIdx.x; i < a.n_grids; i += 256u) s_grid[i] = a.grids[i];
     for (uint32_t i = threadIdx.x; i <= a.n_reqs; i += 256u) s_begin[i] = a.begin[i];
     __syncthreads();
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t lt = (1ull << lane) - 1ull;
     WaveQueue wq;
     wq.init(a);
-    bool alive = false, shadow = false, slow = false;
+    bool alive = false, shadow = false;
     uint32_t req = 0, gi = 0, pix = 0, it = 0;
     RayLane r;
     r.state = 0;
@@ -410,11 +419,10 @@ __global__ __launch_bounds__(256) void k_persist_batch(PersistArgs a) {
                 }
                 if (ok) {
                     gi = q.grid;
-                    lane_start(r, ox, oy, oz, dx, dy, dz, s_grid[gi].bound, (q.flags & WX_TRACE_CLIP) != 0u);
+                    lane_start(r, ox, oy, oz, dx, dy, dz, mixed ? s_grid[gi].bound : one.bound, (q.flags & WX_TRACE_CLIP) != 0u);
                     s_org[0][threadIdx.x] = ox, s_org[1][threadIdx.x] = oy, s_org[2][threadIdx.x] = oz;
                     req = lo;
                     it = 0;
-                    slow = s_grid[gi].bound > kFastBound || !lane_fast(r);
                     shadow = false;
                     alive = true;
                 }
@@ -426,7 +434,7 @@ __global__ __launch_bounds__(256) void k_persist_batch(PersistArgs a) {
             continue;
         }
         if (alive) {
-            const GridDev &g = s_grid[gi];
+            const GridDev &g = mixed ? s_grid[gi] : one;
             if (lane_state(r) == kRun) {
                 ++it;
                 auto step = [&](auto look, auto advance) {
@@ -434,8 +442,8 @@ __global__ __launch_bounds__(256) void k_persist_batch(PersistArgs a) {
                     if (on) advance(r);
                     if (!on || it == kMaxSteps) lane_finish(r, on);
                 };
-                if (g.form == kIndexed) step(lane_look<kGeneral, kIndexed>, lane_advance<kGeneral>);
-                else if (__ballot(slow) == 0ull) step(lane_look<kFast, kTable>, lane_advance<kFast>);
+                if constexpr (!mixed) step(lane_look<kGeneral, kForm>, lane_advance<kGeneral>);
+                else if (g.form == kIndexed) step(lane_look<kGeneral, kIndexed>, lane_advance<kGeneral>);
                 else step(lane_look<kGeneral, kTable>, lane_advance<kGeneral>);
             }
             if (lane_state(r) != kRun) {
@@ -450,7 +458,6 @@ __global__ __launch_bounds__(256) void k_persist_batch(PersistArgs a) {
                         start_shadow(r, q, g.bound, sx, sy, sz);
                         s_org[0][threadIdx.x] = sx, s_org[1][threadIdx.x] = sy, s_org[2][threadIdx.x] = sz;
                         it = 0;
-                        slow = g.bound > kFastBound || !lane_fast(r);
                         shadow = true;
                         alive = true;
                         if (lane_state(r) != kRun) {  // the shadow ray missed the bound box
@@ -865,7 +872,12 @@ int launch_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs
         // sequence stays valid inside a captured graph)
         hipLaunchKernelGGL(k_zero, dim3(1), dim3(256), 0, stream, a.ctr, 16u * kRegions);
         const uint32_t blocks = std::max<uint32_t>(1u, cus * t.waves_per_cu / 4u);
-        hipLaunchKernelGGL(k_persist_batch, dim3(blocks), dim3(256), 0, stream, a);
+        const dim3 n(blocks), th(256);
+        const GridDev &g = grids[0]->dev;
+        if (n_grids != 1u) hipLaunchKernelGGL(k_persist_batch<kMixed>, n, th, 0, stream, a, g);
+        else if (g.form == kOneRoot) hipLaunchKernelGGL(k_persist_batch<kOneRoot>, n, th, 0, stream, a, g);
+        else if (g.form == kTable) hipLaunchKernelGGL(k_persist_batch<kTable>, n, th, 0, stream, a, g);
+        else hipLaunchKernelGGL(k_persist_batch<kIndexed>, n, th, 0, stream, a, g);
     }
     e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "batch: launch");
