@@ -14,9 +14,9 @@ PROGRAM = """
 #include "launch_shape.hpp"
 int main() {
     unsigned long long rays;
-    unsigned cus;
-    while (std::scanf("%llu %u", &rays, &cus) == 2) {
-        const wxk::ListShape s = wxk::list_shape(rays, cus);
+    unsigned cus, refills;
+    while (std::scanf("%llu %u %u", &rays, &cus, &refills) == 3) {
+        const wxk::ListShape s = wxk::list_shape(rays, cus, refills != 0u);
         std::printf("%u %u\\n", s.lg, s.split ? 1u : 0u);
     }
 }
@@ -30,9 +30,9 @@ def shape(tmp_path_factory):
     csrc = os.path.join(HERE, "..", "woxel_amd", "csrc")
     subprocess.run(["g++", "-std=c++17", "-O1", "-I", csrc, str(d / "p.cpp"), "-o", str(d / "p")], check=True)
 
-    def ask(pairs):
-        r = subprocess.run([str(d / "p")], input="".join(f"{n} {c}\n" for n, c in pairs), capture_output=True,
-                           text=True, check=True)
+    def ask(pairs, refills=1):
+        r = subprocess.run([str(d / "p")], input="".join(f"{n} {c} {refills}\n" for n, c in pairs),
+                           capture_output=True, text=True, check=True)
         return [tuple(int(x) for x in line.split()) for line in r.stdout.splitlines()]
 
     return ask
@@ -51,6 +51,12 @@ def test_split_lists_take_whole_sets(shape, cus):
     assert any(s for _, s in got) and not all(s for _, s in got)
     for n, (lg, split) in zip(ns, got):
         assert not split or lg == 6, (n, cus, lg)
+
+
+@pytest.mark.parametrize("cus", CUS)
+def test_grids_without_the_fast_step_keep_their_lists(shape, cus):
+    ns = lengths(cus)
+    assert not any(s for _, s in shape([(n, cus) for n in ns], refills=0))
 
 
 @pytest.mark.parametrize("cus", CUS)

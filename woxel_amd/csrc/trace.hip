@@ -807,7 +807,7 @@ int launch_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs
                 else hipLaunchKernelGGL(k_simple_camera<false>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], lg, band);
             } else {
                 // split: the sets of 64 rays that scatter go to k_persist1, the others stay
-                const ListShape list = list_shape(q[0].w, cus);
+                const ListShape list = list_shape(q[0].w, cus, grids[0]->dev.bound <= kFastBound);
                 const uint32_t lg = list.lg, split = list.split && may_split && !sh ? 1u : 0u;
                 dim3 grid((q[0].w + (2u << lg) - 1u) >> (lg + 1u));
                 if (sh) hipLaunchKernelGGL(k_simple_rays<true>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], lg, 0u);
