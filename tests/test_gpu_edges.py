@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 from test_gpu_trace import assert_hits_equal
+from woxel_amd import scenes
 
 pytestmark = pytest.mark.gpu
 
@@ -149,3 +150,22 @@ def test_persistent_batches_of_every_form(wx, cuda):
             assert np.array_equal(a, b)
             hits += int((a.view(wx.HIT_DTYPE)["state"] == wx.HIT).sum())
         assert hits > 1000
+
+
+def test_autotune_of_one_request_leaves_the_queue_alone(wx, cuda):
+    """One request without shadow rays has no work queue: its chunk and XCD split stay the defaults."""
+    print("autotune of one request", flush=True)
+    p = wx.Vdb345()
+    p.add_spheres(scenes.sphere_set(2, count=300))
+    p.compute_sdf()
+    g = wx.Grid(p)
+    rays = cuda.from_numpy(scenes.incoherent_rays(1 << 18)).cuda().repeat(16, 1)  # the persistent shape wins
+    out = cuda.empty((len(rays), 32), dtype=cuda.uint8, device="cuda")
+    old = wx.tune_get()
+    try:
+        for _ in range(4):
+            t, _ = wx.autotune([g], [wx.rays_request(0, rays, out)])
+            print(t.as_dict(), flush=True)
+            assert (t.chunk, t.xcd_split) == (256, 1)
+    finally:
+        wx.tune_set(old)

@@ -1257,8 +1257,10 @@ int wx_autotune(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs,
         ms = acc / 3.f;
         return WX_OK;
     };
-    // the one-lane-per-ray shape, then a coordinate search over the persistent shape:
-    // waves, refill, chunk, XCD split
+    // the one-lane-per-ray shape, then a coordinate search over the persistent shape: waves,
+    // refill and, where there is a work queue (not for one request without shadow rays), chunk
+    // and XCD split
+    const bool queue = n_reqs > 1u || n_grids > 1u || (reqs[0].flags & WX_TRACE_SHADOW);
     {
         wx_tune c = default_tune();
         c.persistent = 0;
@@ -1288,6 +1290,7 @@ int wx_autotune(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs,
         }
         t = pbest;
         for (uint32_t ch : chunks) {
+            if (!queue) break;
             wx_tune c = t;
             c.chunk = ch;
             float ms;
@@ -1295,7 +1298,7 @@ int wx_autotune(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs,
             if (ms < pms) pms = ms, pbest = c;
         }
         t = pbest;
-        for (uint32_t x = 0; x <= 1; ++x) {
+        for (uint32_t x = 0; x <= 1 && queue; ++x) {
             wx_tune c = t;
             c.xcd_split = x;
             float ms;
