@@ -169,3 +169,14 @@ def test_autotune_of_one_request_leaves_the_queue_alone(wx, cuda):
             assert (t.chunk, t.xcd_split) == (256, 1)
     finally:
         wx.tune_set(old)
+
+
+@pytest.mark.parametrize("freq", [0.11, 2e5, 3e5, 1e6, 3e8, 1e38])
+def test_noise_threshold_of_any_frequency(wx, cuda, freq):
+    """The device's threshold is the host's also where a lattice coordinate leaves int32, which
+    the two convert differently (the frequencies lie on both sides of 2^30 / 4 / 1000)."""
+    print(f"noise threshold at frequency {freq}", flush=True)
+    for lo, hi in (((0, 0, 0), (1000, 40, 30)), ((-1000, 5, -7), (-900, 60, 20))):
+        th = wx.Vdb345().add_noise(9, lo, hi, freq, 0.3, threads=2)
+        td = wx.Vdb345().add_noise(9, lo, hi, freq, 0.3, device=True)
+        assert np.float32(th).view(np.uint32) == np.float32(td).view(np.uint32)

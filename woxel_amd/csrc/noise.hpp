@@ -134,6 +134,18 @@ WX_NOISE_FN float sample(const Params &p, uint64_t &st) {
     return noise3(p.seed, p.f0, (float)q[0], (float)q[1], (float)q[2]);
 }
 
+// Whether every lattice coordinate of the noise in [lo, hi) fits an int32 (with room for its
+// cell's far corner). Beyond it the conversion differs between host and device.
+inline bool lattice_in_range(const Params &p) {
+    float far = 0.0f;
+    for (int a = 0; a < 3; ++a) {
+        const float l = __builtin_fabsf((float)p.lo[a]), h = __builtin_fabsf((float)p.hi[a]);
+        far = far < l ? l : far;
+        far = far < h ? h : far;
+    }
+    return far * p.f0 * (float)(1 << (kOctaves - 1)) < 0x1p30f;
+}
+
 WX_NOISE_FN uint64_t sample_start(uint64_t seed) { return seed * 0x9E3779B97F4A7C15ull + 1; }
 
 // Leaf class from its centre value: 0 = no active voxel, 1 = every voxel active,

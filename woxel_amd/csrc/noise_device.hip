@@ -310,7 +310,9 @@ extern "C" int wx_vdb_add_noise_device(wx_vdb *v, uint64_t seed, const int32_t l
                          2 * piece(slab * 8) + piece(tmp_bytes)) != hipSuccess)
             return set_error(WX_ERR_BUDGET, "wx_vdb_add_noise_device: hipMalloc of the slab buffers failed");
         uint32_t *const dcnt = mem.take<uint32_t>(8);
-        if (int rc = device_threshold(seed, p, rank, mem.take<void>(kThresholdBytes), st)) return rc;
+        void *const tmem = mem.take<void>(kThresholdBytes);
+        if (!wxnoise::lattice_in_range(p)) p.thr = wx::HostVdb::noise_threshold(seed, p, rank);
+        else if (int rc = device_threshold(seed, p, rank, tmem, st)) return rc;
         uint8_t *const masks = mem.take<uint8_t>(slab * 64);
         int32_t *const keys = mem.take<int32_t>(slab * 12);
         uint32_t *const todo = mem.take<uint32_t>(slab * 4), *const idx = mem.take<uint32_t>(slab * 4),

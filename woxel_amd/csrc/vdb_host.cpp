@@ -493,16 +493,20 @@ bool HostVdb::noise_params(uint64_t seed, const int32_t lo[3], const int32_t hi[
     return true;
 }
 
+float HostVdb::noise_threshold(uint64_t seed, const wxnoise::Params &p, size_t rank) {
+    std::vector<float> smp(wxnoise::kSamples);
+    uint64_t st = wxnoise::sample_start(seed);
+    for (float &v : smp) v = wxnoise::sample(p, st);
+    std::nth_element(smp.begin(), smp.begin() + (ptrdiff_t)rank, smp.end());
+    return smp[rank];
+}
+
 bool HostVdb::add_noise(uint64_t seed, const int32_t lo[3], const int32_t hi[3], float base_freq, float occupancy,
                         int threads, float *threshold, std::string &err) {
     wxnoise::Params prm;
     size_t rank = 0;
     if (!noise_params(seed, lo, hi, base_freq, occupancy, prm, rank, err)) return false;
-    std::vector<float> smp(wxnoise::kSamples);
-    uint64_t st = wxnoise::sample_start(seed);
-    for (float &v : smp) v = wxnoise::sample(prm, st);
-    std::nth_element(smp.begin(), smp.begin() + (ptrdiff_t)rank, smp.end());
-    prm.thr = smp[rank];
+    prm.thr = noise_threshold(seed, prm, rank);
     if (threshold) *threshold = prm.thr;
     const int32_t l0[3] = {lo[0] >> 3, lo[1] >> 3, lo[2] >> 3};
     const int32_t l1[3] = {(hi[0] - 1) >> 3, (hi[1] - 1) >> 3, (hi[2] - 1) >> 3};

@@ -119,6 +119,8 @@ class HostVdb {
     // sample that is the threshold (for a generator elsewhere, the device one: same voxels).
     bool noise_params(uint64_t seed, const int32_t lo[3], const int32_t hi[3], float base_freq, float occupancy,
                       wxnoise::Params &p, size_t &rank, std::string &err) const;
+    // The threshold of those parameters: the sample of this rank.
+    static float noise_threshold(uint64_t seed, const wxnoise::Params &p, size_t rank);
     // Append leaves the caller guarantees are new: keys unique and absent from the
     // tree, masks non-zero. No hashing; the key index is rebuilt on the next lookup.
     bool append_new_leaves(const int32_t *keys, const uint64_t *masks, size_t n, std::string &err);
