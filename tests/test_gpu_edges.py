@@ -180,3 +180,31 @@ def test_noise_threshold_of_any_frequency(wx, cuda, freq):
         th = wx.Vdb345().add_noise(9, lo, hi, freq, 0.3, threads=2)
         td = wx.Vdb345().add_noise(9, lo, hi, freq, 0.3, device=True)
         assert np.float32(th).view(np.uint32) == np.float32(td).view(np.uint32)
+
+
+def test_root_keys_of_any_size(wx, cuda):
+    """A descriptor's only node-5 may have any int32 key; one that no voxel has (2^20 past the
+    scene's, which is the same coordinate mod 2^32) leaves every lookup a root miss."""
+    print("root keys", flush=True)
+    p = wx.Vdb345()
+    p.add_spheres(np.array([[400.0, 300.0, 450.0, 120.0]]))
+    p.compute_sdf()
+    lay = p.layout_arrays()
+    cam = wx.camera_basis((1200, 900, -700), (400, 300, 450), (0, 1, 0), 1.5, 45.0, 96.0)
+
+    def records(key, persistent):
+        root = lay["root"].copy().reshape(-1, 4)
+        root[0, :3] = key
+        g = grid_of(wx, root, lay["n5"], lay["n4"], lay["leaves"])
+        out = [cuda.empty((96 * 64, 32), dtype=cuda.uint8, device="cuda") for _ in range(2)]
+        tune = wx.Tune(persistent=persistent, refill=16, chunk=128, waves_per_cu=16, xcd_split=1)
+        wx.trace_batch([g], [wx.camera_request(0, cam, 96, 64, out[0])], tune)
+        wx.trace_batch([g], [wx.camera_request(0, cam, 96, 64, x) for x in out], tune)
+        return wx.hits_to_numpy(out[1])
+
+    assert (records((0, 0, 0), 0)["state"] == wx.HIT).any()
+    away = records((3, 0, 0), 0)  # inside what a key can be, outside the rays' box
+    assert (away["state"] != wx.HIT).all() and (away["lookups"] == 0).all()
+    for key in ((1 << 20, 0, 0), (0, -(1 << 20), 0), (0, 0, -(1 << 31)), ((1 << 20) + 1, 1 << 20, 0)):
+        for persistent in (0, 1):
+            assert_hits_equal(records(key, persistent), away, f"key {key}")

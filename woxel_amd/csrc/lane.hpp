@@ -48,7 +48,8 @@ static_assert(sizeof(GridDev) == 64, "GridDev layout");
 // child indices (measured first) took twice that and lost on the 4096^3 sphere set what
 // the shorter lookup gained: L2 requests per frame 13.4 M (records), 23.9 M (4 bytes).
 // Forms of a grid, from its node counts and records (wx_grid_create):
-//   kOneRoot  compact entries, one node-5 of base 0, every pool within 32-bit byte offsets;
+//   kOneRoot  compact entries, one node-5 of base 0 with a key of 20 bits, every pool within
+//             32-bit byte offsets;
 //   kTable    compact entries, any root table, 64-bit addresses;
 //   kIndexed  4-byte entries (kWalk32 | child index, or the size as a float) for a layout
 //             whose children are not consecutive, which no builder here makes.

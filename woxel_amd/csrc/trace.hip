@@ -1081,7 +1081,11 @@ int grid_new(const wx_grid_desc *d, const char *who, wx_grid **out) {
     // WX_WIDE_LEAVES=1 takes the 64-bit pool addressing at any size (to test it on small grids)
     const char *wide = std::getenv("WX_WIDE_LEAVES");
     const bool narrow = d->n3 <= (1u << 24) && !(wide && wide[0] == '1');
-    g->dev.form = !compact ? kIndexed : (d->n5 == 1u && base[0] == 0u - kWalk && narrow ? kOneRoot : kTable);
+    // a key that 20 bits hold is one that a voxel coordinate mod 2^32 decides (lane_lookup)
+    auto key_fits = [](int32_t k) { return k >= -(1 << 19) && k < (1 << 19); };
+    const bool one_root = d->n5 == 1u && base[0] == 0u - kWalk && key_fits(g->dev.kx) && key_fits(g->dev.ky) &&
+                          key_fits(g->dev.kz);
+    g->dev.form = !compact ? kIndexed : (one_root && narrow ? kOneRoot : kTable);
     *out = g;
     return WX_OK;
 }
