@@ -20,6 +20,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -1014,7 +1015,11 @@ int grid_new(const wx_grid_desc *d, const char *who, wx_grid **out) {
         return set_error(WX_ERR_UNSUPPORTED, w + ": more than 65536 node-5 or 2^20 node-4 nodes");
     std::vector<uint32_t> base;
     bool compact = true;
-    if (int rc = check_desc(d, who, base, compact)) return rc;
+    try {  // base takes 4 bytes per node
+        if (int rc = check_desc(d, who, base, compact)) return rc;
+    } catch (const std::bad_alloc &) {
+        return set_error(WX_ERR_BUDGET, w + ": host allocation failed");
+    }
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) return set_error(WX_ERR_DEVICE, w + ": no HIP device");
     wx_grid *g = new (std::nothrow) wx_grid();
