@@ -14,6 +14,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cstdint>
 #include <cstdlib>
@@ -600,18 +601,16 @@ bool tune_ok(const wx_tune &t) {
 
 }  // namespace
 
-// CUs of the current device (queried once per device; thread-safe).
+// CUs of the current device, queried once per device; no lock and no allocation, as the
+// allocation-free launches ask too.
 int wx::cu_count() {
-    static std::mutex mu;
-    static std::map<int, int> cus;
-    int dev = 0;
+    static std::atomic<int> cus[16];
+    int dev = 0, n = 0;
     (void)hipGetDevice(&dev);
-    std::lock_guard<std::mutex> lk(mu);
-    auto it = cus.find(dev);
-    if (it != cus.end()) return it->second;
-    int n = 0;
+    std::atomic<int> *const known = dev >= 0 && dev < 16 ? &cus[dev] : nullptr;
+    if (known && (n = known->load(std::memory_order_relaxed)) > 0) return n;
     if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cus[dev] = n;
+    if (known) known->store(n, std::memory_order_relaxed);
     return n;
 }
 
