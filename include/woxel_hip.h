@@ -101,15 +101,16 @@ typedef struct wx_tune {
     uint32_t persistent;   /* 0: one lane per ray (a ray list of a million rays or more without
                                  shadow rays also goes through refilled waves, for the runs of 64
                                  whose directions have nothing in common);
-                              1: persistent waves whose idle lanes are refilled: one request in
-                                 equal shares, others from a work queue (fields below);
+                              1: persistent waves whose idle lanes are refilled: one request
+                                 without shadow rays in equal shares, others from a work queue
+                                 (fields below);
                               2, 3: as 0 (two shapes that measured slower than it: compacting
                                  workgroups, node-5 records in LDS) */
     uint32_t refill;       /* 1: refill a wave's idle lanes once at least this many are idle (1..64) */
-    uint32_t chunk;        /* 1, several requests: work slots a wave takes from the queue at once
+    uint32_t chunk;        /* 1, work queue: work slots a wave takes from the queue at once
                               (multiple of 64) */
     uint32_t waves_per_cu; /* 1: waves per CU launched (1..32) */
-    uint32_t xcd_split;    /* 1, several requests: nonzero = one queue region per XCD, stealing when
+    uint32_t xcd_split;    /* 1, work queue: nonzero = one queue region per XCD, stealing when
                               drained; 0 = one region. Shape 0 camera requests: 2 = each XCD takes one
                               contiguous band of the image's 16x8 tiles, else the hardware's
                               round-robin of tiles over the XCDs */
@@ -266,7 +267,9 @@ int wx_grid_create(const wx_grid_desc *desc, wx_grid **out);
  * grid on another device than the replay's, take the host copy. */
 int wx_vdb_grid_create(const wx_vdb *v, float bound, wx_grid **out);
 int wx_grid_destroy(wx_grid *g);
-/* Device bytes held by the grid. */
+/* Device bytes held by the grid: the layout's pools, and the slot entries that the traversal
+ * reads, made of its node records (64 KiB more a node-5, 8 KiB a node-4; twice that where a
+ * node's children are not consecutive). */
 int wx_grid_bytes(const wx_grid *g, uint64_t *out);
 
 /* ---------------- grid-layout cache ----------------
@@ -343,7 +346,7 @@ int wx_tune_set(const wx_tune *t);
  * `stream`; grids must stay alive until the work completes.
  * HIP graph capture: a call with one request on one grid launches kernels whose
  * arguments are all passed by value, and may be captured and replayed (in shape 1
- * without a shadow ray). Other calls (several requests or grids) stage tables and
+ * without shadow rays). Other calls (several requests or grids) stage tables and
  * queue counters in per-stream scratch memory that later calls reuse or grow, and
  * must not be captured. */
 int wx_trace_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs, uint32_t n_reqs,

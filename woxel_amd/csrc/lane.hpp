@@ -44,9 +44,10 @@ static_assert(sizeof(GridDev) == 64, "GridDev layout");
 // the upper half of the float, which holds every distance up to 255; +0.0 is an active
 // tile. Against the records (8 or 16 slots in 16 bytes: child and walk bits, first child,
 // packed distances) an entry needs no bit tests, popcount or distance extraction. A
-// node-5 takes the same 64 KiB, a node-4 8 KiB instead of 4; entries of 4 bytes with whole
-// child indices (measured first) took twice that and lost on the 4096^3 sphere set what
-// the shorter lookup gained: L2 requests per frame 13.4 M (records), 23.9 M (4 bytes).
+// node-5 takes the same 64 KiB, a node-4 8 KiB instead of 4, and the records stay beside them
+// for wx_grid_save (the 2000-sphere grid: 167 MiB with, 134 before entries); entries of 4
+// bytes with whole child indices (measured first) took twice that and lost on the 4096^3
+// sphere set what the shorter lookup gained: L2 requests per frame 13.4 M (records), 23.9 M (4 bytes).
 // Forms of a grid, from its node counts and records (wx_grid_create):
 //   kOneRoot  compact entries, one node-5 of base 0 with a key of 20 bits, every pool within
 //             32-bit byte offsets;
@@ -292,10 +293,10 @@ __device__ __forceinline__ bool opaque_and(bool a, bool b) {
 // The lookup of one iteration (raycast.comp.wgsl:344-494): the step size at voxel (x, y, z).
 // Each level is one region of the lanes that need it, and no region nests in another: a
 // wave alone on its SIMD pays about 25 ns for a divergent region, six VALU instructions.
-// Large frames are bound by VALU issue (95 % of it on the 1080p sphere frame), so the regions
-// are written for their instruction count: offsets by bit-field inserts of shifted
-// coordinates, whose unwanted bits the last insert drops, and an entry's walk mark left in
-// an index and taken off its base instead.
+// Large frames are bound by VALU issue first (VALUBusy 81 % on the 1080p sphere frame, its tail
+// included), so the regions are written for their instruction count: offsets by bit-field
+// inserts of shifted coordinates, whose unwanted bits the last insert drops, and an entry's walk
+// mark left in an index and taken off its base instead.
 template <uint32_t kForm>
 __device__ __forceinline__ float lane_lookup(const GridDev &g, RayLane &r, uint32_t x, uint32_t y, uint32_t z,
                                              const int4 *s_root, bool root_lds) {

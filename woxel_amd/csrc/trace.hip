@@ -9,8 +9,9 @@
 //    have finished, the idle lanes take new slots: of the wave's fixed share of the one
 //    request (also for the scattered sets of a long ray list in the one-lane shape), or of
 //    chunks of a batch's work queue (per-XCD regions, with stealing; shadow rays continue
-//    in the lane of their primary). Every wave exits once its slots are used up and its
-//    lanes are idle; every ray ends within 1000 steps, so the grid always drains.
+//    in the lane of their primary; one kernel per grid form for a batch on one grid). Every
+//    wave exits once its slots are used up and its lanes are idle; every ray ends within 1000
+//    steps, so the grid always drains.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -116,8 +117,10 @@ struct BatchArgs {
     const uint32_t *begin;
     uint32_t n_grids, n_reqs, total, lg;
 };
-// The same with the tables among the kernel's arguments, which take 4 KiB at most: up to
-// 24 requests on 12 grids need no copy before the launch.
+// The same with the tables among the kernel's arguments, which take 4 KiB at most: a request
+// takes 132 bytes and a grid 64, so twice as many requests as grids, 24 on 12, fill them.
+// Such a batch needs no copy before the launch: 24 requests of 64x48 on 4 grids 119 us a call
+// and 25, by copy, 131; 24 on 12 grids 153 and on 13 167.
 constexpr uint32_t kInlineGrids = 12u, kInlineReqs = 24u;
 struct BatchInline {
     ReqDev reqs[kInlineReqs];
@@ -244,11 +247,13 @@ __device__ __forceinline__ bool slot_ray(const ReqDev &q, uint32_t s, uint32_t &
 // together and they take new rays. No counters in memory; rays that are not fast
 // (lane_fast) wait until the wave's others are done, so that the loop holds the fast step
 // of one grid form alone (64 VGPRs, eight waves per SIMD; 103 with the general step beside
-// it). With `split` the wave leaves out the sets whose rays go together: those lose by
-// refilling, which breaks up their lookups, and by a fixed share per wave (16.8 M panorama
-// rays: 2.05 ms one lane per ray, 2.56 refilled, 3.05 in fixed shares without refilling),
-// while scattered rays gain, as one lane per ray leaves nine lanes in ten idle (16.8 M:
-// 4.22 ms one lane per ray, 1.97 here).
+// it; the table form spills three there, at 72 and seven waves 16.8 M rays on eight node-5s
+// take 4992 us instead of 3977). On a grid without the fast step every ray waits so: that is
+// one lane per ray in fixed shares. With `split` the wave leaves out the sets whose rays go
+// together: those lose by refilling, which breaks up their lookups, and by a fixed share per
+// wave (16.8 M panorama rays: 2.05 ms one lane per ray, 2.56 refilled, 3.05 in fixed shares
+// without refilling), while scattered rays gain, as one lane per ray leaves nine lanes in ten
+// idle (16.8 M: 4.22 ms one lane per ray, 1.97 here).
 template <uint32_t KIND, uint32_t kForm>
 __global__ __launch_bounds__(256, 8) void k_persist1(GridDev g, ReqDev q, uint32_t total, uint32_t refill,
                                                    uint32_t split) {
@@ -1006,7 +1011,7 @@ int grid_new(const wx_grid_desc *d, const char *who, wx_grid **out) {
     const std::string w(who);
     if ((d->n5 && !d->root) || (d->n5 && !d->n5_records) || (d->n4 && !d->n4_records))
         return set_error(WX_ERR_INVALID, w + ": NULL pool with a non-zero count");
-    // the traversal's fast quotient relies on |p| <= bound <= 2^100 after the bound test
+    // the general step's quotient (lane.hpp) needs |p| <= 2^100 after the bound test
     if (!(d->bound > 0.0f) || !(d->bound <= 0x1p100f))
         return set_error(WX_ERR_INVALID, w + ": bound must be in (0, 2^100]");
     // at most 4 GiB of records per node level
