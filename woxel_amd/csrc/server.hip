@@ -208,9 +208,34 @@ __device__ void serve_poll(const ServeArgs &a) {
     }
 }
 
+// A pointer to global memory from its words in scalar registers. One that the compiler reads
+// from memory itself may point anywhere to it, and its loads take the form that can also reach
+// LDS, with the whole address in vector registers.
+template <typename T>
+__device__ __forceinline__ const T *global_at(uint32_t lo, uint32_t hi) {
+    return (const T *)(const __attribute__((address_space(1))) T *)((uint64_t)hi << 32 | lo);
+}
+
+// Grid i of the session's table, one word per lane gathered into scalars.
+__device__ __forceinline__ GridDev session_grid(const GridDev *grids, uint32_t i) {
+    const uint32_t v = reinterpret_cast<const uint32_t *>(grids + i)[__lane_id() & 15u];
+    uint32_t w[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) w[k] = (uint32_t)__builtin_amdgcn_readlane((int)v, k);
+    GridDev g;
+    __builtin_memcpy(&g, w, sizeof g);
+    g.root = global_at<int4>(w[0], w[1]);
+    g.n5 = global_at<char>(w[2], w[3]);
+    g.n4 = global_at<char>(w[4], w[5]);
+    g.leaf = global_at<uint32_t>(w[6], w[7]);
+    g.base = global_at<uint32_t>(w[8], w[9]);
+    return g;
+}
+
 // 8 waves per SIMD: the persistent loop keeps loop-invariant values live, which
-// would otherwise hold it to 5 (measured 16 % slower on a burst of 256 requests);
-// the few spills it costs sit outside the traversal loops.
+// would otherwise hold it to 5 (measured 16 % slower on a burst of 256 requests). Scalars
+// spill to vector lanes for it, three or four read back a step; vector registers do not since
+// the grid's descriptor is in scalars (session_grid): that burst 43.2 -> 42.3 ms.
 __global__ __launch_bounds__(256, 8) void k_serve(ServeArgs a) {
     if (blockIdx.x == 0 && threadIdx.x < 64u) {
         serve_poll(a);
@@ -311,7 +336,7 @@ __global__ __launch_bounds__(256, 8) void k_serve(ServeArgs a) {
         }
         const bool ok = request_ok(a, q, req_tiles) && cur >= req_begin && cur < req_end;
         if (ok) {
-            const GridDev g = a.sd->grids[q.grid];
+            const GridDev g = session_grid(a.sd->grids, q.grid);
             const uint32_t slot = band_tile(cur - req_begin, x) * 64u + lane;
             uint32_t px, py;
             if (camera_pixel(q, slot, px, py)) {  // lanes outside the image sit the tile out
