@@ -16,7 +16,8 @@ d.n5, d.n4, d.n3, d.bound = 1, 1 << 20, 0, 4096.0
 d.root = root.ctypes.data_as(C.POINTER(C.c_int32))
 d.n5_records, d.n4_records = [a.ctypes.data_as(C.POINTER(C.c_uint32)) for a in (n5, n4)]
 used = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
-resource.setrlimit(resource.RLIMIT_AS, (used + (8 << 20), resource.RLIM_INFINITY))
+old = resource.getrlimit(resource.RLIMIT_AS)
+resource.setrlimit(resource.RLIMIT_AS, (used + (8 << 20), old[1]))
 hold = []
 try:
     while True:
@@ -25,7 +26,7 @@ except MemoryError:
     pass
 h = C.c_void_p()
 rc = wx.lib.wx_grid_create(C.byref(d), C.byref(h))
-resource.setrlimit(resource.RLIMIT_AS, (resource.RLIM_INFINITY, resource.RLIM_INFINITY))
+resource.setrlimit(resource.RLIMIT_AS, old)
 print("code", rc, wx.lib.wx_last_error().decode())
 """
 
