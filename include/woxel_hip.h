@@ -102,8 +102,8 @@ typedef struct wx_tune {
                                  shadow rays also goes through refilled waves, for the runs of 64
                                  whose directions have nothing in common);
                               1: persistent waves whose idle lanes are refilled: one request
-                                 without shadow rays in equal shares, others from a work queue
-                                 (fields below);
+                                 without shadow rays in equal shares (on a grid of a bound above
+                                 2^20: as 0), others from a work queue (fields below);
                               2, 3: as 0 (two shapes that measured slower than it: compacting
                                  workgroups, node-5 records in LDS) */
     uint32_t refill;       /* 1: refill a wave's idle lanes once at least this many are idle (1..64) */

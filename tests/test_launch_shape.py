@@ -14,9 +14,9 @@ PROGRAM = """
 #include "launch_shape.hpp"
 int main() {
     unsigned long long rays;
-    unsigned cus, refills;
-    while (std::scanf("%llu %u %u", &rays, &cus, &refills) == 3) {
-        const wxk::ListShape s = wxk::list_shape(rays, cus, refills != 0u);
+    unsigned cus, fast;
+    while (std::scanf("%llu %u %u", &rays, &cus, &fast) == 3) {
+        const wxk::ListShape s = wxk::list_shape(rays, cus, fast != 0u);
         std::printf("%u %u\\n", s.lg, s.split ? 1u : 0u);
     }
 }
@@ -30,8 +30,8 @@ def shape(tmp_path_factory):
     csrc = os.path.join(HERE, "..", "woxel_amd", "csrc")
     subprocess.run(["g++", "-std=c++17", "-O1", "-I", csrc, str(d / "p.cpp"), "-o", str(d / "p")], check=True)
 
-    def ask(pairs, refills=1):
-        r = subprocess.run([str(d / "p")], input="".join(f"{n} {c} {refills}\n" for n, c in pairs),
+    def ask(pairs, fast=1):
+        r = subprocess.run([str(d / "p")], input="".join(f"{n} {c} {fast}\n" for n, c in pairs),
                            capture_output=True, text=True, check=True)
         return [tuple(int(x) for x in line.split()) for line in r.stdout.splitlines()]
 
@@ -56,7 +56,7 @@ def test_split_lists_take_whole_sets(shape, cus):
 @pytest.mark.parametrize("cus", CUS)
 def test_grids_without_the_fast_step_keep_their_lists(shape, cus):
     ns = lengths(cus)
-    assert not any(s for _, s in shape([(n, cus) for n in ns], refills=0))
+    assert set(shape([(n, cus) for n in ns], fast=0)) == {(6, 0)}
 
 
 @pytest.mark.parametrize("cus", CUS)

@@ -221,8 +221,8 @@ constexpr float kFastBound = 0x1p20f;
 // is a product of finite numbers, an infinite position ends at the bound test, and nothing in
 // the step is a NaN: one conversion floors, and t equals the minimum exactly when it is <= both
 // others. It and the general step take the quotient in three operations where IEEE division
-// takes eleven each: 1 Mi rays with a -0 start in every wave 755 -> 645 us, on a grid of bound
-// 2^21 10270 -> 10000 us a 1080p frame.
+// takes eleven each: 1 Mi rays with a -0 start in every wave 755 -> 645 us, a 1080p frame of a
+// grid of one node-5 and bound 2^21 4854 -> 3100.
 constexpr int kGeneral = 0, kClean = 1, kFast = 2;
 
 __device__ __forceinline__ bool axis_fast(float d, float inv, float p) {
@@ -488,7 +488,8 @@ __device__ __forceinline__ void lane_run(const GridDev &g, RayLane &r, const int
     if (fast && g.form == kTable) return lane_loop<kFast, kTable>(g, r, s_root, root_lds);
     if (fast) return lane_loop<kFast, kIndexed>(g, r, s_root, root_lds);
     const bool clean = __ballot(lane_state(r) == kRun && !lane_clean(r)) == 0ull;
-    if (clean && g.form != kIndexed) lane_loop<kClean, kTable>(g, r, s_root, root_lds);
+    if (clean && g.form == kOneRoot) lane_loop<kClean, kOneRoot>(g, r, s_root, root_lds);
+    else if (clean && g.form != kIndexed) lane_loop<kClean, kTable>(g, r, s_root, root_lds);
     else if (g.form != kIndexed) lane_loop<kGeneral, kTable>(g, r, s_root, root_lds);
     else lane_loop<kGeneral, kIndexed>(g, r, s_root, root_lds);
 }

@@ -16,7 +16,11 @@ namespace wxk {
 // pixels of the ball 50.4 -> 41.4 us, of an isosurface 77.1 -> 63.9, 160x90 pixels of 1000
 // spheres 112 -> 106, 448x252 164 -> 156; 500 scattered rays 50.5 -> 43.0, 8000 66.5 -> 60.9,
 // 128000 75.2 -> 77.0; panoramas of 8192 and 131072 rays 85.5 -> 74.2 and 129 -> 117.
-inline uint32_t rays_per_wave_log2(uint64_t rays, uint32_t cus) {
+// `fast`: the grid's bound allows the fast step (kFastBound). Beyond it rays sit on cell
+// borders, lane by lane alike, until the step cap: 64 Ki in waves of 16 took 695 us, in waves
+// of 64 491.
+inline uint32_t rays_per_wave_log2(uint64_t rays, uint32_t cus, bool fast) {
+    if (!fast) return 6u;
     uint32_t lg = 0;
     while (lg < 6u && (rays >> lg) > 16u * cus) ++lg;
     return lg == 3u ? 4u : lg;
@@ -31,12 +35,12 @@ struct ListShape {
     uint32_t lg;
     bool split;
 };
-// `refills`: the grid's bound allows the fast step, the only one that k_persist1 refills
-// (kFastBound); beyond it a scattered list of 1 Mi rays took 7537 us split, 6931 in one kernel.
-inline ListShape list_shape(uint64_t rays, uint32_t cus, bool refills) {
+// k_persist1 refills the fast step alone; without it a scattered list of 1 Mi rays took 7537 us
+// split, 6931 in one kernel.
+inline ListShape list_shape(uint64_t rays, uint32_t cus, bool fast) {
     ListShape s;
-    s.split = refills && (rays + 63u) / 64u >= 2u * cus * 32u;
-    s.lg = s.split ? 6u : rays_per_wave_log2(rays, cus);
+    s.split = fast && (rays + 63u) / 64u >= 2u * cus * 32u;
+    s.lg = s.split ? 6u : rays_per_wave_log2(rays, cus, fast);
     return s;
 }
 

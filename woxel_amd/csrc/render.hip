@@ -279,7 +279,7 @@ extern "C" int wx_render_camera(wx_grid *g, const wx_camera *cam, uint32_t w, ui
     a.sdx = s->sun_dir[0], a.sdy = s->sun_dir[1], a.sdz = s->sun_dir[2], a.sa = s->sun_color[3];
     a.scr = s->sun_color[0], a.scg = s->sun_color[1], a.scb = s->sun_color[2];
     a.out = out;
-    const uint32_t lg = rays_per_wave_log2((uint64_t)w * h, (uint32_t)wx::cu_count());
+    const uint32_t lg = rays_per_wave_log2((uint64_t)w * h, (uint32_t)wx::cu_count(), g->dev.bound <= kFastBound);
     const uint32_t lw = 1u + ((lg + 1u) >> 1), lh = lg >> 1;
     const dim3 grid((w + (1u << lw) - 1u) >> lw, (h + (1u << lh) - 1u) >> lh, 1);
     hipStream_t st = static_cast<hipStream_t>(stream);

@@ -248,8 +248,8 @@ __device__ __forceinline__ bool slot_ray(const ReqDev &q, uint32_t s, uint32_t &
 // (lane_fast) wait until the wave's others are done, so that the loop holds the fast step
 // of one grid form alone (64 VGPRs, eight waves per SIMD; 103 with the general step beside
 // it; the table form spills three there, at 72 and seven waves 16.8 M rays on eight node-5s
-// take 4992 us instead of 3977). On a grid without the fast step every ray waits so: that is
-// one lane per ray in fixed shares. With `split` the wave leaves out the sets whose rays go
+// take 4992 us instead of 3977). A grid whose bound rules the fast step out goes to the
+// one-lane shapes instead (16.8 M rays at bound 2^21: 25.9 ms, here 39.6). With `split` the wave leaves out the sets whose rays go
 // together: those lose by refilling, which breaks up their lookups, and by a fixed share per
 // wave (16.8 M panorama rays: 2.05 ms one lane per ray, 2.56 refilled, 3.05 in fixed shares
 // without refilling), while scattered rays gain, as one lane per ray leaves nine lanes in ten
@@ -265,7 +265,7 @@ __global__ __launch_bounds__(256, 8) void k_persist1(GridDev g, ReqDev q, uint32
     const uint32_t lane = threadIdx.x & 63u;
     ReadyRays &ready = s_ready[threadIdx.x >> 6];
     const uint64_t lt = (1ull << lane) - 1ull;
-    const bool clip = (q.flags & WX_TRACE_CLIP) != 0u, bounded = g.bound <= kFastBound;
+    const bool clip = (q.flags & WX_TRACE_CLIP) != 0u;
     const uint64_t stride = (uint64_t)gridDim.x * 256u, end = total;
     const uint64_t first =
         (uint64_t)blockIdx.x * 256u + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~63u));
@@ -294,7 +294,7 @@ __global__ __launch_bounds__(256, 8) void k_persist1(GridDev g, ReqDev q, uint32
                     lane_start(f, o[0], o[1], o[2], d[0], d[1], d[2], g.bound, clip);
                     if (lane_state(f) != kRun) {
                         lane_write(f, o[0], o[1], o[2], q.out + fp);
-                    } else if (!(bounded && lane_fast(f))) {
+                    } else if (!lane_fast(f)) {
                         slow = true;
                         f.state = WX_OOB;
                     }
@@ -357,7 +357,7 @@ __global__ __launch_bounds__(256, 8) void k_persist1(GridDev g, ReqDev q, uint32
         if (KIND == WX_REQ_RAYS && split && rays_together(in, d[0], d[1], d[2])) continue;
         if (!in) continue;
         lane_start(r, o[0], o[1], o[2], d[0], d[1], d[2], g.bound, clip);
-        if (lane_state(r) != kRun || (bounded && lane_fast(r))) continue;
+        if (lane_state(r) != kRun || lane_fast(r)) continue;
         lane_loop<kGeneral, kForm == kIndexed ? kIndexed : kTable>(g, r, s_root_buf, root_lds);
         lane_write(r, o[0], o[1], o[2], q.out + pix);
     }
@@ -801,18 +801,20 @@ int launch_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs
     };
     hipError_t e;
     const uint32_t cus = (uint32_t)wx::cu_count();
-    if (t.persistent != 1u) {  // the one-lane shape
+    bool fast = true;  // every grid's bound allows the fast step
+    for (uint32_t i = 0; i < n_grids; ++i) fast = fast && grids[i]->dev.bound <= kFastBound;
+    if (t.persistent != 1u || (single && !fast)) {  // the one-lane shape
         if (one) {
             const bool sh = (q[0].flags & WX_TRACE_SHADOW) != 0u;
             if (q[0].kind == WX_REQ_CAMERA) {
-                const uint32_t lg = rays_per_wave_log2(total, cus), lw = 1u + ((lg + 1u) >> 1), lh = lg >> 1;
+                const uint32_t lg = rays_per_wave_log2(total, cus, fast), lw = 1u + ((lg + 1u) >> 1), lh = lg >> 1;
                 dim3 grid((q[0].w + (1u << lw) - 1u) >> lw, (q[0].h + (1u << lh) - 1u) >> lh, 1);
                 const uint32_t band = t.xcd_split == 2u ? 1u : 0u;  // XCD-banded tile order
                 if (sh) hipLaunchKernelGGL(k_simple_camera<true>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], lg, band);
                 else hipLaunchKernelGGL(k_simple_camera<false>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], lg, band);
             } else {
                 // split: the sets of 64 rays that scatter go to k_persist1, the others stay
-                const ListShape list = list_shape(q[0].w, cus, grids[0]->dev.bound <= kFastBound);
+                const ListShape list = list_shape(q[0].w, cus, fast);
                 const uint32_t lg = list.lg, split = list.split && may_split && !sh ? 1u : 0u;
                 dim3 grid((q[0].w + (2u << lg) - 1u) >> (lg + 1u));
                 if (sh) hipLaunchKernelGGL(k_simple_rays<true>, grid, dim3(128), 0, stream, grids[0]->dev, q[0], lg, 0u);
@@ -825,7 +827,7 @@ int launch_batch(wx_grid *const *grids, uint32_t n_grids, const wx_request *reqs
                 }
             }
         } else {
-            const uint32_t lg = rays_per_wave_log2(total, cus);
+            const uint32_t lg = rays_per_wave_log2(total, cus, fast);
             const dim3 grid((uint32_t)((total + (2u << lg) - 1u) >> (lg + 1u)));
             if (n_reqs <= kInlineReqs && n_grids <= kInlineGrids) {
                 BatchInline b;
