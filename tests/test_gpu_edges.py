@@ -208,3 +208,42 @@ def test_root_keys_of_any_size(wx, cuda):
     for key in ((1 << 20, 0, 0), (0, -(1 << 20), 0), (0, 0, -(1 << 31)), ((1 << 20) + 1, 1 << 20, 0)):
         for persistent in (0, 1):
             assert_hits_equal(records(key, persistent), away, f"key {key}")
+
+
+@pytest.mark.parametrize("entries", [2, 16, 17, 40])
+def test_first_of_equal_root_keys(wx, cuda, entries):
+    """A descriptor's root table may name a key twice: the first entry is the node, in tables
+    scanned from LDS (up to 16 entries) and from memory, in every shape."""
+    print(f"{entries} root entries", flush=True)
+    p = wx.Vdb345()
+    p.add_spheres(np.array([[400.0, 300.0, 450.0, 120.0]]))
+    p.compute_sdf()
+    lay = p.layout_arrays()
+    n5 = lay["n5"].reshape(1, -1)
+    solid = np.zeros_like(n5)  # every slot an active tile: a hit wherever it is looked up
+    nodes = np.concatenate([n5] + [solid] * (entries - 1))
+    cam = wx.camera_basis((1200, 900, -700), (400, 300, 450), (0, 1, 0), 1.5, 45.0, 96.0)
+
+    def records(where, persistent):
+        root = np.zeros((entries, 4), np.int32)
+        root[:, 0] = 5 + np.arange(entries)  # keys no ray meets
+        root[:, 3] = np.arange(entries)
+        root[where, :3] = lay["root"].reshape(-1, 4)[0, :3]
+        # the sphere's node first among the equal keys
+        root[where[0], 3], root[0, 3] = 0, where[0]
+        g = grid_of(wx, root, nodes, lay["n4"], lay["leaves"])
+        out = [cuda.empty((96 * 64, 32), dtype=cuda.uint8, device="cuda") for _ in range(3)]
+        tune = wx.Tune(persistent=persistent, refill=16, chunk=128, waves_per_cu=16, xcd_split=1)
+        wx.trace_batch([g], [wx.camera_request(0, cam, 96, 64, out[0])], tune)
+        wx.trace_batch([g], [wx.camera_request(0, cam, 96, 64, out[1])] * 2, tune)
+        wx.trace_batch([g, g], [wx.camera_request(k, cam, 96, 64, out[2]) for k in (1, 0)], tune)
+        a = [wx.hits_to_numpy(x) for x in out]
+        assert_hits_equal(a[1], a[0], "batch")
+        assert_hits_equal(a[2], a[0], "batch of several grids")
+        return a[0]
+
+    want = wx.hits_to_numpy(wx.Grid(p).trace_camera(cam, 96, 64, 0.5, clip=True))
+    assert (want["state"] == wx.HIT).any()
+    for where in ([0], [entries - 1], [0, entries - 1], [0, 1], [entries // 2, entries - 1]):
+        for persistent in (0, 1):
+            assert_hits_equal(records(sorted(set(where)), persistent), want, f"{where} {persistent}")
