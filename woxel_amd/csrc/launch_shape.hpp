@@ -17,8 +17,8 @@ namespace wxk {
 // spheres 112 -> 106, 448x252 164 -> 156; 500 scattered rays 50.5 -> 43.0, 8000 66.5 -> 60.9,
 // 128000 75.2 -> 77.0; panoramas of 8192 and 131072 rays 85.5 -> 74.2 and 129 -> 117.
 // `fast`: the grid's bound allows the fast step (kFastBound). Beyond it rays sit on cell
-// borders, lane by lane alike, until the step cap: 64 Ki in waves of 16 took 695 us, in waves
-// of 64 491.
+// borders, lane by lane alike, until the step cap: 64 Ki in waves of 16 took 645 us, in waves
+// of 64 470.
 inline uint32_t rays_per_wave_log2(uint64_t rays, uint32_t cus, bool fast) {
     if (!fast) return 6u;
     uint32_t lg = 0;
@@ -35,8 +35,8 @@ struct ListShape {
     uint32_t lg;
     bool split;
 };
-// k_persist1 refills the fast step alone; without it a scattered list of 1 Mi rays took 7537 us
-// split, 6931 in one kernel.
+// k_persist1 refills the fast step alone; without it a scattered list of 1 Mi rays took 2109 us
+// split, 1835 in one kernel (16 Mi 22.9 and 24.7 ms).
 inline ListShape list_shape(uint64_t rays, uint32_t cus, bool fast) {
     ListShape s;
     s.split = fast && (rays + 63u) / 64u >= 2u * cus * 32u;

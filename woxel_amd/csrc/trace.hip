@@ -247,9 +247,9 @@ __device__ __forceinline__ bool slot_ray(const ReqDev &q, uint32_t s, uint32_t &
 // together and they take new rays. No counters in memory; rays that are not fast
 // (lane_fast) wait until the wave's others are done, so that the loop holds the fast step
 // of one grid form alone (64 VGPRs, eight waves per SIMD; 103 with the general step beside
-// it; the table form spills three there, at 72 and seven waves 16.8 M rays on eight node-5s
-// take 4992 us instead of 3977). A grid whose bound rules the fast step out goes to the
-// one-lane shapes instead (16.8 M rays at bound 2^21: 25.9 ms, here 39.6). With `split` the wave leaves out the sets whose rays go
+// it; the table form spills two to five there, at 72 and seven waves 16.8 M rays on eight
+// node-5s take 4022 us instead of 2944). A grid whose bound rules the fast step out goes to the
+// one-lane shapes instead (16.8 M rays at bound 2^21: 24.7 ms, here 39.6). With `split` the wave leaves out the sets whose rays go
 // together: those lose by refilling, which breaks up their lookups, and by a fixed share per
 // wave (16.8 M panorama rays: 2.05 ms one lane per ray, 2.56 refilled, 3.05 in fixed shares
 // without refilling), while scattered rays gain, as one lane per ray leaves nine lanes in ten
